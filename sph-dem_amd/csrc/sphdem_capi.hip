@@ -32,7 +32,8 @@ struct HostFields {
   long long sphStep;
   int ng, ns, nd, K, lgen, countsClean, gcntZeroAt;
   unsigned gstale;
-  bool listsValid, segsValid, gridValid, recFresh, pvFresh, dFresh;
+  bool listsValid, listsNear, hKept, segsValid, gridValid, pvFresh, dFresh;
+  int recFresh;
   double ssr;
   Grid gs, gc;
   GhostBand band;
@@ -71,19 +72,25 @@ struct sphdem_ctx {
   int tileSeg = 0, walkTPB = 256;
   // cached SPH neighbour lists (valid from their first use until the next reset)
   int *nbl = nullptr, *nbcnt = nullptr;
-  // the per-target search's quantised records (one per entry, plus slack for
-  // a batch read past a range's end) and its two generation flag slots
-  uint2* lrec = nullptr;
+  // the searches' records (k_near's, or k_lists_t's in half the room; one per
+  // entry, plus slack for a batch read past a range's end) and their two
+  // generation flag slots
+  uint4* lrec = nullptr;
   int* lflag = nullptr;
   int lgen = 0;
   // DEM cells with a sphere within one cell, marked with the number in nearGen
   int* demNear = nullptr;
   int demNearCap = 0;
   bool listsValid = false;
-  // the list search's records (recFresh) and the mixed form's P and V records
+  // the valid lists are near lists (k_near); and h has changed since they were
+  // built, its value then kept in hList
+  bool listsNear = false, hKept = false;
+  double* hList = nullptr;  // per SPH-group particle
+  // a search's records (recFresh, REC_*) and the mixed form's P and V records
   // (pvFresh) were written by the last reset's permutation and no position,
   // h or vhat changed since
-  bool recFresh = false, pvFresh = false;
+  int recFresh = REC_NONE;
+  bool pvFresh = false;
   // the mixed form's D records were written by the last EOS pass and no
   // density, pdr2 or h changed since (a box without ghosts)
   bool dFresh = false;
@@ -272,8 +279,8 @@ int allocEntries(sphdem_ctx* ctx, int64_t ghostCap) {
   HIPC(hipMalloc(&tmp, sizeof(int) * ent));
   HIPC(hipMalloc(&perm, sizeof(int) * ent));
   HIPC(hipMalloc(&hinv, sizeof(double2) * ent));
-  uint2* lrec = nullptr;
-  HIPC(hipMalloc(&lrec, sizeof(uint2) * (ent + 64)));
+  uint4* lrec = nullptr;
+  HIPC(hipMalloc(&lrec, sizeof(uint4) * (ent + 128)));
   if (ctx->storeMem[0]) {
     const size_t n = (size_t)ctx->n;
     for (int k = 0; k < kNumVec; k++)
@@ -434,7 +441,10 @@ int tileBlocks(const sphdem_ctx* ctx) {
 constexpr unsigned GS_POSH = 1, GS_VHM = 2, GS_DPO = 4, GS_ALL = 7;
 void markStale(sphdem_ctx* ctx, unsigned groups) {
   ctx->gstale |= groups;
-  if (groups & (GS_POSH | GS_VHM)) ctx->recFresh = ctx->pvFresh = false;
+  if (groups & (GS_POSH | GS_VHM)) {
+    ctx->recFresh = REC_NONE;
+    ctx->pvFresh = false;
+  }
   if (groups & (GS_POSH | GS_DPO)) ctx->dFresh = false;
 }
 int refreshGhosts(sphdem_ctx* ctx, unsigned need) {
@@ -456,32 +466,76 @@ ListQuant listQuant(const Grid& g) {
   q.uinv = ldexp(1.0, 11 - e);
   return q;
 }
-int launchLists(sphdem_ctx* ctx) {
-  CHECK(refreshGhosts(ctx, GS_POSH));
+Quant mixQuant(const Grid& g);
+// the exact lists of positions and h `pos`
+int launchLists(sphdem_ctx* ctx, const double4* pos) {
   if (ctx->tileSeg == 0) {
     if (ctx->ns == 0) return 0;
     const ListQuant lq = listQuant(ctx->gs);
     const int gen = ctx->lgen++ & 1;
-    if (!ctx->recFresh) {  // else the reset's permutation wrote them
-      hipLaunchKernelGGL(k_lrec, dim3(blocks(ctx->ns + ctx->ng)), dim3(TPB), 0, ctx->stream,
-                         ctx->cur.posh, ctx->ns, ctx->n, ctx->ng, lq, ctx->lrec, ctx->lflag, gen,
+    if (ctx->recFresh != REC_EXACT) {  // else the reset's permutation wrote them
+      hipLaunchKernelGGL(k_lrec, dim3(blocks(ctx->ns + ctx->ng)), dim3(TPB), 0, ctx->stream, pos,
+                         ctx->ns, ctx->n, ctx->ng, lq, (uint2*)ctx->lrec, ctx->lflag, gen,
                          ctx->graphMode ? &ctx->dg->ghostTotal : (const int*)nullptr);
       LAUNCHED();
     }
-    ctx->recFresh = false;
+    ctx->recFresh = REC_NONE;
     const int per = (ctx->ns + 7) / 8;
     hipLaunchKernelGGL(k_lists_t<32>, dim3(8 * ((per + TPB - 1) / TPB)), dim3(TPB), 0,
-                       ctx->stream, ctx->cur.posh, ctx->lrec, ctx->cur.cell, ctx->gs, ctx->gbase,
-                       ctx->start, ctx->ns, lq.uinv, ctx->lflag, gen, ctx->nbl, ctx->nbcnt,
+                       ctx->stream, pos, (const uint2*)ctx->lrec, ctx->cur.cell, ctx->gs,
+                       ctx->gbase, ctx->start, ctx->ns, lq.uinv, ctx->lflag, gen, ctx->nbl, ctx->nbcnt,
                        ctx->dg);
     LAUNCHED();
     return 0;
   }
   if (!ctx->segsValid) CHECK(buildSegments(ctx));
-  hipLaunchKernelGGL(k_lists, dim3(tileBlocks(ctx)), dim3(TPB), 0, ctx->stream, ctx->cur.posh,
+  hipLaunchKernelGGL(k_lists, dim3(tileBlocks(ctx)), dim3(TPB), 0, ctx->stream, pos,
                      ctx->cur.cell, ctx->gs, ctx->gbase, ctx->start, ctx->segs,
                      ctx->segOff + ctx->gs.dim[0] * ctx->gs.dim[1], ctx->ns, ctx->nbl,
                      ctx->nbcnt, ctx->dg);
+  LAUNCHED();
+  return 0;
+}
+// Whether a step's walks take near lists: not with a segmented tile shape, and
+// not where a cell holds over kNearOccupancy particles at
+// the initial spacing (h grown at a free surface by a density
+// re-initialisation).  There the near search's mask words overflow their room
+// and the tile's targets are gone through once more: 830 against 277 us a build
+// of the 48^3 dam break re-initialised every step (216 a cell), while at the
+// usual 27 a cell it takes 44 against 125 us (16^3 box), 125 against 199 us
+// (64^3) and 1.89 against 2.71 ms (160^3).
+constexpr double kNearOccupancy = 45.0;
+bool nearSearch(const sphdem_ctx* ctx) {
+  const double e = ctx->P.psep > 0.0 ? ctx->gs.edge / ctx->P.psep : 0.0;
+  return ctx->tileSeg == 0 && e * e * e <= kNearOccupancy;
+}
+// Up to this many targets (two tiles a CU) a tile's columns are searched by nine
+// wavefronts side by side instead of three after one another: a build is then a
+// chain of latencies.  Sedimentation boxes, one build, nine against three:
+// 12^3 23 / 37 us, 16^3 44 / 68, 20^3 27 / 42, 24^3 35 / 38, 28^3 52 / 64;
+// past it the wavefronts queue: 32^3 64 / 52, 64^3 265 / 125.
+constexpr int kNearSmall = 64 * 512;
+// the near lists, right after a reset (positions in their cells)
+int launchNear(sphdem_ctx* ctx) {
+  if (ctx->ns == 0) return 0;
+  const Quant Q = mixQuant(ctx->gs);
+  const int gen = ctx->lgen++ & 1;
+  if (ctx->recFresh != REC_NEAR) {  // else the reset's permutation wrote them
+    hipLaunchKernelGGL(k_near_rec, dim3(blocks(ctx->ns + ctx->ng)), dim3(TPB), 0, ctx->stream,
+                       ctx->cur.posh, ctx->ns, ctx->n, ctx->ng, Q, ctx->lrec, ctx->lflag, gen,
+                       ctx->graphMode ? &ctx->dg->ghostTotal : (const int*)nullptr);
+    LAUNCHED();
+  }
+  ctx->recFresh = REC_NONE;
+  auto launch = [&](auto kernel, int waves) {
+    hipLaunchKernelGGL(kernel, dim3(8 * ((ctx->ns + 511) / 512)), dim3(64 * waves), 0,
+                       ctx->stream, ctx->cur.posh, ctx->lrec, ctx->cur.cell, ctx->gs, ctx->gbase,
+                       ctx->start, ctx->ns, Q.inv, ctx->lflag, gen, ctx->nbl, ctx->nbcnt, ctx->dg);
+  };
+  if (ctx->ns <= kNearSmall)
+    launch(k_near<9>, 9);
+  else
+    launch(k_near<3>, 3);
   LAUNCHED();
   return 0;
 }
@@ -665,7 +719,8 @@ int doReset(sphdem_ctx* ctx, bool keepSsr = false, bool midInit = false,
     return fail(ctx, SPHDEM_E_STATE, "a captured reset needs the state a reset on the same grid "
                                      "leaves");
   ctx->segsValid = false;
-  ctx->recFresh = ctx->pvFresh = ctx->dFresh = false;
+  ctx->recFresh = REC_NONE;
+  ctx->pvFresh = ctx->dFresh = false;
   // hmax_bits is cleared by the previous reset's k_bin (or by the upload);
   // gcnt[n], the scans' closing zero, is written by nothing else
   if (n == 0) HIPC(hipMemsetAsync(&ctx->dg->hmax_bits, 0, sizeof(unsigned long long), ctx->stream));
@@ -785,7 +840,8 @@ int doReset(sphdem_ctx* ctx, bool keepSsr = false, bool midInit = false,
   if (fold.mode && ctx->ns > 0) {
     R.ns = ctx->ns;
     if (ctx->tileSeg == 0) {
-      R.lists = 1;
+      R.lists = nearSearch(ctx) ? REC_NEAR : REC_EXACT;
+      R.Q = mixQuant(ctx->gs);
       R.lq = listQuant(ctx->gs);
       R.rec = ctx->lrec;
       R.lflag = ctx->lflag;
@@ -819,19 +875,40 @@ int doReset(sphdem_ctx* ctx, bool keepSsr = false, bool midInit = false,
   ctx->gstale = 0;  // the permutation copied every ghost from its origin
   std::swap(ctx->cur, ctx->alt);
   std::swap(ctx->storeMem[0], ctx->storeMem[1]);
+  ctx->listsNear = ctx->hKept = false;
   ctx->listsValid = false;  // updateDomain clears every neighbour list (dataLL.cpp:374)
-  ctx->recFresh = R.lists != 0;
+  ctx->recFresh = R.lists;
   ctx->pvFresh = R.mixed != 0;
   return side.join();
 }
 
 // The cached lists are built by the first pair pass after a reset, with the h
-// of that moment (dataLL.impl.h:186-188).
+// of that moment (dataLL.impl.h:186-188).  Near lists in their place are
+// replaced by the exact ones they stand for: the same positions, and the h
+// of their own build.
 int ensureLists(sphdem_ctx* ctx) {
-  if (ctx->listsValid) return 0;
+  if (ctx->listsValid && !ctx->listsNear) return 0;
   Timed tm(ctx, KID_LISTS);
-  CHECK(launchLists(ctx));
+  CHECK(refreshGhosts(ctx, GS_POSH));
+  const double4* pos = ctx->cur.posh;
+  if (ctx->listsValid && ctx->hKept && ctx->ns > 0) {
+    hipLaunchKernelGGL(k_list_pos, dim3(blocks(ctx->ns + ctx->ng)), dim3(TPB), 0, ctx->stream,
+                       ctx->cur.posh, ctx->hList, ctx->ns, ctx->n, ctx->ng, ctx->gorig,
+                       ctx->alt.posh);
+    LAUNCHED();
+    pos = ctx->alt.posh;
+  }
+  CHECK(launchLists(ctx, pos));
   ctx->listsValid = true;
+  ctx->listsNear = ctx->hKept = false;
+  return 0;
+}
+// The step's lists, right after a reset.
+int stepLists(sphdem_ctx* ctx) {
+  if (!nearSearch(ctx)) return ensureLists(ctx);
+  Timed tm(ctx, KID_LISTS);
+  CHECK(launchNear(ctx));
+  ctx->listsValid = ctx->listsNear = true;
   return 0;
 }
 
@@ -989,9 +1066,11 @@ constexpr std::array<void (*)(sphdem_ctx*), sizeof...(F)> forceTable(
 // withOmega (VAR_H only): calcOmega summed in the same walk and omega stored --
 // the step's omega pass, which only the force and dddt of omega's own particle
 // read, fused into the walk that follows it
-int passForce(sphdem_ctx* ctx, bool hinvReady = false, bool withOmega = false) {
+// inStep: the caller has seen to the lists (near ones will do)
+int passForce(sphdem_ctx* ctx, bool hinvReady = false, bool withOmega = false,
+              bool inStep = false) {
   if (withOmega && !varH(ctx)) return fail(ctx, SPHDEM_E_STATE, "fused omega needs VAR_H");
-  CHECK(ensureLists(ctx));
+  if (!inStep) CHECK(ensureLists(ctx));
   CHECK(refreshGhosts(ctx, GS_ALL));
   if (!mixed(ctx) && !hinvReady) CHECK(computeHinv(ctx));
   static constexpr auto table = forceTable<false>(std::make_integer_sequence<int, 32>{});
@@ -1007,10 +1086,10 @@ int passForce(sphdem_ctx* ctx, bool hinvReady = false, bool withOmega = false) {
   if (withOmega) markStale(ctx, GS_DPO);
   return 0;
 }
-// withOmega: as in passForce
-int passDddt(sphdem_ctx* ctx, bool withOmega = false) {
+// withOmega, inStep: as in passForce
+int passDddt(sphdem_ctx* ctx, bool withOmega = false, bool inStep = false) {
   if (withOmega && !varH(ctx)) return fail(ctx, SPHDEM_E_STATE, "fused omega needs VAR_H");
-  CHECK(ensureLists(ctx));
+  if (!inStep) CHECK(ensureLists(ctx));
   CHECK(refreshGhosts(ctx, GS_POSH | GS_VHM));
   if (mixed(ctx)) {
     Timed tm(ctx, KID_DDDT);
@@ -1112,6 +1191,7 @@ int passContacts(sphdem_ctx* ctx) {
 }
 // one iteration of the density re-initialisation (sphIncompress.cpp:29-34)
 int passDensity(sphdem_ctx* ctx) {
+  if (ctx->listsNear) CHECK(ensureLists(ctx));  // before h changes
   hipLaunchKernelGGL(k_hfromdens, dim3(blocks(ctx->ns)), dim3(TPB), 0, ctx->stream, ctx->cur,
                      ctx->ns, ctx->P.hfac);
   LAUNCHED();
@@ -1157,7 +1237,8 @@ int stepStart(sphdem_ctx* ctx, uint32_t bodyMask = 0, const double* accel = null
   return 0;
 }
 // fold: start() (WrapFold mode 1) when the step's start() has not run
-int stepMiddle(sphdem_ctx* ctx, const WrapFold& fold = WrapFold{}) {
+// near: the pair walk may take near lists (the call runs the whole step)
+int stepMiddle(sphdem_ctx* ctx, const WrapFold& fold = WrapFold{}, bool near = false) {
   CHECK(doReset(ctx, false, true, fold));
   bool hinvReady = false;
   {
@@ -1175,11 +1256,11 @@ int stepMiddle(sphdem_ctx* ctx, const WrapFold& fold = WrapFold{}) {
       hinvReady = true;
     }
     side.back();
-    CHECK(ensureLists(ctx));
+    CHECK(near ? stepLists(ctx) : ensureLists(ctx));
     CHECK(side.join());
   }
   // calcOmega (VAR_H) is summed in the force walk: the force of a reads omega_a only
-  CHECK(passForce(ctx, hinvReady, varH(ctx)));
+  CHECK(passForce(ctx, hinvReady, varH(ctx), true));
   const int na = ctx->ns + ctx->nd;
   hipLaunchKernelGGL(k_accel, dim3(reduceBlocks(std::max(na, 1))), dim3(TPB), 0, ctx->stream,
                      ctx->cur, na, ctx->dg);
@@ -1194,7 +1275,8 @@ int stepMiddle(sphdem_ctx* ctx, const WrapFold& fold = WrapFold{}) {
   return 0;
 }
 // foldDrift: the drift of r (and the time's half step) done by the reset's k_wrap
-int stepEnd(sphdem_ctx* ctx, bool foldDrift = false) {
+// near: as in stepMiddle
+int stepEnd(sphdem_ctx* ctx, bool foldDrift = false, bool near = false) {
   WrapFold fold{};
   if (foldDrift) {
     fold.mode = 2;
@@ -1231,15 +1313,18 @@ int stepEnd(sphdem_ctx* ctx, bool foldDrift = false) {
       LAUNCHED();
     }
     side.back();
-    CHECK(passDddt(ctx, fuse));
+    CHECK(near ? stepLists(ctx) : ensureLists(ctx));
+    CHECK(passDddt(ctx, fuse, true));
     CHECK(side.join());
   } else {
-    CHECK(passDddt(ctx, fuse));
+    CHECK(near ? stepLists(ctx) : ensureLists(ctx));
+    CHECK(passDddt(ctx, fuse, true));
   }
   Timed tm(ctx, KID_REST);
   hipLaunchKernelGGL(k_end_rest, dim3(blocks(std::max(ctx->ns, 1))), dim3(TPB), 0, ctx->stream,
-                     ctx->cur, ctx->ns, ctx->P, ctx->dg);
+                     ctx->cur, ctx->ns, ctx->P, ctx->dg, ctx->listsNear ? ctx->hList : nullptr);
   LAUNCHED();
+  ctx->hKept = ctx->listsNear;
   markStale(ctx, GS_ALL);
   return 0;
 }
@@ -1296,7 +1381,7 @@ void freeAll(sphdem_ctx* ctx) {
                   ctx->mixP,        ctx->mixV,        ctx->mixD,    ctx->okey,
                   ctx->posm,        ctx->pairCnt,     ctx->pairOff, ctx->lrec,
                   ctx->lflag,       ctx->demNear,     ctx->nearGen, ctx->gate,
-                  ctx->keepMem,     ctx->dgKeep};
+                  ctx->keepMem,     ctx->dgKeep,      ctx->hList};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
   for (hipEvent_t e : ctx->evPool) (void)hipEventDestroy(e);
@@ -1355,6 +1440,7 @@ int sphdem_create(const sphdem_params* params, int device, int64_t capacity, sph
     HIPC(hipMalloc(&ctx->inv, sizeof(int) * capacity));
     HIPC(hipMalloc(&ctx->nbl, sizeof(int) * (size_t)kMaxNb * capacity));
     HIPC(hipMalloc(&ctx->nbcnt, sizeof(int) * capacity));
+    HIPC(hipMalloc(&ctx->hList, sizeof(double) * capacity));
     HIPC(hipMalloc(&ctx->fieldbuf, sizeof(double) * 3 * capacity));
     HIPC(hipMalloc(&ctx->errflag, sizeof(int)));
     HIPC(hipMalloc(&ctx->lflag, sizeof(int) * 2));
@@ -1632,7 +1718,7 @@ int sphdem_checkpoint_restore(sphdem_ctx* ctx, const void* host, int64_t bytes) 
   ctx->ssr = h.ssr;
   ctx->ng = 0;
   ctx->gridValid = false;
-  ctx->listsValid = false;
+  ctx->listsValid = ctx->listsNear = ctx->hKept = false;
   ctx->loaded = true;
   // the store is in original-index order: sort it with the saved search
   // radius (the grid of the saved state)
@@ -1767,6 +1853,9 @@ static int setField(sphdem_ctx* ctx, int field, const void* src, bool device) {
   }
   FieldLoc L;
   if (!fieldLoc(field, &L)) return fail(ctx, SPHDEM_E_ARG, "unknown or read-only field %d", field);
+  // near lists hold no value of their own: the exact ones, before r or h change
+  if (ctx->listsNear && (field == SPHDEM_FIELD_R || field == SPHDEM_FIELD_H))
+    CHECK(ensureLists(ctx));
   const double* from = (const double*)src;
   if (!device) {
     HIPC(hipMemcpyAsync(ctx->fieldbuf, src, sizeof(double) * L.width * n, hipMemcpyHostToDevice,
@@ -1832,6 +1921,7 @@ int sphdem_sync(sphdem_ctx* ctx) {
 int sphdem_step_start(sphdem_ctx* ctx) {
   CHECK(checkLoaded(ctx));
   HIPC(hipSetDevice(ctx->device));
+  if (ctx->listsNear) CHECK(ensureLists(ctx));  // before r and h change
   CHECK(stepStart(ctx));
   return checkFlags(ctx);
 }
@@ -1887,7 +1977,7 @@ int runOneStep(sphdem_ctx* ctx, int hookset) {
         CHECK(stepStart(ctx, sphMask, g));
       else
         CHECK(stepStart(ctx));
-      CHECK(stepMiddle(ctx));
+      CHECK(stepMiddle(ctx, WrapFold{}, true));
     } else {
       WrapFold fold{};
       fold.mode = 1;
@@ -1900,7 +1990,7 @@ int runOneStep(sphdem_ctx* ctx, int hookset) {
         fold.ay = g[1];
         fold.az = g[2];
       }
-      CHECK(stepMiddle(ctx, fold));
+      CHECK(stepMiddle(ctx, fold, true));
     }
     if (hookset == SPHDEM_HOOKS_SEDIMENT) {  // beforeEnd, sediment3D/customSim.cpp:97-107
       CHECK(hookSumDrag(ctx));
@@ -1913,7 +2003,7 @@ int runOneStep(sphdem_ctx* ctx, int hookset) {
         markStale(ctx, GS_ALL);
       }
     }
-    CHECK(stepEnd(ctx, true));
+    CHECK(stepEnd(ctx, true, true));
     if (hookset == SPHDEM_HOOKS_SEDIMENT) CHECK(hookFreeze(ctx, demMask, ctx->P.time_drop));
   }
   // every buffer a step uses is allocated now (device resets allocate nothing)
@@ -1950,6 +2040,8 @@ HostFields saveHost(const sphdem_ctx* c) {
   h.gcntZeroAt = c->gcntZeroAt;
   h.gstale = c->gstale;
   h.listsValid = c->listsValid;
+  h.listsNear = c->listsNear;
+  h.hKept = c->hKept;
   h.recFresh = c->recFresh;
   h.pvFresh = c->pvFresh;
   h.dFresh = c->dFresh;
@@ -1976,6 +2068,8 @@ void loadHost(sphdem_ctx* c, const HostFields& h) {
   c->gcntZeroAt = h.gcntZeroAt;
   c->gstale = h.gstale;
   c->listsValid = h.listsValid;
+  c->listsNear = h.listsNear;
+  c->hKept = h.hKept;
   c->recFresh = h.recFresh;
   c->pvFresh = h.pvFresh;
   c->dFresh = h.dFresh;
@@ -2110,7 +2204,7 @@ int finishReplays(sphdem_ctx* ctx, int count, int* done, bool* stopped) {
                       ctx->stream));
   HIPC(hipMemcpyAsync(ctx->dg, ctx->dgKeep, sizeof(DevGlobals), hipMemcpyDeviceToDevice,
                       ctx->stream));
-  ctx->listsValid = false;
+  ctx->listsValid = ctx->listsNear = ctx->hKept = false;
   ctx->ng = 0;
   dropGraph(ctx);
   return 0;

@@ -143,14 +143,30 @@ __device__ __forceinline__ float4 mixRecordV(const double4& p, const double4& vh
   return make_float4((float)vh.x, (float)vh.y, (float)vh.z, (float)p.w);
 }
 
+// The near search's record of an SPH-group entry or ghost: its position in
+// Quant's fixed point and, as FP32 rounded up, the square of 2 h in that unit.
+// False (and a zero record) for a non-finite position or a non-positive h.
+__device__ __forceinline__ bool nearRecord(const double4& p, const Quant& Q, uint4& r) {
+  if (!(isfinite(p.x) && isfinite(p.y) && isfinite(p.z) && isfinite(p.w) && p.w > 0.0)) {
+    r = make_uint4(0u, 0u, 0u, 0u);
+    return false;
+  }
+  const double b = 2.0 * p.w * Q.inv;
+  r = make_uint4(quant1(p.x, Q.o[0], Q.inv), quant1(p.y, Q.o[1], Q.inv),
+                 quant1(p.z, Q.o[2], Q.inv),
+                 __float_as_uint((float)fmin(b * b * (1.0 + 1e-6), 1e30)));
+  return true;
+}
+
 // Records a folded reset's permutation writes on the way (WrapFold): the
 // SPH-group entries [0, ns) and the ghosts, from the values it stores.
+enum { REC_NONE, REC_NEAR, REC_EXACT };  // none; k_near's (uint4); k_lists_t's (uint2)
 struct PermRecords {
-  int lists;  // the list search's records (rec; non-finite input to lflag[gen & 1])
+  int lists;  // a search's records (REC_*; non-finite input to lflag[gen & 1])
   int mixed;  // the mixed form's P and V records
   int ns;
   ListQuant lq;
-  uint2* rec;
+  uint4* rec;
   int* lflag;
   int gen;
   Quant Q;

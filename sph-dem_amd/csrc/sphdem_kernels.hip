@@ -574,10 +574,14 @@ __device__ __forceinline__ void ordShift(int ord, int& sx, int& sy, int& sz) {
 // q and vhat-and-mass vh.
 __device__ __forceinline__ void permRecords(const PermRecords& R, int p, const double4& q,
                                             const double4& vh) {
-  if (R.lists) {
+  if (R.lists == REC_NEAR) {
+    uint4 r;
+    if (!nearRecord(q, R.Q, r)) atomicOr(&R.lflag[R.gen & 1], 1);
+    R.rec[p] = r;
+  } else if (R.lists == REC_EXACT) {
     uint2 r;
     if (!listRecord(q, R.lq, r)) atomicOr(&R.lflag[R.gen & 1], 1);
-    R.rec[p] = r;
+    reinterpret_cast<uint2*>(R.rec)[p] = r;
   }
   if (R.mixed) {
     R.P[p] = mixRecordP(q, vh, R.Q);
@@ -1514,13 +1518,16 @@ __global__ void k_dem_kick(Store S, int ns, int nd, sphdem_params P, DevGlobals*
 
 // driftRest + calcEnergies on sph/sphBoundary (sphIncompress.cpp:245-249;
 // sphIncompress.h:678-704, 769-781)
-__global__ void k_end_rest(Store S, int ns, sphdem_params P, DevGlobals* g) {
+// hList (optional): receives the h before driftRest
+__global__ void k_end_rest(Store S, int ns, sphdem_params P, DevGlobals* g,
+                           double* __restrict__ hList) {
   const int a = blockIdx.x * blockDim.x + threadIdx.x;
   if (a >= ns || !isSphT(S.iam[a])) return;
   const double dt = g->dt / 2;
   double4 d = S.dpo[a];
   const double dddt = S.vh0d[a].w;
   d.x += dt * dddt;
+  if (hList) hList[a] = S.posh[a].w;
   if (!(P.flags & SPHDEM_F_CONST_H)) S.posh[a].w = P.hfac * pow_third(S.vhm[a].w / d.x);
   double press;
   if (P.flags & SPHDEM_F_LIQ_DEM)

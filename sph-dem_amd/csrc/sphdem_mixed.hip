@@ -212,7 +212,14 @@ __global__ void __launch_bounds__(256) k_force_m(Store S, int ns, const int* __r
   static_assert(VARH || !OMG, "omega is only fused under VAR_H");
   const int a = xcdThread();
   const double inf = __longlong_as_double(0x7ff0000000000000ll);
-  double newDt = inf;
+  constexpr bool perPair = ARTIF || VISC == VISC_MON;  // the signal speed is the pair's
+  // the least condition so far, by any particle: a bound below which only few
+  // pairs lie (an older value serves as well)
+  double newDt = perPair ? __longlong_as_double((long long)g->newDt_bits) : inf;
+  // the dt conditions 0.6 hav and cdiff hav^2 and their rounded values increase
+  // with h_b: their minima are those of the smallest h_b over the pairs.  minHb
+  // is that of the certain pairs, anyHb of all entries.
+  float minHb = __builtin_inff(), anyHb = __builtin_inff();
   if (a < ns) {
     const bool fluid = S.iam[a] == T_SPH;
     const uint4 qa = Pq[a];
@@ -230,11 +237,10 @@ __global__ void __launch_bounds__(256) k_force_m(Store S, int ns, const int* __r
     const float cs2 = (float)(2.0 * P.spsound), alpha = (float)P.alpha_artificial;
     const float nu198 = (float)(19.8 * P.viscosity), alphaM = (float)monaghanAlpha(P);
     const double vsigC = (VISC == VISC_MOR || VISC == VISC_CLE) ? 2.0 * P.spsound : 0.0;
-    const double cdiff = VISC == VISC_MON ? 0.06 : 0.125;  // viscDiffusionCondition
-    // the dt conditions 0.6 hav and cdiff hav^2 are increasing in hav, and so
-    // are their correctly rounded values: their minima are those of the
-    // smallest hav, taken once at the end
-    double minHav = inf;
+    // certainly a pair of is_neighbr (particle.h:236-238), within 2 ha: the
+    // fixed-point positions move r by less than sqrt(3) res, r2 by less than
+    // 7 ha res, and FP32 rounding r2 by less than 1e-6 of it
+    const float haf = fabsf((float)ha), sure2 = haf * (3.99998f * haf - 8.0f * res);
     // f is the sum of the pressure, viscous and artificial-viscosity parts,
     // added once at the end
     double ax = 0.0, ay = 0.0, az = 0.0, px = 0.0, py = 0.0, pz = 0.0, vx = 0.0, vy = 0.0,
@@ -245,6 +251,8 @@ __global__ void __launch_bounds__(256) k_force_m(Store S, int ns, const int* __r
       SPHDEM_FETCH_ENTRIES(U)
       uint4 q[U];
       float4 v[U], d[U];
+      float vs[U] = {};   // the signal speeds of entries that may be no pairs
+      double low = inf;  // the batch's smallest Courant condition
 #pragma unroll
       for (int u = 0; u < U; u++) {
         q[u] = Pq[e[u]];
@@ -273,6 +281,7 @@ __global__ void __launch_bounds__(256) k_force_m(Store S, int ns, const int* __r
           const float Gbar = 0.5f * (Ga + Gb);
           const double hav = 0.5 * (ha + (double)v[u].w);
           const float havf = (float)hav;
+          const bool sure = dx.r2 < sure2;
           float fvs = 0.0f;  // fv = dv * fvs (Morris)
           float fvr = 0.0f;  // fv = dx * fvr (Cleary, Monaghan)
           float vsig = (float)vsigC;
@@ -307,11 +316,15 @@ __global__ void __launch_bounds__(256) k_force_m(Store S, int ns, const int* __r
             ay += (double)(s * dx.y);
             az += (double)(s * dx.z);
             vsig = fmaxf(vsig, avsig);
-            newDt = dmin2(newDt, 0.6 * hav / (double)vsig);
-          } else if (VISC == VISC_MON) {
-            newDt = dmin2(newDt, 0.6 * hav / (double)vsig);
           }
-          minHav = dmin2(minHav, hav);
+          if (perPair) {
+            const double lim = 0.6 * hav / (double)vsig;
+            newDt = dmin2(newDt, sure ? lim : inf);
+            low = dmin2(low, lim);
+            vs[u] = sure ? 0.0f : vsig;
+          }
+          anyHb = fminf(anyHb, v[u].w);
+          minHb = fminf(minHb, sure ? v[u].w : __builtin_inff());
           constexpr bool alongDr = VISC == VISC_CLE || VISC == VISC_MON;
           const double f0 = (double)(alongDr ? dx.x * fvr : dv0 * fvs);
           const double f1 = (double)(alongDr ? dx.y * fvr : dv1 * fvs);
@@ -326,10 +339,14 @@ __global__ void __launch_bounds__(256) k_force_m(Store S, int ns, const int* __r
         py += q1;
         pz += q2;
       }
-    }
-    if (minHav != inf) {
-      if (!ARTIF && VISC != VISC_MON) newDt = dmin2(newDt, (0.6 * minHav) / vsigC);
-      newDt = dmin2(newDt, (cdiff * (minHav * minHav)) / P.viscosity);
+      if (perPair && low < newDt)  // by an entry that may be no pair
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+          const double lim = 0.6 * (0.5 * (ha + (double)v[u].w)) / (double)vs[u];
+          if (vs[u] > 0.0f && lim < newDt &&
+              pairWithin(S.posh[a], S.posh[nbl[nbEntry(k0 + u, a, ns)]]))
+            newDt = lim;
+        }
     }
     double fx = px + vx + ax, fy = py + vy + ay, fz = pz + vz + az;
     if (OMG) {
@@ -359,6 +376,32 @@ __global__ void __launch_bounds__(256) k_force_m(Store S, int ns, const int* __r
     S.frc[a] = f;
     S.fp[a] = fpa;
     S.fv[a] = fva;
+  }
+  // a particle whose smallest entry may be no pair and would set the wavefront's
+  // condition: the wavefront goes through its list by the FP64 test, a lane per
+  // entry
+  const int lane = threadIdx.x & 63;
+  const double vsigC = (VISC == VISC_MOR || VISC == VISC_CLE) ? 2.0 * P.spsound : 0.0;
+  const double cdiff = VISC == VISC_MON ? 0.06 : 0.125;  // viscDiffusionCondition
+  const double ha = a < ns ? S.posh[a].w : 0.0;
+  auto lower = [&](float hb) {  // the conditions of the smallest h_b
+    if (hb == __builtin_inff()) return inf;
+    const double hav = 0.5 * (ha + (double)hb);
+    const double m = (cdiff * (hav * hav)) / P.viscosity;
+    return perPair ? m : dmin2((0.6 * hav) / vsigC, m);
+  };
+  newDt = dmin2(newDt, lower(minHb));
+  const double sureDt = waveMin(newDt), lowDt = lower(anyHb);
+  for (unsigned long long todo = __ballot(lowDt < sureDt); todo; todo &= todo - 1) {
+    const int s = __builtin_ctzll(todo), as = __builtin_amdgcn_readlane(a, s);
+    const double4 pa = S.posh[as];
+    double x = inf;
+    for (int k = lane, n = nbcnt[as]; k < n; k += 64) {
+      const int j = nbl[nbEntry(k, as, ns)];
+      if (pairWithin(pa, S.posh[j])) x = dmin2(x, (double)V[j].w);
+    }
+    x = waveMin(x);
+    if (lane == s) newDt = dmin2(newDt, lower((float)x));
   }
   atomicMinPos(&g->newDt_bits, newDt);
 }

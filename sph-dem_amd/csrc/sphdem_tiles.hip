@@ -442,6 +442,413 @@ __global__ void __launch_bounds__(256) k_lists_t(const double4* __restrict__ pos
   nbcnt[t] = c;
 }
 
+// ---- near lists: the step's own search -----------------------------------------------
+// A superset of the lists above for the step's pair walks, in the same order:
+// every SPH neighbour within 2 max(h) and a few just beyond, whose kernel
+// terms are exactly zero (the walks take the pairs of the dt conditions by the
+// FP64 test).  So no candidate needs the FP64 test here, and the distance
+// tests run on the matrix cores.
+//
+// A workgroup takes a tile of 64 consecutive targets of the cell-sorted store,
+// lane l of every wavefront owning target l.  Its W = 3 wavefronts take the
+// columns of x - 1, x and x + 1 (W = 9: one column each): each streams the
+// candidates of its columns (y order; the cells one below the first target's
+// to one above the last's; in a column holding ghosts each cell's real part,
+// then its ghosts) 64 at a time, and eight 32x32x2 products give the 64 x 64
+// squared distances.
+//
+// The products run on records of 32-bit fixed point over the grid (Quant) with
+// the radius's square T_b = (2 h_b)^2.  A pair's radius squared, the larger of
+// T_a and T_b, is at most T_a + T_b - T0 with T0 no larger than either: T0 is
+// the smallest T_a of the targets at hand, and T_b is raised to it.  (It is
+// that larger one exactly where all h are equal, and beyond it by no more than
+// the targets' h differ.)  Relative to an origin near the first target, as FP32,
+//   (|b|^2 - T_b) - 2 a.b + (|a|^2 - T_a + T0)
+// is a sum of four products, two 32x32x2 products, and negative for a pair.
+// The stencil reaches two edges across and 3.5 along the column, so the terms
+// stay below 40 edge^2: the rounding of the sums (7 x 2.4e-6), of |b|^2 (4e-6)
+// and of the coordinates (7e-6 on the largest grid) stays below kNearSlack =
+// 6e-5 edge^2, by which T_a is raised: 3e-5 of the radius.  (Where a T is
+// larger than that, its own rounding is, too, but every candidate lies far
+// inside it.)
+//
+// Each lane's sign bits over 32 candidates make one mask word.  The words wait
+// in LDS; when the wavefronts know their counts, every lane pops its entries
+// behind those of the columns before, four at a time into one 16-byte store.
+//
+// What bounds it: vector instructions (64 sign folds, and some 40 of placing
+// and masks, a batch; some 15 an entry popped) at four wavefronts a SIMD, and
+// in a small box the chain of them.  Half the products are skipped where only
+// the cells of the other 32 targets reach a batch, and a batch's records are
+// fetched while the one before is tested.  In place of the FP64 tests of a
+// thread per target (k_lists_t, 125 us a build of a 16^3 box, 199 of 64^3, 701
+// of a 95^3, 2710 of a 160^3): 44, 125, 448 and 1890 us.
+typedef float float16v __attribute__((ext_vector_type(16)));
+// A record relative to the origin o, and its squared length.
+struct NearPoint {
+  float x, y, z, b2;
+};
+__device__ __forceinline__ NearPoint nearPoint(const uint4& r, unsigned ox, unsigned oy,
+                                               unsigned oz) {
+  NearPoint p;
+  p.x = (float)(int)(r.x - ox);
+  p.y = (float)(int)(r.y - oy);
+  p.z = (float)(int)(r.z - oz);
+  p.b2 = p.x * p.x + p.y * p.y + p.z * p.z;
+  return p;
+}
+// One operand of the products for rows (or columns) 0-31 and one for 32-63:
+// lane l of the first holds item l % 32, the first term in the lower half of
+// the wavefront and the second in the upper.
+struct NearOperand {
+  float lo, hi;
+};
+__device__ __forceinline__ NearOperand nearOperand(float a, float b) {
+  const auto s =
+      __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+  return NearOperand{__uint_as_float(s[0]), __uint_as_float(s[1])};
+}
+// m = (m << 16) | the sign bits of v, first element highest
+__device__ __forceinline__ unsigned foldSigns(unsigned m, const float16v& v) {
+#pragma unroll
+  for (int i = 0; i < 16; i++) m = __builtin_amdgcn_alignbit(m, __float_as_uint(v[i]), 31);
+  return m;
+}
+// The near search's records of the SPH-group entries [0, ns) and the ghosts
+// [n, n + ng); flag slots as for k_lrec.
+__global__ void k_near_rec(const double4* __restrict__ posh, int ns, int n, int ng, Quant Q,
+                           uint4* __restrict__ rec, int* __restrict__ lflag, int gen,
+                           const int* __restrict__ ngp) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i == 0) lflag[(gen + 1) & 1] = 0;
+  if (i >= ns + (ngp ? min(*ngp, ng) : ng)) return;
+  const int s = i < ns ? i : n + (i - ns);
+  uint4 r;
+  if (!nearRecord(posh[s], Q, r)) atomicOr(&lflag[gen & 1], 1);
+  rec[s] = r;
+}
+// bits [32 - k, 32) set: the first k of a word's candidates
+__device__ __forceinline__ unsigned highBits(int k) {
+  return k >= 32 ? ~0u : (k <= 0 ? 0u : ~(~0u >> k));
+}
+
+constexpr float kNearSlack = 6e-5f;
+constexpr int kNearSpan = 4;    // cells along z the targets of one group span at most
+// LDS words per lane of a wavefront: masks from below, index maps from above
+constexpr int nearSlots(int waves) { return waves == 3 ? 32 : 20; }
+template <int SLOTS>
+struct NearWave {
+  unsigned word[SLOTS][64];
+  int base[SLOTS];       // a word's first candidate, or ~ its place in the maps
+  int count[64];         // entries of the slab
+  int over;              // the slab's words or maps did not fit
+};
+
+// Grid: 8 * ceil(ns / 512) workgroups, one per tile of 64 targets; XCD
+// blockIdx % 8 takes the corresponding eighth of the tiles (a spatially
+// coherent slab for its L2).  A target whose near list would not fit kMaxNb
+// entries or whose slab overflows, and every target where the records are no
+// bounds (a non-finite position or a non-positive h anywhere: lflag), gets its
+// exact list.
+template <int W>
+__global__ void __launch_bounds__(64 * W, W == 3 ? 4 : 3)
+    k_near(const double4* __restrict__ pos, const uint4* __restrict__ rec,
+           const int* __restrict__ cellc, Grid g, int gbase, const int* __restrict__ start, int ns,
+           double qinv, const int* __restrict__ lflag, int gen, int* __restrict__ nbl,
+           int* __restrict__ nbcnt, DevGlobals* dg) {
+  constexpr int kNearSlots = nearSlots(W);
+  __shared__ NearWave<kNearSlots> lds[W];
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  NearWave<kNearSlots>& L = lds[w];
+  const int t0 = ((int)(blockIdx.x & 7) * ((ns + 511) >> 9) + (int)(blockIdx.x >> 3)) << 6;
+  if (t0 >= ns) return;  // uniform per workgroup
+  const int t = t0 + lane;
+  const bool act = t < ns;
+  const CPtr<int> cstart = (CPtr<int>)start;
+  const int tl = act ? t : t0;
+  const uint4 own = rec[tl];
+  const float ownT = __uint_as_float(own.w);
+  const int cell = cellc[tl], cz = cellZ(cell);
+  const double eu = g.edge * qinv;  // the edge in the records' unit
+  const float slack = kNearSlack * (float)(eu * eu);
+  const unsigned up = (unsigned)(1.5 * eu);
+  // the candidate a lane loads of 64: row l % 32 of product tile l / 32, placed
+  // so that a lane's sums of tile t and element i belong to candidate
+  // 32 (lane / 32) + 16 t + i
+  const int cand = ((lane >> 2) & 1) * 32 + (lane >> 5) * 16 + ((lane >> 3) & 3) * 4 + (lane & 3);
+
+  unsigned long long exact = 0ull;  // targets left to the exact search
+  unsigned long long todo = __ballot(act);
+  if (lflag[gen & 1] != 0) {
+    exact = todo;
+    todo = 0ull;
+  }
+  while (todo) {
+    // a group: targets of one column whose cells span at most kNearSpan
+    const int lead = __builtin_ctzll(todo);
+    const int lcell = __builtin_amdgcn_readlane(cell, lead);
+    const int X = cellX(lcell) - 1 + w / (W / 3), cy = cellY(lcell), z0 = cellZ(lcell);
+    const unsigned long long grp =
+        __ballot(((todo >> lane) & 1) && cellX(cell) == cellX(lcell) && cellY(cell) == cy &&
+                 cz >= z0 && cz < z0 + kNearSpan);
+    todo &= ~grp;
+    const bool in = (grp >> lane) & 1;
+
+    // ---- the mask words of the slab x = cx - 1 + w
+    int pend = 0;     // entries
+    unsigned bm = 0;  // the slots (slot 0 highest) that hold them
+    int nslot = 0, nmap = 0;
+    bool over = false;
+    if (X >= 0 && X < g.dim[0]) {
+      const int z1 = __builtin_amdgcn_readlane(cz, 63 - __builtin_clzll(grp));
+      const int Z0 = max(z0 - 1, 0), Z1 = min(z1 + 1, g.dim[2] - 1);
+      // cells around the group's targets 0-31 and 32-63
+      const unsigned glo = (unsigned)grp, ghi = (unsigned)(grp >> 32);
+      const int zl1 = glo ? __builtin_amdgcn_readlane(cz, 31 - __builtin_clz(glo)) : Z0;
+      const int zh0 = ghi ? __builtin_amdgcn_readlane(cz, 32 + __builtin_ctz(ghi)) : Z1 + 1;
+      // The columns' bounds, one load: lanes 16 y + i the first entry of cell Z0 + i
+      // (i = 7: the column's end), lanes 16 y + 8 + i its first ghost.
+      int bound = 0;
+      {
+        const int Y = cy + (W == 3 ? -1 + (lane >> 4) : -1 + w % 3);
+        const bool ghost = (lane & 8) != 0;
+        if ((lane >> 4) < 9 / W && Y >= 0 && Y < g.dim[1] && (!ghost || gbase > 0))
+          bound = start[(ghost ? gbase : g.base) + (X * g.dim[1] + Y) * g.dim[2] +
+                        min(Z0 + (lane & 7), Z1 + 1)];
+      }
+      // the origin: the first target, 1.5 cells up (its column's stencil reaches
+      // two cells down and five up)
+      const unsigned ox = __builtin_amdgcn_readlane(own.x, lead);
+      const unsigned oy = __builtin_amdgcn_readlane(own.y, lead);
+      const unsigned oz = (unsigned)__builtin_amdgcn_readlane(own.z, lead) + up;
+      const NearPoint a = nearPoint(own, ox, oy, oz);
+      const NearOperand Bxy = nearOperand(-2.0f * a.x, -2.0f * a.y);
+      const NearOperand Bzb = nearOperand(-2.0f * a.z, 1.0f);
+      float least = in ? ownT : __builtin_inff();
+      for (int d = 32; d > 0; d >>= 1) least = fminf(least, __shfl_xor(least, d, 64));
+      float16v c0, c1;
+      {
+        const unsigned v = __float_as_uint(in ? a.b2 - (ownT - least + slack) : 1e30f);
+        const auto s = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+#pragma unroll
+        for (int i = 0; i < 16; i++) {
+          c0[i] = __uint_as_float(s[0]);
+          c1[i] = __uint_as_float(s[1]);
+        }
+      }
+
+      // candidates base + (0 .. 63) (or, base < 0, those of a map), the first k
+      // valid, rc this lane's record; self: the target's own place among them
+      auto test = [&](const uint4& rc, int base, int k, int self, bool lower, bool upper) {
+        const NearPoint b = nearPoint(rc, ox, oy, oz);
+        const NearOperand Axy = nearOperand(b.x, b.y);
+        const NearOperand Azb =
+            nearOperand(b.z, b.b2 - fmaxf(__uint_as_float(rc.w), least));
+        auto signs = [&](float colXy, float colZb, const float16v& c) {
+          auto half = [&](unsigned m, float xy, float zb) {
+            return foldSigns(
+                m, __builtin_amdgcn_mfma_f32_32x32x2f32(
+                       xy, colXy, __builtin_amdgcn_mfma_f32_32x32x2f32(zb, colZb, c, 0, 0, 0), 0,
+                       0, 0));
+          };
+          return half(half(0u, Axy.lo, Azb.lo), Axy.hi, Azb.hi);
+        };
+        // lane l: words of targets l % 32 and 32 + l % 32; then of target l
+        const unsigned m0 = lower ? signs(Bxy.lo, Bzb.lo, c0) : 0u;
+        const unsigned m1 = upper ? signs(Bxy.hi, Bzb.hi, c1) : 0u;
+        const auto words = __builtin_amdgcn_permlane32_swap(m0, m1, false, false);
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+          unsigned v = highBits(k - 32 * h);
+          if ((unsigned)(self - 32 * h) < 32u) v &= ~(0x80000000u >> (self - 32 * h));
+          const unsigned yes = words[h] & v;
+          if (__ballot(yes != 0u) == 0ull) continue;
+          L.word[nslot][lane] = yes;
+          if (lane == 0) L.base[nslot] = base >= 0 ? base + 32 * h : ~(~base + 32 * h);
+          pend += __popc(yes);
+          if (yes) bm |= 0x80000000u >> nslot;
+          nslot++;
+        }
+      };
+      // the batches of 64 candidates: column y, from its entry p on
+      int y = -1, p = 0, total = 0, J0 = 0, J1 = 0;
+      bool ghosts = false;
+      auto at = [&](int i) { return __builtin_amdgcn_readlane(bound, 16 * y + i); };
+      auto advance = [&]() {
+        p += 64;
+        while (p >= total) {
+          if (++y == 9 / W) return false;
+          J0 = at(0), J1 = at(7);
+          const int ng = at(15) - at(8);
+          ghosts = ng != 0;
+          total = J1 - J0 + ng;
+          p = 0;
+        }
+        return true;
+      };
+      // this lane's candidate, and its target's own place in the batch
+      int j = 0, self = -1;
+      auto locate = [&]() {
+        const bool mid = w / (W / 3) == 1 && (W == 3 ? y == 1 : w % 3 == 1) && in;
+        j = J0 + p + cand;
+        self = mid ? t - (J0 + p) : -1;
+        if (ghosts) {  // each cell's real part, then its ghosts
+          const int c = p + cand;
+          int off = 0;
+          j = t0;
+          self = -1;
+          for (int i = 0; i < Z1 - Z0 + 1; i++) {
+            const int r0 = at(i), nr = at(i + 1) - r0, h0 = at(8 + i), nh = at(9 + i) - h0;
+            if (mid && cz == Z0 + i) self = off + (t - r0) - p;
+            if (c >= off && c < off + nr) j = r0 + (c - off);
+            off += nr;
+            if (c >= off && c < off + nh) j = h0 + (c - off);
+            off += nh;
+          }
+        }
+      };
+      bool more = advance();
+      uint4 next = make_uint4(0u, 0u, 0u, 0u);
+      if (more) {
+        locate();
+        next = rec[j];
+      }
+      while (more) {
+        if (nslot + nmap + 3 > kNearSlots) {
+          over = true;
+          break;
+        }
+        const uint4 rc = next;
+        const int k = total - p, me = self;
+        int base = J0 + p;
+        bool lower = glo != 0u, upper = ghi != 0u;
+        if (ghosts) {
+          nmap++;
+          L.word[kNearSlots - nmap][cand] = (unsigned)j;
+          base = ~((kNearSlots - nmap) * 64);
+        } else {
+          lower = lower && base < at(min(zl1 + 1, Z1) + 1 - Z0);
+          upper = upper && base + 64 > at(max(zh0 - 1, Z0) - Z0);
+        }
+        more = advance();
+        if (more) {
+          locate();
+          next = rec[j];
+        }
+        test(rc, base, k, me, lower, upper);
+      }
+    }
+
+    // ---- each slab's entries behind those of the slabs before it
+    L.count[lane] = pend;
+    if (lane == 0) L.over = over ? 1 : 0;
+    __syncthreads();
+    int all = 0, pos0 = 0;
+    bool bad = false;
+#pragma unroll
+    for (int i = 0; i < W; i++) {
+      if (i == w) pos0 = all;
+      all += lds[i].count[lane];
+      bad |= lds[i].over != 0;
+    }
+    exact |= __ballot(in && (bad || all > kMaxNb));
+    if ((exact >> lane) & 1) pend = 0;
+    if (in && w == 0 && !((exact >> lane) & 1)) nbcnt[t] = all;
+    // the word in hand and the one behind it, on its way from LDS
+    unsigned m = 0, m1 = 0;
+    int base = 0, base1 = 0;
+    auto fetch = [&]() {
+      const int s = bm ? __builtin_clz(bm) : 0;
+      bm &= ~(0x80000000u >> s);
+      m1 = L.word[s][lane];
+      base1 = L.base[s];
+    };
+    fetch();
+    auto pop = [&]() {
+      if (m == 0) {
+        m = m1;
+        base = base1;
+        fetch();
+      }
+      const int bit = __builtin_clz(m);
+      m &= ~(0x80000000u >> bit);
+      return base >= 0 ? base + bit : (int)(&L.word[0][0])[~base + bit];
+    };
+    // single entries up to a multiple of four, then 16-byte pieces, then single
+    // entries
+#pragma unroll 1
+    for (int part = 0; part < 2; part++) {
+      while (__any(pend > 0 && (part || (pos0 & 3) != 0)))
+        if (pend > 0 && (part || (pos0 & 3) != 0)) {
+          nbl[nbEntry(pos0, t, ns)] = pop();
+          pos0++;
+          pend--;
+        }
+      if (part) break;
+      while (__any(pend >= 4))
+        if (pend >= 4) {
+          const int e0 = pop(), e1 = pop(), e2 = pop(), e3 = pop();
+          *reinterpret_cast<int4*>(nbl + nbEntry(pos0, t, ns)) = make_int4(e0, e1, e2, e3);
+          pos0 += 4;
+          pend -= 4;
+        }
+    }
+    __syncthreads();
+  }
+
+  // ---- exact lists: the FP64 test of is_neighbr (particle.h:236-238) over the
+  // 27 cells, a lane per candidate; the wavefronts take the targets in turn
+  for (; exact; exact &= exact - 1) {
+    const int s = __builtin_ctzll(exact);
+    if (s % W != w) continue;
+    const int scell = __builtin_amdgcn_readlane(cell, s), st = t0 + s;
+    const double4 p = pos[st];
+    const double lima2 = (2.0 * p.w) * (2.0 * p.w);
+    int c = 0;
+    for (int X = max(cellX(scell) - 1, 0); X <= min(cellX(scell) + 1, g.dim[0] - 1); X++)
+      for (int Y = max(cellY(scell) - 1, 0); Y <= min(cellY(scell) + 1, g.dim[1] - 1); Y++)
+        for (int z = max(cellZ(scell) - 1, 0); z <= min(cellZ(scell) + 1, g.dim[2] - 1); z++)
+          for (int part = 0; part < (gbase > 0 ? 2 : 1); part++) {
+            const int k = (part ? gbase : g.base) + (X * g.dim[1] + Y) * g.dim[2] + z;
+            for (int j0 = cstart[k]; j0 < cstart[k + 1]; j0 += 64) {
+              const int j = j0 + lane;
+              bool ok = false;
+              if (j < cstart[k + 1] && j != st) {
+                const double4 q = pos[j];
+                const double dx = p.x - q.x, dy = p.y - q.y, dz = p.z - q.z;
+                const double l2 = dot3(dx, dy, dz, dx, dy, dz);
+                const double hb2 =
+                    __longlong_as_double(__double_as_longlong(q.w) + (1ll << 52));
+                ok = l2 <= fmax(lima2, hb2 * hb2);
+              }
+              const unsigned long long m = __ballot(ok);
+              const int at = c + (int)__builtin_amdgcn_mbcnt_hi(
+                                     (unsigned)(m >> 32),
+                                     __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
+              if (ok && at < kMaxNb) nbl[nbEntry(at, st, ns)] = j;
+              c += __popcll(m);
+            }
+          }
+    if (lane == 0) {
+      if (c > kMaxNb) atomicOr(&dg->errflags, 2u);
+      nbcnt[st] = min(c, kMaxNb);
+    }
+  }
+}
+
+// Positions with another h (hList, of real entries) for a list search: the
+// SPH-group entries [0, ns) and the ghosts [n, n + ng), whose h is their
+// origin's.
+__global__ void k_list_pos(const double4* __restrict__ posh, const double* __restrict__ hList,
+                           int ns, int n, int ng, const int* __restrict__ gorig,
+                           double4* __restrict__ out) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= ns + ng) return;
+  const int e = i < ns ? i : n + (i - ns);
+  const double4 p = posh[e];
+  out[e] = make_double4(p.x, p.y, p.z, hList[i < ns ? i : gorig[i - ns]]);
+}
+
 // The cached lists as (a, b, image) triples of original indices, for the
 // parity enumeration of the SPH pair set: a ghost neighbour reports its
 // origin and its image code.
@@ -631,14 +1038,18 @@ __global__ void __launch_bounds__(256, 3) k_dddt_l(Store S, int ns, Box B,
   S.vh0d[a].w = dddt;
 }
 
+// is_neighbr (particle.h:236-238) of two entries
+__device__ __forceinline__ bool pairWithin(const double4& pa, const double4& pb) {
+  const double x = pa.x - pb.x, y = pa.y - pb.y, z = pa.z - pb.z;
+  const double l = 2.0 * dmax2(fabs(pa.w), fabs(pb.w));
+  return dot3(x, y, z, x, y, z) <= l * l;
+}
 // ---- calcForce (sphIncompress.h:899-972; sph.h:579-666, 692-734) over the list --
 // One instantiation per combination of the flags that change the pair
 // arithmetic (VISC: the viscosity variant, VISC_NONE..VISC_MON).  The per-pair
-// dt conditions (sph.h:545-560) are min-reduced into newDt_bits.  When the
-// signal speed is the constant 2*SPSOUND (or 0) -- Morris or Cleary without
-// artificial viscosity -- x -> RN(x/c) is monotone, so the minimum over pairs
-// of RN(0.6*hav / vsig) is RN(min(0.6*hav) / vsig): the numerators are
-// min-reduced and divided once (likewise c_diff*hav^2 / VISCOSITY).
+// dt conditions (sph.h:545-560) are min-reduced into newDt_bits: those of the
+// artificial and Monaghan viscosities pair by pair, the others, whose signal
+// speed is constant, through the smallest neighbour h.
 //
 // OMG (VAR_H only): calcOmega fused into the same walk.  Under VAR_H every
 // force term of a is linear in 1/omega_a and in nothing else of omega
@@ -674,7 +1085,9 @@ __global__ void __launch_bounds__(256) k_force_l(Store S, int ns, Box B,
     const double vsigC = (VISC == VISC_MOR || VISC == VISC_CLE) ? 2.0 * P.spsound : 0.0;
     const double cdiff = VISC == VISC_MON ? 0.06 : 0.125;  // viscDiffusionCondition
     const double alphaM = monaghanAlpha(P);
-    double minA = inf, minB = inf;  // min over pairs of 0.6*hav and cdiff*hav^2
+    // 0.6 hav and cdiff hav^2 and their rounded values increase with h_b: their
+    // minima are those of the smallest h_b, formed once at the end
+    double minHb = inf;
     const double4 zero4 = make_double4(0.0, 0.0, 0.0, 0.0);
     double4 f = OMG ? zero4 : S.frc[a], fpa = OMG ? zero4 : S.fp[a], fva = OMG ? zero4 : S.fv[a];
     const int n = nbcnt[a];
@@ -709,6 +1122,10 @@ __global__ void __launch_bounds__(256) k_force_l(Store S, int ns, Box B,
           const double dv0 = va.x - v[u].x, dv1 = va.y - v[u].y, dv2 = va.z - v[u].z;
           const double Gbar = 0.5 * (Ga + Gb);  // gradW-bar = dr * Gbar
           const double hav = 0.5 * (ha + hb);
+          // the dt conditions are those of the pairs of is_neighbr
+          // (particle.h:236-238): a near list also holds others
+          const double lim = 2.0 * dmax2(fabs(ha), fabs(hb));
+          const bool isPair = l2 <= lim * lim;
           double fvs = 0.0;  // fv = dv * fvs (Morris)
           double fvr = 0.0;  // fv = dr * fvr (Cleary, Monaghan: m_b visc gradW-bar)
           double vsig = vsigC;
@@ -744,13 +1161,9 @@ __global__ void __launch_bounds__(256) k_force_l(Store S, int ns, Box B,
             f.y += sg * dy;
             f.z += sg * dz;
             vsig = dmax2(vsig, avsig);
-            newDt = dmin2(newDt, 0.6 * hav / vsig);
-          } else if (VISC == VISC_MON) {
-            newDt = dmin2(newDt, 0.6 * hav / vsig);
-          } else {
-            minA = dmin2(minA, 0.6 * hav);
           }
-          minB = dmin2(minB, cdiff * (hav * hav));
+          if (ARTIF || VISC == VISC_MON) newDt = dmin2(newDt, isPair ? 0.6 * hav / vsig : inf);
+          minHb = dmin2(minHb, isPair ? hb : inf);
           constexpr bool alongDr = VISC == VISC_CLE || VISC == VISC_MON;
           const double fv0 = alongDr ? dx * fvr : dv0 * fvs;
           const double fv1 = alongDr ? dy * fvr : dv1 * fvs;
@@ -774,8 +1187,11 @@ __global__ void __launch_bounds__(256) k_force_l(Store S, int ns, Box B,
         f.z += p2;
       }
     }
-    if (!ARTIF && VISC != VISC_MON && minA != inf) newDt = dmin2(newDt, minA / vsigC);
-    if (minB != inf) newDt = dmin2(newDt, minB / P.viscosity);
+    if (minHb != inf) {
+      const double hav = 0.5 * (ha + minHb);
+      if (!ARTIF && VISC != VISC_MON) newDt = dmin2(newDt, 0.6 * hav / vsigC);
+      newDt = dmin2(newDt, cdiff * (hav * hav) / P.viscosity);
+    }
     if (OMG) {
       const double omega = 1 + ha * om / (da.x * 3);
       S.dpo[a].z = omega;
