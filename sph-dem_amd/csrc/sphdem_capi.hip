@@ -126,7 +126,7 @@ struct sphdem_ctx {
   Grid gs{}, gc{};
   Box box{};
   CouplingRule rule{};
-  int K = 0, reachShep = 1, reachFull = 1;
+  int K = 0, reachShep = 1;
   bool loaded = false;
   // measurement window: events bracketing each launch of one kernel
   int timedKernel = -1;
@@ -370,26 +370,31 @@ int ensureKeys(sphdem_ctx* ctx, int K) {
   return 0;
 }
 
-// exclusive scan of in[0..m) into out (m <= SCAN_TILE^2); copyLast (device,
-// optional) also receives out[m - 1]
-int scanInts(sphdem_ctx* ctx, const int* in, int* out, int m, int* copyLast = nullptr) {
+// exclusive scan of in[0..nin), then zeros, into out[0..m) (m <= SCAN_TILE^2);
+// copyLast (device, optional) also receives out[m - 1]
+template <class T>
+int scanItems(sphdem_ctx* ctx, const int* in, int nin, T* out, int m, T* copyLast = nullptr) {
   const int tiles = (m + SCAN_TILE - 1) / SCAN_TILE;
   if (tiles > SCAN_TILE) return fail(ctx, SPHDEM_E_CAPACITY, "scan of %d items", m);
   if (tiles + 1 > ctx->tileCap) {
     if (ctx->tiles) HIPC(hipFree(ctx->tiles));
     ctx->tileCap = tiles + 1 + (tiles + 1) / 4;
-    HIPC(hipMalloc(&ctx->tiles, sizeof(int) * ctx->tileCap));
+    HIPC(hipMalloc(&ctx->tiles, sizeof(long long) * ctx->tileCap));
     ctx->allocEpoch++;
   }
-  hipLaunchKernelGGL(k_scan_tile, dim3(tiles), dim3(SCAN_THREADS), 0, ctx->stream, in, out,
-                     ctx->tiles, m, tiles == 1 ? copyLast : (int*)nullptr);
+  T* sums = reinterpret_cast<T*>(ctx->tiles);
+  hipLaunchKernelGGL(k_scan_tile<T>, dim3(tiles), dim3(SCAN_THREADS), 0, ctx->stream, in, nin, out,
+                     sums, m, tiles == 1 ? copyLast : (T*)nullptr);
   LAUNCHED();
   if (tiles > 1) {
-    hipLaunchKernelGGL(k_scan_add, dim3(tiles), dim3(SCAN_THREADS), 0, ctx->stream, out,
-                       ctx->tiles, m, copyLast);
+    hipLaunchKernelGGL(k_scan_add<T>, dim3(tiles), dim3(SCAN_THREADS), 0, ctx->stream, out, sums, m,
+                       copyLast);
     LAUNCHED();
   }
   return 0;
+}
+int scanInts(sphdem_ctx* ctx, const int* in, int* out, int m, int* copyLast = nullptr) {
+  return scanItems<int>(ctx, in, m, out, m, copyLast);
 }
 int scanCounts(sphdem_ctx* ctx, int m) { return scanInts(ctx, ctx->counts, ctx->start, m); }
 
@@ -575,8 +580,6 @@ void setupGrids(sphdem_ctx* ctx) {
   if (liqDem(ctx)) {
     const double Rc = P.coupling_radius;
     ctx->reachShep = std::max(1, (int)ceil(Rc * (1.0 + 1e-9) / gs.edge));
-    ctx->reachFull =
-        (int)ceil((ctx->rule.nc + 1) * ctx->rule.e / gc.edge) + 1;
   }
 }
 
@@ -2635,39 +2638,37 @@ static int getPairs(sphdem_ctx* ctx, int kind, int64_t* count, int32_t* a, int32
     ctx->pairCap = 0;
     const int cap = nq + nq / 4;
     HIPC(hipMalloc(&ctx->pairCnt, sizeof(int) * cap));
-    HIPC(hipMalloc(&ctx->pairOff, sizeof(long long) * cap));
+    HIPC(hipMalloc(&ctx->pairOff, sizeof(long long) * (cap + 1)));
     ctx->pairCap = cap;
   }
-  int* cnt = ctx->pairCnt;
   long long* off = ctx->pairOff;
-  HIPC(hipMemsetAsync(cnt, 0, sizeof(int) * nq, ctx->stream));
-  auto enumerate = [&](int mode, const long long* o, int* da, int* db, int* di) -> int {
+  const double half = (ctx->rule.nc + 2) * ctx->rule.e * (1.0 + 1e-6);
+  auto enumerate = [&](int mode, int* da, int* db, int* di) -> int {
     if (kind == SPHDEM_PAIRS_SPH) {
-      if (mode == 0)
-        HIPC(hipMemcpyAsync(cnt, ctx->nbcnt, sizeof(int) * nq, hipMemcpyDeviceToDevice,
-                            ctx->stream));
+      if (mode == 0) return 0;  // nbcnt
+      hipLaunchKernelGGL(k_list_pairs, dim3((nq + 3) / 4), dim3(TPB), 0, ctx->stream, ctx->cur,
+                         ctx->ns, ctx->n, ctx->nbl, ctx->nbcnt, ctx->gcode, off, da, db, di);
+    } else {
+      auto launch = [&](auto kernel, int lanes) {
+        const int per = TPB / lanes;
+        hipLaunchKernelGGL(kernel, dim3((nq + per - 1) / per), dim3(TPB), 0, ctx->stream, ctx->cur,
+                           ctx->ns, ctx->nd, kind, ctx->gs, ctx->gc, ctx->start, ctx->box,
+                           ctx->rule, half, mode, ctx->pairCnt, off, da, db, di);
+      };
+      if (kind == SPHDEM_PAIRS_DEM2SPH)
+        launch(k_pairs<64>, 64);
       else
-        hipLaunchKernelGGL(k_list_pairs, dim3(blocks(nq)), dim3(TPB), 0, ctx->stream, ctx->cur,
-                           ctx->ns, ctx->n, ctx->nbl, ctx->nbcnt, ctx->gcode, o, da, db, di);
-      LAUNCHED();
-      return 0;
+        launch(k_pairs<16>, 16);
     }
-    hipLaunchKernelGGL(k_pairs, dim3(blocks(nq)), dim3(TPB), 0, ctx->stream, ctx->cur, ctx->ns,
-                       ctx->nd, kind, ctx->gs, ctx->gc, ctx->start, ctx->box, ctx->rule,
-                       ctx->reachFull, mode, cnt, o, da, db, di);
     LAUNCHED();
     return 0;
   };
-  CHECK(enumerate(0, nullptr, nullptr, nullptr, nullptr));
-  std::vector<int> hc(nq);
-  HIPC(hipMemcpyAsync(hc.data(), cnt, sizeof(int) * nq, hipMemcpyDeviceToHost, ctx->stream));
-  HIPC(hipStreamSynchronize(ctx->stream));
-  std::vector<long long> ho(nq);
+  CHECK(enumerate(0, nullptr, nullptr, nullptr));
   long long tot = 0;
-  for (int i = 0; i < nq; i++) {
-    ho[i] = tot;
-    tot += hc[i];
-  }
+  CHECK(scanItems<long long>(ctx, kind == SPHDEM_PAIRS_SPH ? ctx->nbcnt : ctx->pairCnt, nq, off,
+                             nq + 1));
+  HIPC(hipMemcpyAsync(&tot, off + nq, sizeof(long long), hipMemcpyDeviceToHost, ctx->stream));
+  HIPC(hipStreamSynchronize(ctx->stream));
   *count = tot;
   if (a && b && image && tot > 0) {
     if (tot > capacity)
@@ -2682,8 +2683,7 @@ static int getPairs(sphdem_ctx* ctx, int kind, int64_t* count, int32_t* a, int32
       HIPC(hipMalloc(&db, sizeof(int) * tot));
       HIPC(hipMalloc(&di, sizeof(int) * tot));
     }
-    HIPC(hipMemcpyAsync(off, ho.data(), sizeof(long long) * nq, hipMemcpyHostToDevice, ctx->stream));
-    CHECK(enumerate(1, off, da, db, di));
+    CHECK(enumerate(1, da, db, di));
     if (!device) {
       HIPC(hipMemcpyAsync(a, da, sizeof(int) * tot, hipMemcpyDeviceToHost, ctx->stream));
       HIPC(hipMemcpyAsync(b, db, sizeof(int) * tot, hipMemcpyDeviceToHost, ctx->stream));

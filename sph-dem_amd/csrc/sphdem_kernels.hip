@@ -444,40 +444,41 @@ constexpr int SCAN_THREADS = 1024;
 constexpr int SCAN_ITEMS = 4;
 constexpr int SCAN_TILE = SCAN_THREADS * SCAN_ITEMS;
 
-// copyLast (optional): also receives out[n - 1]
-__global__ void __launch_bounds__(SCAN_THREADS) k_scan_tile(const int* __restrict__ in,
-                                                            int* __restrict__ out,
-                                                            int* __restrict__ tileSums, int n,
-                                                            int* copyLast) {
-  __shared__ int waveTot[SCAN_THREADS / 64];
+// Items from nin on count as 0.  copyLast (optional): also receives out[n - 1]
+template <class T>
+__global__ void __launch_bounds__(SCAN_THREADS) k_scan_tile(const int* __restrict__ in, int nin,
+                                                            T* __restrict__ out,
+                                                            T* __restrict__ tileSums, int n,
+                                                            T* copyLast) {
+  __shared__ T waveTot[SCAN_THREADS / 64];
   const int base = blockIdx.x * SCAN_TILE + threadIdx.x * SCAN_ITEMS;
-  int v[SCAN_ITEMS];
-  int run = 0;
+  T v[SCAN_ITEMS];
+  T run = 0;
   for (int k = 0; k < SCAN_ITEMS; k++) {
-    const int x = (base + k < n) ? in[base + k] : 0;
+    const T x = (base + k < nin) ? in[base + k] : 0;
     v[k] = run;
     run += x;
   }
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  int incl = run;
+  T incl = run;
   for (int d = 1; d < 64; d <<= 1) {
-    const int y = __shfl_up(incl, d, 64);
+    const T y = __shfl_up(incl, d, 64);
     if (lane >= d) incl += y;
   }
   if (lane == 63) waveTot[wave] = incl;
   __syncthreads();
   if (wave == 0) {
-    int w = (lane < SCAN_THREADS / 64) ? waveTot[lane] : 0;
-    int wi = w;
+    T w = (lane < SCAN_THREADS / 64) ? waveTot[lane] : 0;
+    T wi = w;
     for (int d = 1; d < 64; d <<= 1) {
-      const int y = __shfl_up(wi, d, 64);
+      const T y = __shfl_up(wi, d, 64);
       if (lane >= d) wi += y;
     }
     if (lane < SCAN_THREADS / 64) waveTot[lane] = wi - w;
     if (lane == SCAN_THREADS / 64 - 1 && tileSums) tileSums[blockIdx.x] = wi;
   }
   __syncthreads();
-  const int excl = waveTot[wave] + incl - run;
+  const T excl = waveTot[wave] + incl - run;
   for (int k = 0; k < SCAN_ITEMS; k++)
     if (base + k < n) {
       out[base + k] = excl + v[k];
@@ -487,13 +488,14 @@ __global__ void __launch_bounds__(SCAN_THREADS) k_scan_tile(const int* __restric
 // Second pass: block b adds the sum of tiles [0, b) to tile b.  The first
 // wavefront reduces those tile sums (each block redoes this small prefix,
 // which saves a launch for the scan of the tile sums).
-__global__ void __launch_bounds__(SCAN_THREADS) k_scan_add(int* __restrict__ out,
-                                                           const int* __restrict__ tileSums,
-                                                           int n, int* copyLast) {
-  __shared__ int pre;
+template <class T>
+__global__ void __launch_bounds__(SCAN_THREADS) k_scan_add(T* __restrict__ out,
+                                                           const T* __restrict__ tileSums,
+                                                           int n, T* copyLast) {
+  __shared__ T pre;
   const int b = blockIdx.x;
   if (threadIdx.x < 64) {
-    int acc = 0;
+    T acc = 0;
     for (int t = threadIdx.x; t < b; t += 64) acc += tileSums[t];
     for (int d = 32; d >= 1; d >>= 1) acc += __shfl_xor(acc, d, 64);
     if (threadIdx.x == 0) pre = acc;
@@ -504,7 +506,7 @@ __global__ void __launch_bounds__(SCAN_THREADS) k_scan_add(int* __restrict__ out
   for (int k = 0; k < SCAN_ITEMS; k++) {
     const int i = base + k * SCAN_THREADS;
     if (i < n) {
-      const int v = out[i] + pre;
+      const T v = out[i] + pre;
       out[i] = v;
       if (copyLast && i == n - 1) *copyLast = v;
     }
@@ -802,31 +804,51 @@ __global__ void k_hfromdens(Store S, int ns, double hfac) {
   S.posh[a].w = h;
 }
 
+// The cells [lo, hi] of dimension d within reach of t's, or (half > 0) those of
+// t - half to t + half.
+struct CellSpan {
+  int lo, hi;
+};
+__device__ __forceinline__ CellSpan cellSpan(double t, const Grid& g, int d, int reach,
+                                             double half) {
+  int lo, hi;
+  if (half > 0.0) {
+    lo = cellOf(t - half, g, d);
+    hi = cellOf(t + half, g, d);
+  } else {
+    const int c = cellOf(t, g, d);
+    lo = c - reach;
+    hi = c + reach;
+  }
+  return CellSpan{max(lo, 0), min(hi, g.dim[d] - 1)};
+}
 // The candidate ranges of forCells for a wave-uniform query point: visit(j0,
-// j1, sx, sy, sz) once per column range, in forCells' order.
+// j1, sx, sy, sz) once per column range, in forCells' order.  half > 0: only the
+// cells of the coordinates within half of the query's (cellOf is monotone: they
+// hold every particle that near).
 template <class V>
 __device__ __forceinline__ void forCellRanges(const Grid& g, const int* __restrict__ start,
                                               const Box& B, double qx, double qy, double qz,
-                                              int reach, V&& visit) {
+                                              int reach, V&& visit, double half = 0.0) {
   const int nsx = B.periodic[0] ? 3 : 1, nsy = B.periodic[1] ? 3 : 1, nsz = B.periodic[2] ? 3 : 1;
   const double q[3] = {qx, qy, qz};
   for (int ix = 0; ix < nsx; ix++) {
     const int sx = ix == 0 ? 0 : (ix == 1 ? -1 : 1);
     const double tx = sx == 0 ? q[0] : (sx == 1 ? q[0] - B.Lp[0] : q[0] - B.Lm[0]);
-    const int cx = cellOf(tx, g, 0);
-    const int x0 = max(cx - reach, 0), x1 = min(cx + reach, g.dim[0] - 1);
+    const CellSpan cx = cellSpan(tx, g, 0, reach, half);
+    const int x0 = cx.lo, x1 = cx.hi;
     if (x0 > x1) continue;
     for (int iy = 0; iy < nsy; iy++) {
       const int sy = iy == 0 ? 0 : (iy == 1 ? -1 : 1);
       const double ty = sy == 0 ? q[1] : (sy == 1 ? q[1] - B.Lp[1] : q[1] - B.Lm[1]);
-      const int cy = cellOf(ty, g, 1);
-      const int y0 = max(cy - reach, 0), y1 = min(cy + reach, g.dim[1] - 1);
+      const CellSpan cy = cellSpan(ty, g, 1, reach, half);
+      const int y0 = cy.lo, y1 = cy.hi;
       if (y0 > y1) continue;
       for (int iz = 0; iz < nsz; iz++) {
         const int sz = iz == 0 ? 0 : (iz == 1 ? -1 : 1);
         const double tz = sz == 0 ? q[2] : (sz == 1 ? q[2] - B.Lp[2] : q[2] - B.Lm[2]);
-        const int cz = cellOf(tz, g, 2);
-        const int z0 = max(cz - reach, 0), z1 = min(cz + reach, g.dim[2] - 1);
+        const CellSpan cz = cellSpan(tz, g, 2, reach, half);
+        const int z0 = cz.lo, z1 = cz.hi;
         if (z0 > z1) continue;
         for (int a = x0; a <= x1; a++)
           for (int b = y0; b <= y1; b++) {
@@ -1789,65 +1811,71 @@ __global__ void k_cell_coords(Store S, int n, Grid gs, CouplingRule R, int* __re
   }
 }
 
-// Pair enumeration of one search kind; mode 0 counts, mode 1 writes.
-__global__ void k_pairs(Store S, int ns, int nd, int kind, Grid gs, Grid gc,
-                        const int* __restrict__ start, Box B, CouplingRule R, int reachFull,
-                        int mode, int* __restrict__ cnt, const long long* __restrict__ off,
-                        int* __restrict__ oa, int* __restrict__ ob, int* __restrict__ oimg) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  int a;
-  if (kind == SPHDEM_PAIRS_SPH || kind == SPHDEM_PAIRS_SPH2DEM) {
-    if (i >= ns) return;
-    a = i;
-    if (!isSphT(S.iam[a])) return;
-  } else {
-    if (i >= nd) return;
-    a = ns + i;
+// Pair enumeration of one search kind; mode 0 counts, mode 1 writes from off on.
+// G lanes take a query together: G consecutive candidates of a column at a time,
+// the accepted ones written behind one another by their rank among the lanes
+// (ballot), so the order is that of one lane going through them all.
+//
+// What bounds it: the tests, at the share of lanes a column fills.  A thread per
+// query is a chain of dependent loads (8192 spheres are 128 wavefronts, on 1024
+// SIMDs) with scattered 4-byte stores.  On 65536 fluid and 24576 wall particles
+// with 8192 spheres, one count or write, a thread a query before and G lanes
+// now: DEM2SPH 437-449 and 43-46 us (G = 64: columns of 81 candidates), SPH2DEM
+// 464-495 and 135-145 us (G = 16: columns of about 25; the narrower range of
+// cells, 49 in place of 343, is part of it), DEM 89-93 and 23 us (G = 16).
+//
+// half (SPH2DEM): no sphere farther than this along an axis is accepted: an
+// accepted image lies within nc sphere cells of edge e, i.e. nc + 1 of them (and
+// one more where the cells around 0 truncate to one).
+template <int G>
+__global__ void __launch_bounds__(256) k_pairs(Store S, int ns, int nd, int kind, Grid gs, Grid gc,
+                                               const int* __restrict__ start, Box B,
+                                               CouplingRule R, double half, int mode,
+                                               int* __restrict__ cnt,
+                                               const long long* __restrict__ off,
+                                               int* __restrict__ oa, int* __restrict__ ob,
+                                               int* __restrict__ oimg) {
+  const int gl = threadIdx.x & (G - 1);
+  const int i = xcdBlock() * (256 / G) + threadIdx.x / G;
+  const bool fromSph = kind == SPHDEM_PAIRS_SPH2DEM;
+  if (i >= (fromSph ? ns : nd)) return;
+  const int a = fromSph ? i : ns + i;
+  if (fromSph && !isSphT(S.iam[a])) {
+    if (mode == 0 && gl == 0) cnt[i] = 0;
+    return;
   }
   const double4 pa = S.posh[a];
+  const int oaId = S.orig[a];
+  const int ca[3] = {demCell(R, pa.x, 0), demCell(R, pa.y, 1), demCell(R, pa.z, 2)};
   long long w = (mode == 1) ? off[i] : 0;
-  int c = 0;
-  auto emit = [&](int b, int sx, int sy, int sz) {
-    if (mode == 1) {
-      oa[w] = S.orig[a];
-      ob[w] = S.orig[b];
-      oimg[w] = (sx + 1) + 3 * (sy + 1) + 9 * (sz + 1);
-      w++;
-    }
-    c++;
+  auto accept = [&](int b, int sx, int sy, int sz) {
+    if (b == a && (sx | sy | sz) == 0) return false;
+    const double4 pb = S.posh[b];
+    if (fromSph && (sx | sy | sz) != 0 && !demImageExists(R, B, pb, sx, sy, sz)) return false;
+    const Img im = imagePos(pb, sx, sy, sz, B);
+    const double dx = pa.x - im.x, dy = pa.y - im.y, dz = pa.z - im.z;
+    const double l2 = dot3(dx, dy, dz, dx, dy, dz);
+    if (fromSph) return couplingAccept(R, ca, im.x, im.y, im.z, l2, true);
+    const double lim = 2.0 * dmax2(pa.w, pb.w);
+    return l2 <= lim * lim;
   };
-  if (kind == SPHDEM_PAIRS_SPH || kind == SPHDEM_PAIRS_DEM2SPH) {
-    forCells(gs, start, B, pa.x, pa.y, pa.z, 1, [&](int b, int sx, int sy, int sz) {
-      if (b == a && (sx | sy | sz) == 0) return;
-      const double4 pb = S.posh[b];
-      const Img im = imagePos(pb, sx, sy, sz, B);
-      const double dx = pa.x - im.x, dy = pa.y - im.y, dz = pa.z - im.z;
-      const double l2 = dot3(dx, dy, dz, dx, dy, dz);
-      const double lim = 2.0 * dmax2(pa.w, pb.w);
-      if (l2 <= lim * lim) emit(b, sx, sy, sz);
-    });
-  } else if (kind == SPHDEM_PAIRS_DEM) {
-    forCells(gc, start, B, pa.x, pa.y, pa.z, 1, [&](int b, int sx, int sy, int sz) {
-      if (b == a && (sx | sy | sz) == 0) return;
-      const double4 pb = S.posh[b];
-      const Img im = imagePos(pb, sx, sy, sz, B);
-      const double dx = pa.x - im.x, dy = pa.y - im.y, dz = pa.z - im.z;
-      const double l2 = dot3(dx, dy, dz, dx, dy, dz);
-      const double lim = 2.0 * dmax2(pa.w, pb.w);
-      if (l2 <= lim * lim) emit(b, sx, sy, sz);
-    });
-  } else {
-    const int ca[3] = {demCell(R, pa.x, 0), demCell(R, pa.y, 1), demCell(R, pa.z, 2)};
-    forCells(gc, start, B, pa.x, pa.y, pa.z, reachFull, [&](int j, int sx, int sy, int sz) {
-      const double4 pj = S.posh[j];
-      if ((sx | sy | sz) != 0 && !demImageExists(R, B, pj, sx, sy, sz)) return;
-      const Img im = imagePos(pj, sx, sy, sz, B);
-      const double dx = pa.x - im.x, dy = pa.y - im.y, dz = pa.z - im.z;
-      const double l2 = dot3(dx, dy, dz, dx, dy, dz);
-      if (couplingAccept(R, ca, im.x, im.y, im.z, l2, true)) emit(j, sx, sy, sz);
-    });
-  }
-  if (mode == 0) cnt[i] = c;
+  forCellRanges(kind == SPHDEM_PAIRS_DEM2SPH ? gs : gc, start, B, pa.x, pa.y, pa.z, 1,
+                [&](int j0, int j1, int sx, int sy, int sz) {
+    for (int jj = j0; jj < j1; jj += G) {
+      const int b = jj + gl;
+      const bool ok = b < j1 && accept(b, sx, sy, sz);
+      unsigned long long m = __ballot(ok);
+      if (G < 64) m = (m >> (threadIdx.x & 63 & ~(G - 1))) & ((1ull << (G & 63)) - 1);
+      if (mode == 1 && ok) {
+        const long long at = w + __popcll(m & ((1ull << gl) - 1));
+        oa[at] = oaId;
+        ob[at] = S.orig[b];
+        oimg[at] = imageCode(sx, sy, sz);
+      }
+      w += __popcll(m);
+    }
+  }, fromSph ? half : 0.0);
+  if (mode == 0 && gl == 0) cnt[i] = (int)w;
 }
 
 }  // namespace sphdem

@@ -851,21 +851,26 @@ __global__ void k_list_pos(const double4* __restrict__ posh, const double* __res
 
 // The cached lists as (a, b, image) triples of original indices, for the
 // parity enumeration of the SPH pair set: a ghost neighbour reports its
-// origin and its image code.
-__global__ void k_list_pairs(Store S, int ns, int n, const int* __restrict__ nbl,
-                             const int* __restrict__ nbcnt, const int* __restrict__ gcode,
-                             const long long* __restrict__ off, int* __restrict__ oa,
-                             int* __restrict__ ob, int* __restrict__ oimg) {
-  const int a = blockIdx.x * blockDim.x + threadIdx.x;
+// origin and its image code.  A wavefront per target, a lane per entry: the
+// triples leave in whole lines (a thread a target stores 4 bytes a line apart:
+// 359 us for 90112 targets of 110 entries; so 38, 120 MB written).
+__global__ void __launch_bounds__(256) k_list_pairs(Store S, int ns, int n,
+                                                    const int* __restrict__ nbl,
+                                                    const int* __restrict__ nbcnt,
+                                                    const int* __restrict__ gcode,
+                                                    const long long* __restrict__ off,
+                                                    int* __restrict__ oa, int* __restrict__ ob,
+                                                    int* __restrict__ oimg) {
+  const int a = xcdBlock() * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
   if (a >= ns) return;
   const int cnt = nbcnt[a];
   const int ia = S.orig[a];
-  long long w = off[a];
-  for (int k = 0; k < cnt; k++, w++) {
+  const long long w = off[a];
+  for (int k = lane; k < cnt; k += 64) {
     const int e = nbl[nbEntry(k, a, ns)];
-    oa[w] = ia;
-    ob[w] = S.orig[e];
-    oimg[w] = e >= n ? gcode[e - n] : 13;
+    oa[w + k] = ia;
+    ob[w + k] = S.orig[e];
+    oimg[w + k] = e >= n ? gcode[e - n] : 13;
   }
 }
 
