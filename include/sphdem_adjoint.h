@@ -28,11 +28,11 @@
  *   - Pairs are (a, b, image) triples of sphdem_get_pairs: b's periodic image
  *     sits at r_b + ((img%3)-1, (img/3)%3-1, img/9-1) * shift_len.  The
  *     per-query passes take them grouped by a: query[i] = a, its partners
- *     b[off[i] .. off[i+1]) with their images; one thread per query keeps a's
+ *     b[off[i] .. off[i+1]) with their images; the lanes that take a query keep a's
  *     sums in registers.
  *   - Forward outputs and backward adjoints are ADDED to the arrays given (the
  *     caller zeroes them).  The backward kernels of force, omega and dddt
- *     gather: the thread of a particle also adds the terms of the pairs in
+ *     gather: the lanes of a particle also add the terms of the pairs in
  *     which it is the partner, which requires a symmetric pair set (every
  *     (a, b, img) has its (b, a, 26 - img)); the SPH set of sphdem_get_pairs
  *     is symmetric (the criterion uses max(h_a, h_b)).  The coupling, fpi

@@ -33,15 +33,39 @@ namespace sphdem_adj {
 constexpr int kTPB = 256;
 constexpr int SPH_T = 0;
 
-// Thread index with the grid's blocks dealt to the 8 XCDs in contiguous
-// ranges (the hardware deals consecutive blocks round-robin): consecutive
-// queries are neighbours in space, so each XCD's L2 then holds the partner
-// data of its own range instead of every XCD fetching all of it.  A bijection
-// on the grid.
-__device__ __forceinline__ int xcdIndex() {
+// Lanes that take a query together: SPH lists (about 110 entries), a fluid
+// particle's spheres (0 to some 30), a sphere's fluid particles (about 110; few
+// queries).  With a thread a query, 90112 queries are 1.4 wavefronts a SIMD
+// (8192 spheres 0.1), each a chain of 110 rounds of gathers, and the lists are
+// read a line a lane; with a group the rounds are few, the lists are read in
+// whole lines and enough wavefronts wait side by side: bound by the FP64
+// arithmetic (forces) or the gathers.  Before -> now at 90112 queries of 110
+// entries, 8192 spheres, us: force 294 -> 81, its backward 492 -> 197; omega
+// 202 -> 48 and 484 -> 96 (one walk in place of two); dddt 227 -> 50 and
+// 355 -> 125; drag on spheres 233 -> 24 and 1075 -> 181 (383 before waveAdd3);
+// coupling backward 382 + 223 -> 38 + 128.
+constexpr int kSphLanes = 16, kCplLanes = 8, kFpiLanes = 64;
+
+// Query of G consecutive lanes, with the grid's blocks dealt to the 8 XCDs in
+// contiguous ranges (the hardware deals consecutive blocks round-robin):
+// consecutive queries are neighbours in space, so each XCD's L2 then holds the
+// partner data of its own range instead of every XCD fetching all of it.  A
+// bijection on the grid.
+template <int G>
+__device__ __forceinline__ int queryIndex() {
   const int nb = gridDim.x, x = blockIdx.x & 7, r = blockIdx.x >> 3;
   const int q = nb >> 3, rem = nb & 7;
-  return (x * q + min(x, rem) + r) * blockDim.x + threadIdx.x;
+  return (x * q + min(x, rem) + r) * (kTPB / G) + (int)threadIdx.x / G;
+}
+template <int G>
+__device__ __forceinline__ int queryLane() {
+  return threadIdx.x & (G - 1);
+}
+// Sums each value over a query's lanes, in a fixed order; every lane gets it.
+template <int G, class... T>
+__device__ __forceinline__ void sumLanes(T&... v) {
+#pragma unroll
+  for (int o = G / 2; o > 0; o >>= 1) ((v += __shfl_xor(v, o, 64)), ...);
 }
 
 __device__ __forceinline__ double3 ld3(const double* p, int i) {
@@ -53,6 +77,32 @@ __device__ __forceinline__ void add3(double* p, int i, double x, double y, doubl
   unsafeAtomicAdd(p + 3 * i + 2, z);
 }
 __device__ __forceinline__ void add1(double* p, int i, double x) { unsafeAtomicAdd(p + i, x); }
+
+// add3 of every lane of a wavefront (idx < 0: none), the 192 additions taken in
+// the order of their addresses: three neighbouring lanes add to one particle's
+// x, y and z, so they reach the L2, whose atomics bound these kernels, as one
+// request instead of three.  Every lane must call it.
+struct Add3Stage {
+  double v[192];
+  int idx[64];
+};
+__device__ __forceinline__ void waveAdd3(Add3Stage& L, double* p, int idx, double x, double y,
+                                         double z) {
+  const int lane = threadIdx.x & 63;
+  __builtin_amdgcn_wave_barrier();
+  L.v[3 * lane] = x;
+  L.v[3 * lane + 1] = y;
+  L.v[3 * lane + 2] = z;
+  L.idx[lane] = idx;
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+  for (int k = 0; k < 3; k++) {
+    const int s = 64 * k + lane, m = s / 3, i = L.idx[m];
+    if (i >= 0) unsafeAtomicAdd(p + 3 * i + (s - 3 * m), L.v[s]);
+  }
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+}
 
 // b's periodic image: r_b + shift
 __device__ __forceinline__ double3 imageOf(const double* r, int b, int img, const double* L) {
@@ -115,20 +165,20 @@ __device__ void blockAdd(double (&v)[NV], double* dst) {
 //     visc = 2 nu rho0 / (rho_a rho_b),  d = r^2 (Fa + Fb) ia / 2,
 //     den = r^2 + 0.01 hav^2,  hav = (h_a + h_b)/2
 //   pressure:         B  = -m_b (pdr2_a Fa + pdr2_b Fb) ia,  fp_a += B dx
-// One thread per query particle: its sums stay in registers.
+// A query's lanes keep partial sums in registers and add them at the end.
 __global__ void __launch_bounds__(kTPB) k_force_fwd(int32_t nq, const int32_t* __restrict__ query,
                             const int64_t* __restrict__ off, const int32_t* __restrict__ pb,
                             const int32_t* __restrict__ pimg, sphdem_adj_fields in,
                             sphdem_adj_consts C, double* __restrict__ fv,
                             double* __restrict__ fp) {
-  const int i = xcdIndex();
+  const int i = queryIndex<kSphLanes>(), gl = queryLane<kSphLanes>();
   if (i >= nq) return;
   const int a = query[i];
   const double3 ra = ld3(in.r, a), va = ld3(in.vhat, a);
   const double ha = in.h[a], ia = 1.0 / in.omega[a], rhoa = in.dens[a], pda = in.pdr2[a];
   const bool sphA = in.iam[a] == SPH_T;
   double vx = 0.0, vy = 0.0, vz = 0.0, px = 0.0, py = 0.0, pz = 0.0;
-  for (int64_t j = off[i]; j < off[i + 1]; j++) {
+  for (int64_t j = off[i] + gl; j < off[i + 1]; j += kSphLanes) {
     const int b = pb[j];
     const double3 rb = imageOf(in.r, b, pimg[j], C.shift_len);
     const double dx = ra.x - rb.x, dy = ra.y - rb.y, dz = ra.z - rb.z;
@@ -154,6 +204,8 @@ __global__ void __launch_bounds__(kTPB) k_force_fwd(int32_t nq, const int32_t* _
     py += B * dy;
     pz += B * dz;
   }
+  sumLanes<kSphLanes>(vx, vy, vz, px, py, pz);
+  if (gl != 0) return;
   fv[3 * a] += vx;
   fv[3 * a + 1] += vy;
   fv[3 * a + 2] += vz;
@@ -162,18 +214,18 @@ __global__ void __launch_bounds__(kTPB) k_force_fwd(int32_t nq, const int32_t* _
   fp[3 * a + 2] += pz;
 }
 
-// Backward over the symmetric SPH lists, gathered: the thread of a adds the
+// Backward over the symmetric SPH lists, gathered: the lanes of a add the
 // adjoints of a's inputs from its own force terms (a the query) and from the
 // terms of its partners' forces in which a is the partner (b the query: the
 // same r, dx and dv with their signs flipped, F taken on both h, divided by
-// omega_b), so every adjoint is written by one thread, without atomics.  The
+// omega_b), so every adjoint is written by one lane, without atomics.  The
 // viscosity adjoint is summed over the own terms only (each pair once).
 __global__ void __launch_bounds__(kTPB) k_force_bwd(int32_t nq, const int32_t* __restrict__ query,
                             const int64_t* __restrict__ off, const int32_t* __restrict__ pb,
                             const int32_t* __restrict__ pimg, sphdem_adj_fields in,
                             sphdem_adj_consts C, const double* __restrict__ gfv,
                             const double* __restrict__ gfp, sphdem_adj_grads g) {
-  const int i = xcdIndex();
+  const int i = queryIndex<kSphLanes>(), gl = queryLane<kSphLanes>();
   double gnu[1] = {0.0};
   if (i < nq) {
     const int a = query[i];
@@ -184,7 +236,7 @@ __global__ void __launch_bounds__(kTPB) k_force_bwd(int32_t nq, const int32_t* _
     const double3 gv = ld3(gfv, a), gp = ld3(gfp, a);
     double grx = 0.0, gry = 0.0, grz = 0.0, gvx = 0.0, gvy = 0.0, gvz = 0.0;
     double gha = 0.0, gda = 0.0, gia = 0.0, gpa = 0.0;
-    for (int64_t j = off[i]; j < off[i + 1]; j++) {
+    for (int64_t j = off[i] + gl; j < off[i + 1]; j += kSphLanes) {
       const int b = pb[j];
       const double3 rb = imageOf(in.r, b, pimg[j], C.shift_len);
       const double dx = ra.x - rb.x, dy = ra.y - rb.y, dz = ra.z - rb.z;
@@ -274,16 +326,19 @@ __global__ void __launch_bounds__(kTPB) k_force_bwd(int32_t nq, const int32_t* _
       gry += dgy + sc * dy;
       grz += dgz + sc * dz;
     }
-    g.r[3 * a] += grx;
-    g.r[3 * a + 1] += gry;
-    g.r[3 * a + 2] += grz;
-    g.vhat[3 * a] += gvx;
-    g.vhat[3 * a + 1] += gvy;
-    g.vhat[3 * a + 2] += gvz;
-    g.h[a] += gha;
-    g.dens[a] += gda;
-    g.omega[a] += -gia * ia * ia;  // ia = 1/omega_a
-    g.pdr2[a] += gpa;
+    sumLanes<kSphLanes>(grx, gry, grz, gvx, gvy, gvz, gha, gda, gia, gpa);
+    if (gl == 0) {
+      g.r[3 * a] += grx;
+      g.r[3 * a + 1] += gry;
+      g.r[3 * a + 2] += grz;
+      g.vhat[3 * a] += gvx;
+      g.vhat[3 * a + 1] += gvy;
+      g.vhat[3 * a + 2] += gvz;
+      g.h[a] += gha;
+      g.dens[a] += gda;
+      g.omega[a] += -gia * ia * ia;  // ia = 1/omega_a
+      g.pdr2[a] += gpa;
+    }
   }
   blockAdd<1>(gnu, g.params);
 }
@@ -313,28 +368,29 @@ __global__ void __launch_bounds__(kTPB) k_omega_fwd(int32_t nq, const int32_t* _
                             const int64_t* __restrict__ off, const int32_t* __restrict__ pb,
                             const int32_t* __restrict__ pimg, sphdem_adj_fields in,
                             sphdem_adj_consts C, double* __restrict__ omega) {
-  const int i = xcdIndex();
+  const int i = queryIndex<kSphLanes>(), gl = queryLane<kSphLanes>();
   if (i >= nq) return;
   const int a = query[i];
   const double3 ra = ld3(in.r, a);
   const double ha = in.h[a];
   double P, t0, t1;
   wendP(C.wcon, 0.0, ha, P, t0, t1);
-  double S = in.mass[a] * P;
-  for (int64_t j = off[i]; j < off[i + 1]; j++) {
+  double S = gl == 0 ? in.mass[a] * P : 0.0;
+  for (int64_t j = off[i] + gl; j < off[i + 1]; j += kSphLanes) {
     const int b = pb[j];
     const double3 rb = imageOf(in.r, b, pimg[j], C.shift_len);
     const double dx = ra.x - rb.x, dy = ra.y - rb.y, dz = ra.z - rb.z;
     wendP(C.wcon, sqrt(dx * dx + dy * dy + dz * dz), ha, P, t0, t1);
     S += in.mass[b] * P;
   }
-  omega[a] += ha * S / (in.dens[a] * 3.0);
+  sumLanes<kSphLanes>(S);
+  if (gl == 0) omega[a] += ha * S / (in.dens[a] * 3.0);
 }
 
 // Backward of omega over the symmetric SPH lists (b in the list of a iff a is
-// in the list of b, with the opposite image): the thread of a adds the terms
+// in the list of b, with the opposite image): the lanes of a add the terms
 // of its own sum and, from the same entries, those of its partners' sums in
-// which a appears, so every adjoint is written by one thread, without atomics.
+// which a appears, so every adjoint is written by one lane, without atomics.
 //   own:     Sbar_a = go_a h_a / (3 rho_a),  r_a += Sbar_a m_b dP(r, h_a)/dr dx/r
 //   partner: r_a   += Sbar_b m_a dP(r, h_b)/dr dx/r     (dx = r_a - r_b')
 __global__ void __launch_bounds__(kTPB) k_omega_bwd(int32_t nq, const int32_t* __restrict__ query,
@@ -342,7 +398,7 @@ __global__ void __launch_bounds__(kTPB) k_omega_bwd(int32_t nq, const int32_t* _
                             const int32_t* __restrict__ pimg, sphdem_adj_fields in,
                             sphdem_adj_consts C, const double* __restrict__ gomega,
                             sphdem_adj_grads g) {
-  const int i = xcdIndex();
+  const int i = queryIndex<kSphLanes>(), gl = queryLane<kSphLanes>();
   if (i >= nq) return;
   const int a = query[i];
   const double go = gomega[a];
@@ -350,29 +406,19 @@ __global__ void __launch_bounds__(kTPB) k_omega_bwd(int32_t nq, const int32_t* _
   const double ha = in.h[a], rhoa = in.dens[a], ma = in.mass[a];
   double P0, dP0r, dP0h, P, dPr, dPh;
   wendP(C.wcon, 0.0, ha, P0, dP0r, dP0h);
-  double S = ma * P0;
-  if (go != 0.0) {
-    for (int64_t j = off[i]; j < off[i + 1]; j++) {
-      const int b = pb[j];
-      const double3 rb = imageOf(in.r, b, pimg[j], C.shift_len);
-      const double dx = ra.x - rb.x, dy = ra.y - rb.y, dz = ra.z - rb.z;
-      wendP(C.wcon, sqrt(dx * dx + dy * dy + dz * dz), ha, P, dPr, dPh);
-      S += in.mass[b] * P;
-    }
-  }
   const double Sbar = go * ha / (3.0 * rhoa);
-  double gha = go * S / (3.0 * rhoa) + Sbar * ma * dP0h;
-  const double gda = -go * ha * S / (3.0 * rhoa * rhoa);
-  double grx = 0.0, gry = 0.0, grz = 0.0;
-  for (int64_t j = off[i]; j < off[i + 1]; j++) {
+  double S = 0.0, gha = 0.0, grx = 0.0, gry = 0.0, grz = 0.0;
+  for (int64_t j = off[i] + gl; j < off[i + 1]; j += kSphLanes) {
     const int b = pb[j];
     const double3 rb = imageOf(in.r, b, pimg[j], C.shift_len);
     const double dx = ra.x - rb.x, dy = ra.y - rb.y, dz = ra.z - rb.z;
     const double r = sqrt(dx * dx + dy * dy + dz * dz);
     double k = 0.0;
-    if (Sbar != 0.0) {  // a's own sum
+    if (go != 0.0) {  // a's own sum
+      const double mb = in.mass[b];
       wendP(C.wcon, r, ha, P, dPr, dPh);
-      const double c = Sbar * in.mass[b];
+      S += mb * P;
+      const double c = Sbar * mb;
       gha += c * dPh;
       k += c * dPr;
     }
@@ -390,11 +436,14 @@ __global__ void __launch_bounds__(kTPB) k_omega_bwd(int32_t nq, const int32_t* _
       grz += kr * dz;
     }
   }
+  sumLanes<kSphLanes>(S, gha, grx, gry, grz);
+  if (gl != 0) return;
+  S += ma * P0;
   g.r[3 * a] += grx;
   g.r[3 * a + 1] += gry;
   g.r[3 * a + 2] += grz;
-  g.h[a] += gha;
-  g.dens[a] += gda;
+  g.h[a] += gha + go * S / (3.0 * rhoa) + Sbar * ma * dP0h;
+  g.dens[a] += -go * ha * S / (3.0 * rhoa * rhoa);
 }
 
 // ---------------------------------------------------------------- dddt
@@ -404,13 +453,13 @@ __global__ void __launch_bounds__(kTPB) k_dddt_fwd(int32_t nq, const int32_t* __
                            const int64_t* __restrict__ off, const int32_t* __restrict__ pb,
                            const int32_t* __restrict__ pimg, sphdem_adj_fields in,
                            sphdem_adj_consts C, double* __restrict__ dddt) {
-  const int i = xcdIndex();
+  const int i = queryIndex<kSphLanes>(), gl = queryLane<kSphLanes>();
   if (i >= nq) return;
   const int a = query[i];
   const double3 ra = ld3(in.r, a), va = ld3(in.vhat, a);
   const double ha = in.h[a], ia = 1.0 / in.omega[a];
   double sum = 0.0;
-  for (int64_t j = off[i]; j < off[i + 1]; j++) {
+  for (int64_t j = off[i] + gl; j < off[i + 1]; j += kSphLanes) {
     const int b = pb[j];
     const double3 rb = imageOf(in.r, b, pimg[j], C.shift_len);
     const double dx = ra.x - rb.x, dy = ra.y - rb.y, dz = ra.z - rb.z;
@@ -421,11 +470,13 @@ __global__ void __launch_bounds__(kTPB) k_dddt_fwd(int32_t nq, const int32_t* __
     const double u = (va.x - vb.x) * dx + (va.y - vb.y) * dy + (va.z - vb.z) * dz;
     sum += in.mass[b] * u * F * ia;
   }
+  sumLanes<kSphLanes>(sum);
+  if (gl != 0) return;
   dddt[a] += sum;
 }
 
 // Backward of dddt over the symmetric SPH lists, gathered as for omega: the
-// thread of a adds the terms of dddt_a and of every dddt_b in which a is the
+// lanes of a add the terms of dddt_a and of every dddt_b in which a is the
 // partner (u = dv.dx and dx change sign between the two, F is taken on the
 // query's h, divided by the query's omega).
 __global__ void __launch_bounds__(kTPB) k_dddt_bwd(int32_t nq, const int32_t* __restrict__ query,
@@ -433,14 +484,14 @@ __global__ void __launch_bounds__(kTPB) k_dddt_bwd(int32_t nq, const int32_t* __
                            const int32_t* __restrict__ pimg, sphdem_adj_fields in,
                            sphdem_adj_consts C, const double* __restrict__ gdddt,
                            sphdem_adj_grads g) {
-  const int i = xcdIndex();
+  const int i = queryIndex<kSphLanes>(), gl = queryLane<kSphLanes>();
   if (i >= nq) return;
   const int a = query[i];
   const double gd = gdddt[a];
   const double3 ra = ld3(in.r, a), va = ld3(in.vhat, a);
   const double ha = in.h[a], ia = 1.0 / in.omega[a], ma = in.mass[a];
   double grx = 0.0, gry = 0.0, grz = 0.0, gvx = 0.0, gvy = 0.0, gvz = 0.0, gha = 0.0, gia = 0.0;
-  for (int64_t j = off[i]; j < off[i + 1]; j++) {
+  for (int64_t j = off[i] + gl; j < off[i + 1]; j += kSphLanes) {
     const int b = pb[j];
     const double gdb = gdddt[b];
     if (gd == 0.0 && gdb == 0.0) continue;
@@ -477,6 +528,8 @@ __global__ void __launch_bounds__(kTPB) k_dddt_bwd(int32_t nq, const int32_t* __
     gry += ubar * dvy + kr * dy;
     grz += ubar * dvz + kr * dz;
   }
+  sumLanes<kSphLanes>(grx, gry, grz, gvx, gvy, gvz, gha, gia);
+  if (gl != 0) return;
   g.r[3 * a] += grx;
   g.r[3 * a + 1] += gry;
   g.r[3 * a + 2] += grz;
@@ -501,13 +554,13 @@ __global__ void __launch_bounds__(kTPB) k_cpl_fwd1(int32_t nq, const int32_t* __
                            const int32_t* __restrict__ pimg, sphdem_adj_fields in,
                            sphdem_adj_consts C, double* __restrict__ por_sum,
                            double* __restrict__ shep) {
-  const int i = xcdIndex();
+  const int i = queryIndex<kCplLanes>(), gl = queryLane<kCplLanes>();
   if (i >= nq) return;
   const int a = query[i];
   const double3 ra = ld3(in.r, a);
   const double va = in.mass[a] / in.dens[a], hc = 0.5 * C.coupling_radius;
   double por = 0.0;
-  for (int64_t j = off[i]; j < off[i + 1]; j++) {
+  for (int64_t j = off[i] + gl; j < off[i + 1]; j += kCplLanes) {
     const int d = pd[j];
     const double3 rd = imageOf(in.r, d, pimg[j], C.shift_len);
     const double dx = ra.x - rd.x, dy = ra.y - rd.y, dz = ra.z - rd.z;
@@ -516,6 +569,8 @@ __global__ void __launch_bounds__(kTPB) k_cpl_fwd1(int32_t nq, const int32_t* __
     por += C.porosity_incr * W;
     if (W != 0.0) add1(shep, d, va * W);
   }
+  sumLanes<kCplLanes>(por);
+  if (gl != 0) return;
   por_sum[a] += por;
 }
 
@@ -523,13 +578,13 @@ __global__ void __launch_bounds__(kTPB) k_cpl_fwd2(int32_t nq, const int32_t* __
                            const int64_t* __restrict__ off, const int32_t* __restrict__ pd,
                            const int32_t* __restrict__ pimg, sphdem_adj_fields in,
                            sphdem_adj_consts C, double* __restrict__ drag) {
-  const int i = xcdIndex();
+  const int i = queryIndex<kCplLanes>(), gl = queryLane<kCplLanes>();
   if (i >= nq) return;
   const int a = query[i];
   const double3 ra = ld3(in.r, a);
   const double rhoa = in.dens[a], hc = 0.5 * C.coupling_radius;
   double x = 0.0, y = 0.0, z = 0.0;
-  for (int64_t j = off[i]; j < off[i + 1]; j++) {
+  for (int64_t j = off[i] + gl; j < off[i + 1]; j += kCplLanes) {
     const int d = pd[j];
     const double sd = in.shep[d];
     if (!(sd > 0.0)) continue;
@@ -543,88 +598,102 @@ __global__ void __launch_bounds__(kTPB) k_cpl_fwd2(int32_t nq, const int32_t* __
     y -= c * fd.y;
     z -= c * fd.z;
   }
+  sumLanes<kCplLanes>(x, y, z);
+  if (gl != 0) return;
   drag[3 * a] += x;
   drag[3 * a + 1] += y;
   drag[3 * a + 2] += z;
 }
 
-// first backward launch: the drag and porosity terms; shepbar[d] collects the
-// adjoint of the Shepard sums
+// first backward launch: shepbar[d] collects the adjoint of the Shepard sums
 __global__ void __launch_bounds__(kTPB) k_cpl_bwd1(int32_t nq, const int32_t* __restrict__ query,
                            const int64_t* __restrict__ off, const int32_t* __restrict__ pd,
                            const int32_t* __restrict__ pimg, sphdem_adj_fields in,
-                           sphdem_adj_consts C, const double* __restrict__ gpor,
-                           const double* __restrict__ gdrag, double* __restrict__ shepbar,
-                           sphdem_adj_grads g) {
-  const int i = xcdIndex();
+                           sphdem_adj_consts C, const double* __restrict__ gdrag,
+                           double* __restrict__ shepbar) {
+  const int i = queryIndex<kCplLanes>(), gl = queryLane<kCplLanes>();
   if (i >= nq) return;
   const int a = query[i];
   const double3 ra = ld3(in.r, a), gdr = ld3(gdrag, a);
-  const double gp = gpor[a];
   const double rhoa = in.dens[a], hc = 0.5 * C.coupling_radius;
-  double grx = 0.0, gry = 0.0, grz = 0.0, gda = 0.0;
-  for (int64_t j = off[i]; j < off[i + 1]; j++) {
+  for (int64_t j = off[i] + gl; j < off[i + 1]; j += kCplLanes) {
     const int d = pd[j];
+    const double sd = in.shep[d];
+    if (!(sd > 0.0)) continue;
     const double3 rd = imageOf(in.r, d, pimg[j], C.shift_len);
     const double dx = ra.x - rd.x, dy = ra.y - rd.y, dz = ra.z - rd.z;
-    const double r = sqrt(dx * dx + dy * dy + dz * dz);
-    double W, dWr, t1;
-    wendW(C.wcon, r, hc, W, dWr, t1);
-    double Wbar = gp * C.porosity_incr;
-    const double sd = in.shep[d];
-    if (sd > 0.0) {
-      const double md = in.mass[d];
-      const double c = md * W / (rhoa * sd);
-      const double3 fd = ld3(in.fdrag, d);
-      const double cbar = -(gdr.x * fd.x + gdr.y * fd.y + gdr.z * fd.z);
-      add3(g.fdrag, d, -c * gdr.x, -c * gdr.y, -c * gdr.z);
-      if (cbar != 0.0) add1(shepbar, d, -cbar * c / sd);
-      gda += -cbar * c / rhoa;
-      Wbar += cbar * md / (rhoa * sd);
-    }
-    if (r > 0.0 && Wbar != 0.0) {
-      const double k = Wbar * dWr / r;
-      grx += k * dx;
-      gry += k * dy;
-      grz += k * dz;
-      add3(g.r, d, -k * dx, -k * dy, -k * dz);
-    }
+    double W, t0, t1;
+    wendW(C.wcon, sqrt(dx * dx + dy * dy + dz * dz), hc, W, t0, t1);
+    const double c = in.mass[d] * W / (rhoa * sd);
+    const double3 fd = ld3(in.fdrag, d);
+    const double sb = (gdr.x * fd.x + gdr.y * fd.y + gdr.z * fd.z) * c / sd;
+    if (sb != 0.0) add1(shepbar, d, sb);
   }
-  add3(g.r, a, grx, gry, grz);
-  add1(g.dens, a, gda);
 }
 
-// second backward launch: the Shepard sums
+// second backward launch: the drag, porosity and Shepard terms.  A wavefront's
+// queries take their steps together: the additions to the spheres go through
+// waveAdd3.
 __global__ void __launch_bounds__(kTPB) k_cpl_bwd2(int32_t nq, const int32_t* __restrict__ query,
                            const int64_t* __restrict__ off, const int32_t* __restrict__ pd,
                            const int32_t* __restrict__ pimg, sphdem_adj_fields in,
-                           sphdem_adj_consts C, const double* __restrict__ shepbar,
+                           sphdem_adj_consts C, const double* __restrict__ gpor,
+                           const double* __restrict__ gdrag, const double* __restrict__ shepbar,
                            sphdem_adj_grads g) {
-  const int i = xcdIndex();
-  if (i >= nq) return;
-  const int a = query[i];
-  const double3 ra = ld3(in.r, a);
+  __shared__ Add3Stage stage[kTPB / 64];
+  Add3Stage& L = stage[threadIdx.x >> 6];
+  const int i = queryIndex<kCplLanes>(), gl = queryLane<kCplLanes>();
+  const int a = i < nq ? query[i] : 0;
+  int64_t j = i < nq ? off[i] + gl : 0;
+  const int64_t end = i < nq ? off[i + 1] : 0;
+  const double3 ra = ld3(in.r, a), gdr = ld3(gdrag, a);
+  const double gp = gpor[a];
   const double rhoa = in.dens[a], va = in.mass[a] / rhoa, hc = 0.5 * C.coupling_radius;
   double grx = 0.0, gry = 0.0, grz = 0.0, gda = 0.0;
-  for (int64_t j = off[i]; j < off[i + 1]; j++) {
-    const int d = pd[j];
-    const double sb = shepbar[d];
-    if (sb == 0.0) continue;
-    const double3 rd = imageOf(in.r, d, pimg[j], C.shift_len);
-    const double dx = ra.x - rd.x, dy = ra.y - rd.y, dz = ra.z - rd.z;
-    const double r = sqrt(dx * dx + dy * dy + dz * dz);
-    double W, dWr, t1;
-    wendW(C.wcon, r, hc, W, dWr, t1);
-    // shep_d += (m_a / rho_a) W
-    gda += -sb * va * W / rhoa;
-    if (r > 0.0) {
-      const double k = sb * va * dWr / r;
-      grx += k * dx;
-      gry += k * dy;
-      grz += k * dz;
-      add3(g.r, d, -k * dx, -k * dy, -k * dz);
+  for (; __any(j < end); j += kCplLanes) {
+    int d = -1;
+    double fx = 0.0, fy = 0.0, fz = 0.0, kx = 0.0, ky = 0.0, kz = 0.0;
+    if (j < end) {
+      d = pd[j];
+      const double3 rd = imageOf(in.r, d, pimg[j], C.shift_len);
+      const double dx = ra.x - rd.x, dy = ra.y - rd.y, dz = ra.z - rd.z;
+      const double r = sqrt(dx * dx + dy * dy + dz * dz);
+      double W, dWr, t1;
+      wendW(C.wcon, r, hc, W, dWr, t1);
+      double Wbar = gp * C.porosity_incr;
+      const double sd = in.shep[d];
+      if (sd > 0.0) {
+        const double md = in.mass[d];
+        const double c = md * W / (rhoa * sd);
+        const double3 fd = ld3(in.fdrag, d);
+        const double cbar = -(gdr.x * fd.x + gdr.y * fd.y + gdr.z * fd.z);
+        fx = -c * gdr.x;
+        fy = -c * gdr.y;
+        fz = -c * gdr.z;
+        gda += -cbar * c / rhoa;
+        Wbar += cbar * md / (rhoa * sd);
+      }
+      // shep_d += (m_a / rho_a) W
+      const double sb = shepbar[d];
+      if (sb != 0.0) {
+        gda += -sb * va * W / rhoa;
+        Wbar += sb * va;
+      }
+      if (r > 0.0 && Wbar != 0.0) {
+        const double k = Wbar * dWr / r;
+        kx = k * dx;
+        ky = k * dy;
+        kz = k * dz;
+        grx += kx;
+        gry += ky;
+        grz += kz;
+      }
     }
+    waveAdd3(L, g.fdrag, fx == 0.0 && fy == 0.0 && fz == 0.0 ? -1 : d, fx, fy, fz);
+    waveAdd3(L, g.r, kx == 0.0 && ky == 0.0 && kz == 0.0 ? -1 : d, -kx, -ky, -kz);
   }
+  sumLanes<kCplLanes>(grx, gry, grz, gda);
+  if (i >= nq || gl != 0) return;
   add3(g.r, a, grx, gry, grz);
   add1(g.dens, a, gda);
 }
@@ -651,7 +720,7 @@ __device__ __forceinline__ void fpiSums(const sphdem_adj_fields& in, const sphde
                                         const int32_t* __restrict__ pimg, Fpi& o) {
   o.S = o.Pn = 0.0;
   o.U = o.Gp = o.Gv = make_double3(0.0, 0.0, 0.0);
-  for (int64_t j = j0; j < j1; j++) {
+  for (int64_t j = j0 + queryLane<kFpiLanes>(); j < j1; j += kFpiLanes) {
     const int n = pb[j];
     const double3 rn = imageOf(in.r, n, pimg[j], C.shift_len);
     const double dx = rp.x - rn.x, dy = rp.y - rn.y, dz = rp.z - rn.z;
@@ -673,19 +742,21 @@ __device__ __forceinline__ void fpiSums(const sphdem_adj_fields& in, const sphde
     o.Gv.y += (mW + dvW) * fvn.y;
     o.Gv.z += (mW + dvW) * fvn.z;
   }
+  sumLanes<kFpiLanes>(o.S, o.Pn, o.U.x, o.U.y, o.U.z, o.Gp.x, o.Gp.y, o.Gp.z, o.Gv.x, o.Gv.y,
+                      o.Gv.z);
 }
 
 __global__ void __launch_bounds__(kTPB) k_fpi_fwd(int32_t nq, const int32_t* __restrict__ query,
                           const int64_t* __restrict__ off, const int32_t* __restrict__ pb,
                           const int32_t* __restrict__ pimg, sphdem_adj_fields in,
                           sphdem_adj_consts C, double* __restrict__ fdrag) {
-  const int i = xcdIndex();
+  const int i = queryIndex<kFpiLanes>();
   if (i >= nq) return;
   const int p = query[i];
   const double3 rp = ld3(in.r, p);
   Fpi o;
   fpiSums(in, C, rp, off[i], off[i + 1], pb, pimg, o);
-  if (!(o.S > 0.5)) return;
+  if (queryLane<kFpiLanes>() != 0 || !(o.S > 0.5)) return;
   const double iS = 1.0 / o.S;
   const double por = o.Pn * iS;
   const double3 vp = ld3(in.vhat, p);
@@ -714,7 +785,8 @@ __global__ void __launch_bounds__(kTPB) k_fpi_bwd(int32_t nq, const int32_t* __r
                           const int32_t* __restrict__ pimg, sphdem_adj_fields in,
                           sphdem_adj_consts C, const double* __restrict__ gfd,
                           sphdem_adj_grads g) {
-  const int i = xcdIndex();
+  const int i = queryIndex<kFpiLanes>(), gl = queryLane<kFpiLanes>();
+  __shared__ Add3Stage stage[kTPB / 64];
   double gpar[3] = {0.0, 0.0, 0.0};  // nu, drag_a, drag_b
   const int p = i < nq ? query[i] : 0;
   Fpi o;
@@ -774,7 +846,7 @@ __global__ void __launch_bounds__(kTPB) k_fpi_bwd(int32_t nq, const int32_t* __r
       // dv = por (fvel - vhat_p)
       porbar += dvbx * ex + dvby * ey + dvbz * ez;
       fvelbar = make_double3(por * dvbx, por * dvby, por * dvbz);
-      add3(g.vhat, p, -por * dvbx, -por * dvby, -por * dvbz);
+      if (gl == 0) add3(g.vhat, p, -por * dvbx, -por * dvby, -por * dvbz);
     }
     // fvel = U/S, por = Pn/S
     const double3 Ubar = make_double3(fvelbar.x * iS, fvelbar.y * iS, fvelbar.z * iS);
@@ -783,40 +855,51 @@ __global__ void __launch_bounds__(kTPB) k_fpi_bwd(int32_t nq, const int32_t* __r
     Sbar -= porbar * por * iS;
     // back through the sums, pair by pair
     double rpx = 0.0, rpy = 0.0, rpz = 0.0;
-    for (int64_t j = off[i]; j < off[i + 1]; j++) {
-      const int n = pb[j];
-      const double3 rn = imageOf(in.r, n, pimg[j], C.shift_len);
-      const double dx = rp.x - rn.x, dy = rp.y - rn.y, dz = rp.z - rn.z;
-      const double r = sqrt(dx * dx + dy * dy + dz * dz);
-      double W, dWdr, dWdh;
-      wendW(C.wcon, r, in.h[n], W, dWdr, dWdh);
-      if (W == 0.0 && dWdr == 0.0 && dWdh == 0.0) continue;
-      const double mn = in.mass[n], rhon = in.dens[n];
-      const double dvol = mn / rhon;
-      const double dvW = dvol * W, mW = mn * W;
-      const double3 vn = ld3(in.vhat, n), fpn = ld3(in.fpfb, n), fvn = ld3(in.fv, n);
-      const double porn = in.por[n];
-      const double dvWbar = Ubar.x * vn.x + Ubar.y * vn.y + Ubar.z * vn.z + Pnbar * porn + Sbar +
-                            Gbar.x * fvn.x + Gbar.y * fvn.y + Gbar.z * fvn.z;
-      const double mWbar = Gbar.x * (fpn.x + fvn.x) + Gbar.y * (fpn.y + fvn.y) +
-                           Gbar.z * (fpn.z + fvn.z);
-      add3(g.vhat, n, dvW * Ubar.x, dvW * Ubar.y, dvW * Ubar.z);
-      add1(g.por, n, dvW * Pnbar);
-      add3(g.fpfb, n, mW * Gbar.x, mW * Gbar.y, mW * Gbar.z);
-      add3(g.fv, n, (mW + dvW) * Gbar.x, (mW + dvW) * Gbar.y, (mW + dvW) * Gbar.z);
-      const double Wbar = dvWbar * dvol + mWbar * mn;
-      add1(g.dens, n, -dvWbar * W * mn / (rhon * rhon));
-      add1(g.h, n, Wbar * dWdh);
-      if (r > 0.0) {
-        const double c = Wbar * dWdr / r;
-        rpx += c * dx;
-        rpy += c * dy;
-        rpz += c * dz;
-        add3(g.r, n, -c * dx, -c * dy, -c * dz);
+    for (int64_t jw = off[i]; jw < off[i + 1]; jw += kFpiLanes) {
+      const int64_t j = jw + gl;
+      int n = -1;
+      double dvW = 0.0, mW = 0.0, c = 0.0, dx = 0.0, dy = 0.0, dz = 0.0;
+      if (j < off[i + 1]) {
+        n = pb[j];
+        const double3 rn = imageOf(in.r, n, pimg[j], C.shift_len);
+        dx = rp.x - rn.x, dy = rp.y - rn.y, dz = rp.z - rn.z;
+        const double r = sqrt(dx * dx + dy * dy + dz * dz);
+        double W, dWdr, dWdh;
+        wendW(C.wcon, r, in.h[n], W, dWdr, dWdh);
+        if (W == 0.0 && dWdr == 0.0 && dWdh == 0.0) {
+          n = -1;
+        } else {
+          const double mn = in.mass[n], rhon = in.dens[n];
+          const double dvol = mn / rhon;
+          dvW = dvol * W, mW = mn * W;
+          const double3 vn = ld3(in.vhat, n), fpn = ld3(in.fpfb, n), fvn = ld3(in.fv, n);
+          const double porn = in.por[n];
+          const double dvWbar = Ubar.x * vn.x + Ubar.y * vn.y + Ubar.z * vn.z + Pnbar * porn +
+                                Sbar + Gbar.x * fvn.x + Gbar.y * fvn.y + Gbar.z * fvn.z;
+          const double mWbar = Gbar.x * (fpn.x + fvn.x) + Gbar.y * (fpn.y + fvn.y) +
+                               Gbar.z * (fpn.z + fvn.z);
+          const double Wbar = dvWbar * dvol + mWbar * mn;
+          add1(g.por, n, dvW * Pnbar);
+          add1(g.dens, n, -dvWbar * W * mn / (rhon * rhon));
+          add1(g.h, n, Wbar * dWdh);
+          if (r > 0.0) {
+            c = Wbar * dWdr / r;
+            rpx += c * dx;
+            rpy += c * dy;
+            rpz += c * dz;
+          }
+        }
       }
+      waveAdd3(stage[threadIdx.x >> 6], g.vhat, n, dvW * Ubar.x, dvW * Ubar.y, dvW * Ubar.z);
+      waveAdd3(stage[threadIdx.x >> 6], g.fpfb, n, mW * Gbar.x, mW * Gbar.y, mW * Gbar.z);
+      const double w = mW + dvW;
+      waveAdd3(stage[threadIdx.x >> 6], g.fv, n, w * Gbar.x, w * Gbar.y, w * Gbar.z);
+      waveAdd3(stage[threadIdx.x >> 6], g.r, n, -c * dx, -c * dy, -c * dz);
     }
-    add3(g.r, p, rpx, rpy, rpz);
+    sumLanes<kFpiLanes>(rpx, rpy, rpz);
+    if (gl == 0) add3(g.r, p, rpx, rpy, rpz);
   }
+  if (gl != 0) gpar[0] = gpar[1] = gpar[2] = 0.0;  // every lane holds the query's
   blockAdd<3>(gpar, g.params);
 }
 
@@ -888,7 +971,9 @@ __global__ void __launch_bounds__(kTPB) k_contacts_bwd(int64_t np, const int32_t
   blockAdd<2>(gpar, g.params + 3);
 }
 
-inline unsigned gridFor(int64_t n) { return (unsigned)((n + kTPB - 1) / kTPB); }
+inline unsigned gridFor(int64_t n, int lanes = 1) {
+  return (unsigned)((n * lanes + kTPB - 1) / kTPB);
+}
 
 }  // namespace sphdem_adj
 
@@ -945,7 +1030,7 @@ int sphdem_adj_force(int32_t nquery, const int32_t* query, const int64_t* off, c
   if (!SPHDEM_ADJ_CSR_OK(in) || !in->h || !in->vhat || !in->dens || !in->omega || !in->pdr2 ||
       !in->iam)
     return SPHDEM_E_ARG;
-  hipLaunchKernelGGL(sphdem_adj::k_force_fwd, dim3(sphdem_adj::gridFor(nquery)),
+  hipLaunchKernelGGL(sphdem_adj::k_force_fwd, dim3(sphdem_adj::gridFor(nquery, sphdem_adj::kSphLanes)),
                      dim3(sphdem_adj::kTPB), 0, (hipStream_t)stream, nquery, query, off, b, img,
                      *in, *c, fv, fp);
   return adjLaunched();
@@ -960,7 +1045,7 @@ int sphdem_adj_force_bwd(int32_t nquery, const int32_t* query, const int64_t* of
   if (!SPHDEM_ADJ_CSR_OK(in) || !in->h || !in->vhat || !in->dens || !in->omega || !in->pdr2 ||
       !in->iam || !g->r || !g->vhat || !g->h || !g->dens || !g->omega || !g->pdr2 || !g->params)
     return SPHDEM_E_ARG;
-  hipLaunchKernelGGL(sphdem_adj::k_force_bwd, dim3(sphdem_adj::gridFor(nquery)),
+  hipLaunchKernelGGL(sphdem_adj::k_force_bwd, dim3(sphdem_adj::gridFor(nquery, sphdem_adj::kSphLanes)),
                      dim3(sphdem_adj::kTPB), 0, (hipStream_t)stream, nquery, query, off, b, img,
                      *in, *c, gfv, gfp, *g);
   return adjLaunched();
@@ -972,7 +1057,7 @@ int sphdem_adj_omega(int32_t nquery, const int32_t* query, const int64_t* off, c
   if (nquery < 0 || !in || !c || !omega) return SPHDEM_E_ARG;
   if (nquery == 0) return 0;
   if (!SPHDEM_ADJ_CSR_OK(in) || !in->h || !in->dens) return SPHDEM_E_ARG;
-  hipLaunchKernelGGL(sphdem_adj::k_omega_fwd, dim3(sphdem_adj::gridFor(nquery)),
+  hipLaunchKernelGGL(sphdem_adj::k_omega_fwd, dim3(sphdem_adj::gridFor(nquery, sphdem_adj::kSphLanes)),
                      dim3(sphdem_adj::kTPB), 0, (hipStream_t)stream, nquery, query, off, b, img,
                      *in, *c, omega);
   return adjLaunched();
@@ -986,7 +1071,7 @@ int sphdem_adj_omega_bwd(int32_t nquery, const int32_t* query, const int64_t* of
   if (nquery == 0) return 0;
   if (!SPHDEM_ADJ_CSR_OK(in) || !in->h || !in->dens || !g->r || !g->h || !g->dens)
     return SPHDEM_E_ARG;
-  hipLaunchKernelGGL(sphdem_adj::k_omega_bwd, dim3(sphdem_adj::gridFor(nquery)),
+  hipLaunchKernelGGL(sphdem_adj::k_omega_bwd, dim3(sphdem_adj::gridFor(nquery, sphdem_adj::kSphLanes)),
                      dim3(sphdem_adj::kTPB), 0, (hipStream_t)stream, nquery, query, off, b, img,
                      *in, *c, gomega, *g);
   return adjLaunched();
@@ -998,7 +1083,7 @@ int sphdem_adj_dddt(int32_t nquery, const int32_t* query, const int64_t* off, co
   if (nquery < 0 || !in || !c || !dddt) return SPHDEM_E_ARG;
   if (nquery == 0) return 0;
   if (!SPHDEM_ADJ_CSR_OK(in) || !in->h || !in->vhat || !in->omega) return SPHDEM_E_ARG;
-  hipLaunchKernelGGL(sphdem_adj::k_dddt_fwd, dim3(sphdem_adj::gridFor(nquery)),
+  hipLaunchKernelGGL(sphdem_adj::k_dddt_fwd, dim3(sphdem_adj::gridFor(nquery, sphdem_adj::kSphLanes)),
                      dim3(sphdem_adj::kTPB), 0, (hipStream_t)stream, nquery, query, off, b, img,
                      *in, *c, dddt);
   return adjLaunched();
@@ -1013,7 +1098,7 @@ int sphdem_adj_dddt_bwd(int32_t nquery, const int32_t* query, const int64_t* off
   if (!SPHDEM_ADJ_CSR_OK(in) || !in->h || !in->vhat || !in->omega || !g->r || !g->vhat || !g->h ||
       !g->omega)
     return SPHDEM_E_ARG;
-  hipLaunchKernelGGL(sphdem_adj::k_dddt_bwd, dim3(sphdem_adj::gridFor(nquery)),
+  hipLaunchKernelGGL(sphdem_adj::k_dddt_bwd, dim3(sphdem_adj::gridFor(nquery, sphdem_adj::kSphLanes)),
                      dim3(sphdem_adj::kTPB), 0, (hipStream_t)stream, nquery, query, off, b, img,
                      *in, *c, gdddt, *g);
   return adjLaunched();
@@ -1027,7 +1112,7 @@ int sphdem_adj_coupling(int32_t nquery, const int32_t* query, const int64_t* off
   if (nquery == 0) return 0;
   const int32_t* b = d;
   if (!SPHDEM_ADJ_CSR_OK(in) || !in->dens || !in->fdrag) return SPHDEM_E_ARG;
-  const dim3 grid(sphdem_adj::gridFor(nquery)), block(sphdem_adj::kTPB);
+  const dim3 grid(sphdem_adj::gridFor(nquery, sphdem_adj::kCplLanes)), block(sphdem_adj::kTPB);
   hipLaunchKernelGGL(sphdem_adj::k_cpl_fwd1, grid, block, 0, (hipStream_t)stream, nquery, query,
                      off, d, img, *in, *c, por_sum, shep);
   if (adjLaunched()) return SPHDEM_E_HIP;
@@ -1048,12 +1133,12 @@ int sphdem_adj_coupling_bwd(int32_t nquery, const int32_t* query, const int64_t*
   if (!SPHDEM_ADJ_CSR_OK(in) || !in->dens || !in->fdrag || !in->shep || !g->r || !g->dens ||
       !g->fdrag)
     return SPHDEM_E_ARG;
-  const dim3 grid(sphdem_adj::gridFor(nquery)), block(sphdem_adj::kTPB);
+  const dim3 grid(sphdem_adj::gridFor(nquery, sphdem_adj::kCplLanes)), block(sphdem_adj::kTPB);
   hipLaunchKernelGGL(sphdem_adj::k_cpl_bwd1, grid, block, 0, (hipStream_t)stream, nquery, query,
-                     off, d, img, *in, *c, gpor, gdrag, work, *g);
+                     off, d, img, *in, *c, gdrag, work);
   if (adjLaunched()) return SPHDEM_E_HIP;
   hipLaunchKernelGGL(sphdem_adj::k_cpl_bwd2, grid, block, 0, (hipStream_t)stream, nquery, query,
-                     off, d, img, *in, *c, (const double*)work, *g);
+                     off, d, img, *in, *c, gpor, gdrag, (const double*)work, *g);
   return adjLaunched();
 }
 
@@ -1078,12 +1163,12 @@ int sphdem_adj_coupling_bwd_noalloc(int32_t nquery, const int32_t* query, const 
                        (hipStream_t)stream, work, n);
     if (adjLaunched()) return SPHDEM_E_HIP;
   }
-  const dim3 grid(sphdem_adj::gridFor(nquery)), block(sphdem_adj::kTPB);
+  const dim3 grid(sphdem_adj::gridFor(nquery, sphdem_adj::kCplLanes)), block(sphdem_adj::kTPB);
   hipLaunchKernelGGL(sphdem_adj::k_cpl_bwd1, grid, block, 0, (hipStream_t)stream, nquery, query,
-                     off, d, img, *in, *c, gpor, gdrag, work, *g);
+                     off, d, img, *in, *c, gdrag, work);
   if (adjLaunched()) return SPHDEM_E_HIP;
   hipLaunchKernelGGL(sphdem_adj::k_cpl_bwd2, grid, block, 0, (hipStream_t)stream, nquery, query,
-                     off, d, img, *in, *c, (const double*)work, *g);
+                     off, d, img, *in, *c, gpor, gdrag, (const double*)work, *g);
   return adjLaunched();
 }
 
@@ -1095,7 +1180,7 @@ int sphdem_adj_fpi(int32_t nquery, const int32_t* query, const int64_t* off, con
   if (!query || !off || !b || !img || !in->r || !in->vhat || !in->h || !in->dens ||
       !in->mass || !in->fpfb || !in->fv || !in->por)
     return SPHDEM_E_ARG;
-  hipLaunchKernelGGL(sphdem_adj::k_fpi_fwd, dim3(sphdem_adj::gridFor(nquery)),
+  hipLaunchKernelGGL(sphdem_adj::k_fpi_fwd, dim3(sphdem_adj::gridFor(nquery, sphdem_adj::kFpiLanes)),
                      dim3(sphdem_adj::kTPB), 0, (hipStream_t)stream, nquery, query, off, b, img,
                      *in, *c, fdrag);
   return adjLaunched();
@@ -1111,7 +1196,7 @@ int sphdem_adj_fpi_bwd(int32_t nquery, const int32_t* query, const int64_t* off,
       !in->mass || !in->fpfb || !in->fv || !in->por || !g->r || !g->vhat || !g->h ||
       !g->dens || !g->fpfb || !g->fv || !g->por || !g->params)
     return SPHDEM_E_ARG;
-  hipLaunchKernelGGL(sphdem_adj::k_fpi_bwd, dim3(sphdem_adj::gridFor(nquery)),
+  hipLaunchKernelGGL(sphdem_adj::k_fpi_bwd, dim3(sphdem_adj::gridFor(nquery, sphdem_adj::kFpiLanes)),
                      dim3(sphdem_adj::kTPB), 0, (hipStream_t)stream, nquery, query, off, b, img,
                      *in, *c, gfdrag, *g);
   return adjLaunched();
