@@ -860,6 +860,77 @@ __device__ __forceinline__ void forCellRanges(const Grid& g, const int* __restri
   }
 }
 
+__device__ __forceinline__ int imageCode(int sx, int sy, int sz) {
+  return (sx + 1) + 3 * (sy + 1) + 9 * (sz + 1);
+}
+// The same ranges for a wavefront's query: visit(j0, len, code) once per 64
+// columns of an image, with the ranges [j0, j0 + len) of consecutive lanes in
+// forCells' order, so that their bounds are one round of loads and the
+// candidates come 64 at a time whatever the columns hold (a column by itself: two
+// dependent rounds each, 81 candidates in 128 lanes).  k_shepsum of 64 k spheres
+// beside the list search 1.75 -> 1.29 ms, of 4096 30 -> 24 us; k_fpi of 64 k
+// 3.0 -> 2.5 ms, of 64 (a 16^3 box) 34 -> 22 us.
+template <class V>
+__device__ __forceinline__ void waveCellRanges(const Grid& g, const int* __restrict__ start,
+                                               const Box& B, double qx, double qy, double qz,
+                                               int reach, int lane, V&& visit) {
+  const int nsx = B.periodic[0] ? 3 : 1, nsy = B.periodic[1] ? 3 : 1, nsz = B.periodic[2] ? 3 : 1;
+  for (int ix = 0; ix < nsx; ix++) {
+    const int sx = ix == 0 ? 0 : (ix == 1 ? -1 : 1);
+    const CellSpan cx =
+        cellSpan(sx == 0 ? qx : (sx == 1 ? qx - B.Lp[0] : qx - B.Lm[0]), g, 0, reach, 0.0);
+    if (cx.lo > cx.hi) continue;
+    for (int iy = 0; iy < nsy; iy++) {
+      const int sy = iy == 0 ? 0 : (iy == 1 ? -1 : 1);
+      const CellSpan cy =
+          cellSpan(sy == 0 ? qy : (sy == 1 ? qy - B.Lp[1] : qy - B.Lm[1]), g, 1, reach, 0.0);
+      if (cy.lo > cy.hi) continue;
+      for (int iz = 0; iz < nsz; iz++) {
+        const int sz = iz == 0 ? 0 : (iz == 1 ? -1 : 1);
+        const CellSpan cz =
+            cellSpan(sz == 0 ? qz : (sz == 1 ? qz - B.Lp[2] : qz - B.Lm[2]), g, 2, reach, 0.0);
+        if (cz.lo > cz.hi) continue;
+        const int ny = cy.hi - cy.lo + 1, ncol = (cx.hi - cx.lo + 1) * ny;
+        for (int c0 = 0; c0 < ncol; c0 += 64) {
+          int j0 = 0, len = 0;
+          if (c0 + lane < ncol) {
+            const int c = c0 + lane;
+            const int k0 = g.base + ((cx.lo + c / ny) * g.dim[1] + cy.lo + c % ny) * g.dim[2];
+            j0 = start[k0 + cz.lo];
+            len = start[k0 + cz.hi + 1] - j0;
+          }
+          visit(j0, len, imageCode(sx, sy, sz));
+        }
+      }
+    }
+  }
+}
+// Entries of the ranges that consecutive lanes hold, 64 at a time.
+struct WaveEntries {
+  int j0, len;
+  unsigned long long cols;  // ranges not finished
+  int off = 0;              // entries of the first of them already taken
+  __device__ __forceinline__ WaveEntries(int j0_, int len_)
+      : j0(j0_), len(len_), cols(__ballot(len_ > 0)) {}
+  // the next entries (up to 64): this lane's in j; returns how many
+  __device__ __forceinline__ int next(int lane, int& j) {
+    int n = 0;
+    while (cols && n < 64) {
+      const int c = __builtin_ctzll(cols);
+      const int left = __builtin_amdgcn_readlane(len, c) - off, at = lane - n;
+      if (at >= 0 && at < left) j = __builtin_amdgcn_readlane(j0, c) + off + at;
+      const int took = min(left, 64 - n);
+      n += took;
+      off += took;
+      if (took == left) {
+        cols &= cols - 1;
+        off = 0;
+      }
+    }
+    return n;
+  }
+};
+
 // Accepted candidates of one wavefront, compacted in LDS so that the pair
 // arithmetic runs on full wavefronts: lanes test 64 consecutive candidates,
 // the accepted ones are appended in lane order (ballot + prefix count), and
@@ -867,13 +938,14 @@ __device__ __forceinline__ void forCellRanges(const Grid& g, const int* __restri
 // The order of the entries, and so of every lane's partial sums, depends
 // only on the candidate order: results are the same run to run.
 constexpr int kCompactCap = 128;  // 64 carried over + 64 appended
-// ranges(visit) calls visit(j0, j1, code) for each candidate range (code: an
-// image code the body receives with the candidate); test(j, code) decides a
-// candidate, body(j, code) runs for each accepted one.
-template <class Ranges, class Test, class Body>
+// ranges(visit) calls visit(j0, len, code) as waveCellRanges does (code: an
+// image code the body receives with the candidate); load(j) fetches what
+// test(data, j, code) decides a candidate by, 64 candidates ahead of it;
+// body(j, code) runs for each accepted one.
+template <class Ranges, class Load, class Test, class Body>
 __device__ __forceinline__ void compactedPairs(int* __restrict__ lb, int* __restrict__ lc,
-                                               int lane, Ranges&& ranges, Test&& test,
-                                               Body&& body) {
+                                               int lane, Ranges&& ranges, Load&& load,
+                                               Test&& test, Body&& body) {
   int cnt = 0;  // wave-uniform
   auto flush = [&](int m) {
     __builtin_amdgcn_wave_barrier();
@@ -881,10 +953,18 @@ __device__ __forceinline__ void compactedPairs(int* __restrict__ lb, int* __rest
     if (lane < m) body(lb[lane], lc[lane]);
     __builtin_amdgcn_wave_barrier();
   };
-  ranges([&](int j0, int j1, int code) {
-    for (int jj = j0; jj < j1; jj += 64) {
-      const int j = jj + lane;
-      const bool ok = j < j1 && test(j, code);
+  ranges([&](int j0, int len, int code) {
+    WaveEntries E(j0, len);
+    int jn = 0, n = E.next(lane, jn);
+    if (n == 0) return;
+    if (lane >= n) jn = __builtin_amdgcn_readfirstlane(jn);  // loads stay in the store
+    auto ahead = load(jn);
+    while (n > 0) {
+      const int j = jn, m0 = n;
+      const auto data = ahead;
+      n = E.next(lane, jn);
+      if (n > 0) ahead = load(jn);  // lanes past n: an earlier entry again
+      const bool ok = lane < m0 && test(data, j, code);
       const unsigned long long m = __ballot(ok);
       if (ok) {
         const int at = cnt + (int)__builtin_amdgcn_mbcnt_hi(
@@ -911,9 +991,6 @@ __device__ __forceinline__ void compactedPairs(int* __restrict__ lb, int* __rest
     }
   });
   if (cnt > 0) flush(cnt);
-}
-__device__ __forceinline__ int imageCode(int sx, int sy, int sz) {
-  return (sx + 1) + 3 * (sy + 1) + 9 * (sz + 1);
 }
 __device__ __forceinline__ void imageShift(int code, int& sx, int& sy, int& sz) {
   sx = code % 3 - 1;
@@ -947,17 +1024,22 @@ __device__ __forceinline__ int demCell(const CouplingRule& R, double x, int d) {
 // accepted(l2) with the whole-cell (addAll) branch; `full` keeps addAll pairs
 // whatever their distance (the reference's list), otherwise only pairs that
 // can carry a nonzero kernel value are reported.
-__device__ __forceinline__ bool couplingAccept(const CouplingRule& R, const int* ca, double ix,
-                                               double iy, double iz, double l2, bool full) {
-  const int d0 = demCell(R, ix, 0) - ca[0];
-  const int d1 = demCell(R, iy, 1) - ca[1];
-  const int d2 = demCell(R, iz, 2) - ca[2];
+// d: the image's DEM cell less the SPH particle's.
+__device__ __forceinline__ bool cellsAccept(const CouplingRule& R, int d0, int d1, int d2,
+                                            double l2, bool full) {
   if (d0 < -R.nc || d0 > R.nc || d1 < -R.nc || d1 > R.nc || d2 < -R.nc || d2 > R.nc) return false;
   const int plus = (d0 + 1) * (d0 + 1) + (d1 + 1) * (d1 + 1) + (d2 + 1) * (d2 + 1);
   const int minus = (d0 - 1) * (d0 - 1) + (d1 - 1) * (d1 - 1) + (d2 - 1) * (d2 - 1);
   if (plus < R.thr) return full || l2 <= R.skip2;
   if (minus < R.thr) return l2 < R.rc2;
   return false;
+}
+__device__ __forceinline__ bool couplingAccept(const CouplingRule& R, const int* ca, double ix,
+                                               double iy, double iz, double l2, bool full) {
+  const int d0 = demCell(R, ix, 0) - ca[0];
+  const int d1 = demCell(R, iy, 1) - ca[1];
+  const int d2 = demCell(R, iz, 2) - ca[2];
+  return cellsAccept(R, d0, d1, d2, l2, full);
 }
 __device__ __forceinline__ bool demImageExists(const CouplingRule& R, const Box& B,
                                                const double4& p, int sx, int sy, int sz) {
@@ -1001,28 +1083,32 @@ __global__ void __launch_bounds__(256) k_shepsum(Store S, int ns, int nd, Grid g
           const int sz = iz == 0 ? 0 : (iz == 1 ? -1 : 1);
           if ((sx | sy | sz) != 0 && !demImageExists(R, B, pj, sx, sy, sz)) continue;
           const Img im = imagePos(pj, sx, sy, sz, B);
-          forCellRanges(gs, start, B0, im.x, im.y, im.z, reach,
-                        [&](int j0, int j1, int, int, int) { visit(j0, j1, imageCode(sx, sy, sz)); });
+          waveCellRanges(gs, start, B0, im.x, im.y, im.z, reach, lane,
+                         [&](int j0, int len, int) { visit(j0, len, imageCode(sx, sy, sz)); });
         }
   };
-  auto dist2 = [&](int a, int code, Img& im) {
+  auto dist2 = [&](const double4& pa, int code, Img& im) {
     int sx, sy, sz;
     imageShift(code, sx, sy, sz);
     im = imagePos(pj, sx, sy, sz, B);
-    const double4 pa = S.posh[a];
     const double dx = pa.x - im.x, dy = pa.y - im.y, dz = pa.z - im.z;
     return dot3(dx, dy, dz, dx, dy, dz);
   };
   // the test keeps the cheap distance cut; the coupling cell rule runs on the
   // compacted candidates
-  compactedPairs(lbuf[w], lcode[w], lane, ranges, [&](int a, int code) {
-    if (!isSphT(S.iam[a])) return false;
+  struct Cand {
+    double4 p;
+    int t;
+  };
+  compactedPairs(lbuf[w], lcode[w], lane, ranges, [&](int a) {
+    return Cand{S.posh[a], S.iam[a]};
+  }, [&](const Cand& c, int, int code) {
     Img im;
-    return dist2(a, code, im) <= R.skip2;
+    return isSphT(c.t) && dist2(c.p, code, im) <= R.skip2;
   }, [&](int a, int code) {
     Img im;
-    const double l2 = dist2(a, code, im);
     const double4 pa = S.posh[a];
+    const double l2 = dist2(pa, code, im);
     const int ca[3] = {demCell(R, pa.x, 0), demCell(R, pa.y, 1), demCell(R, pa.z, 2)};
     if (!couplingAccept(R, ca, im.x, im.y, im.z, l2, false)) return;
     const double dv = S.vhm[a].w / S.dpo[a].x;
@@ -1033,9 +1119,6 @@ __global__ void __launch_bounds__(256) k_shepsum(Store S, int ns, int nd, Grid g
   if (lane == 0) S.fp[j].w = sum;
 }
 
-// SPH side of middle()'s coupling block (sphIncompress.cpp:64-78): calcPorosity
-// (sph.h:1323-1341), calcDEMtoSPHDrag (sph.h:1343-1362) and finalisePorosity
-// (sph.h:1289-1296), one gather over the DEM partners.
 // DEM cells with a DEM particle within one cell (the 3x3x3 block around them):
 // near[c] == gen.  A coupling search centred on any other cell of the DEM grid
 // finds no candidate and is skipped.
@@ -1053,43 +1136,153 @@ __global__ void k_dem_near(Store S, int ns, int nd, Grid gc, int* __restrict__ n
         near[(a * gc.dim[1] + b) * gc.dim[2] + d] = gen;
 }
 
-__global__ void k_coupling_sph(Store S, int ns, int nd, Grid gc, const int* __restrict__ start,
-                               Box B, CouplingRule R, sphdem_params P,
-                               const int* __restrict__ near, const int* __restrict__ genp) {
+// SPH side of middle()'s coupling block (sphIncompress.cpp:64-78): calcPorosity
+// (sph.h:1323-1341), calcDEMtoSPHDrag (sph.h:1343-1362) and finalisePorosity
+// (sph.h:1289-1296), one gather over the DEM partners.
+//
+// A lane per SPH particle; the spheres are taken by the wavefront.  Its 64
+// consecutive particles lie in a cell or three of one column, so their 27-cell
+// blocks of the DEM grid nearly coincide: for each column group (and image shift)
+// the lanes read the bounds of all cell columns around the group at once, load
+// 64 spheres at a time (position, cell, drag and sums: a lane a sphere) into
+// LDS, and every lane goes through these in the order it would meet them alone;
+// what lies outside its own block fails its distance test.
+//
+// What bounds it: the FP64 arithmetic of the tests and accepted pairs.  A walk of
+// each lane's own cells is a chain of some 40 dependent loads, and takes the
+// accepted pairs' arithmetic whenever one lane has one.  286 k particles with
+// 4096 spheres 65 us alone, 106 beside the list search; so 39 and 54 us.  4.9 M
+// with 64 k spheres 956 us; so 564.
+constexpr int kCplColumns = 64;
+struct CplSphere {
+  double x, y, z;        // the image's position
+  double s, fx, fy, fz;  // mass / Shepard sum, drag
+  int c0, c1, c2, pad;   // its DEM cell
+};
+__global__ void __launch_bounds__(256) k_coupling_sph(Store S, int ns, int nd, Grid gc,
+                                                      const int* __restrict__ start, Box B,
+                                                      CouplingRule R, sphdem_params P,
+                                                      const int* __restrict__ near,
+                                                      const int* __restrict__ genp) {
+  __shared__ CplSphere buf[4][64];
+  CplSphere* const L = buf[threadIdx.x >> 6];
+  const int lane = threadIdx.x & 63;
   const int a = xcdThread();
-  if (a >= ns || !isSphT(S.iam[a])) return;
+  const bool act = a < ns && isSphT(S.iam[a]);
+  const int al = a < ns ? a : ns - 1;
   const int gen = *genp;
-  const double4 pa = S.posh[a];
+  const double4 pa = S.posh[al];
+  const int cell = S.cell[al] & ((1 << 22) - 1);  // the SPH column
   const double Rc = P.coupling_radius;
-  const double rdens = 1.0 / S.dpo[a].x;
+  const double rdens = 1.0 / S.dpo[al].x;
   const int ca[3] = {demCell(R, pa.x, 0), demCell(R, pa.y, 1), demCell(R, pa.z, 2)};
   double por = 0.0;
   double fd0 = 0.0, fd1 = 0.0, fd2 = 0.0;
-  // forCells over the DEM grid, skipping each image shift whose centre cell
-  // lies in the grid with no DEM particle around it
-  auto keep = [&](int cx, int cy, int cz) {
-    if (cx < 0 || cy < 0 || cz < 0 || cx >= gc.dim[0] || cy >= gc.dim[1] || cz >= gc.dim[2])
-      return true;
-    return near[(cx * gc.dim[1] + cy) * gc.dim[2] + cz] == gen;
-  };
-  forCells(gc, start, B, pa.x, pa.y, pa.z, 1, [&](int j, int sx, int sy, int sz) {
-    const double4 pj = S.posh[j];
-    if ((sx | sy | sz) != 0 && !demImageExists(R, B, pj, sx, sy, sz)) return;
-    const Img im = imagePos(pj, sx, sy, sz, B);
-    const double dx = pa.x - im.x, dy = pa.y - im.y, dz = pa.z - im.z;
-    const double l2 = dot3(dx, dy, dz, dx, dy, dz);
-    if (l2 > R.skip2) return;
-    if (!couplingAccept(R, ca, im.x, im.y, im.z, l2, false)) return;
-    const double r = sqrt(l2);
-    const double w = wendW(P.wcon, r * (2.0 / Rc), Rc / 2.0);
-    por += P.porosity_incr * w;
-    const double4 fdj = S.fdrag[j];
-    const double s = S.vhm[j].w * rdens;
-    const double shep = S.fp[j].w;
-    fd0 -= s * fdj.x * w / shep;
-    fd1 -= s * fdj.y * w / shep;
-    fd2 -= s * fdj.z * w / shep;
-  }, 0, 1, keep);
+  const int nsx = B.periodic[0] ? 3 : 1, nsy = B.periodic[1] ? 3 : 1, nsz = B.periodic[2] ? 3 : 1;
+  for (int ix = 0; ix < nsx; ix++) {
+    const int sx = ix == 0 ? 0 : (ix == 1 ? -1 : 1);
+    const int cx = cellOf(sx == 0 ? pa.x : (sx == 1 ? pa.x - B.Lp[0] : pa.x - B.Lm[0]), gc, 0);
+    if (!__any(act && cx >= -1 && cx <= gc.dim[0])) continue;
+    for (int iy = 0; iy < nsy; iy++) {
+      const int sy = iy == 0 ? 0 : (iy == 1 ? -1 : 1);
+      const int cy = cellOf(sy == 0 ? pa.y : (sy == 1 ? pa.y - B.Lp[1] : pa.y - B.Lm[1]), gc, 1);
+      if (!__any(act && cy >= -1 && cy <= gc.dim[1])) continue;
+      for (int iz = 0; iz < nsz; iz++) {
+        const int sz = iz == 0 ? 0 : (iz == 1 ? -1 : 1);
+        const int cz = cellOf(sz == 0 ? pa.z : (sz == 1 ? pa.z - B.Lp[2] : pa.z - B.Lm[2]), gc, 2);
+        // searched where the block overlaps the grid, but for a centre cell with
+        // no sphere around it
+        bool want = act && cx >= -1 && cx <= gc.dim[0] && cy >= -1 && cy <= gc.dim[1] &&
+                    cz >= -1 && cz <= gc.dim[2];
+        if (want && cx >= 0 && cy >= 0 && cz >= 0 && cx < gc.dim[0] && cy < gc.dim[1] &&
+            cz < gc.dim[2])
+          want = near[(cx * gc.dim[1] + cy) * gc.dim[2] + cz] == gen;
+        unsigned long long todo = __ballot(want);
+        while (todo) {
+          // a group: one column of the SPH grid, a few cells of it
+          const int lead = __builtin_ctzll(todo);
+          const int lc = __builtin_amdgcn_readlane(cell, lead);
+          int x0 = __builtin_amdgcn_readlane(cx, lead), x1 = x0;
+          int y0 = __builtin_amdgcn_readlane(cy, lead), y1 = y0;
+          int z0 = __builtin_amdgcn_readlane(cz, lead), z1 = z0;
+          const bool in = ((todo >> lane) & 1) && cell == lc && cz >= z0 - 4 && cz <= z0 + 4;
+          todo &= ~__ballot(in);
+          while (__any(in && cx < x0)) x0--;
+          while (__any(in && cx > x1)) x1++;
+          while (__any(in && cy < y0)) y0--;
+          while (__any(in && cy > y1)) y1++;
+          while (__any(in && cz < z0)) z0--;
+          while (__any(in && cz > z1)) z1++;
+          x0 = max(x0 - 1, 0), x1 = min(x1 + 1, gc.dim[0] - 1);
+          y0 = max(y0 - 1, 0), y1 = min(y1 + 1, gc.dim[1] - 1);
+          z0 = max(z0 - 1, 0), z1 = min(z1 + 1, gc.dim[2] - 1);
+          const int ny = y1 - y0 + 1, ncol = (x1 - x0 + 1) * ny;
+          for (int col0 = 0; col0 < ncol; col0 += kCplColumns) {
+            const int nc = min(ncol - col0, kCplColumns);
+            int j0 = 0, len = 0;
+            if (lane < nc) {
+              const int c = col0 + lane;
+              const int k0 = gc.base + ((x0 + c / ny) * gc.dim[1] + y0 + c % ny) * gc.dim[2];
+              j0 = start[k0 + z0];
+              len = start[k0 + z1 + 1] - j0;
+            }
+            WaveEntries E(j0, len);
+            int j = 0;
+            for (int n = E.next(lane, j); n > 0; n = E.next(lane, j)) {
+              // up to 64 spheres into LDS
+              __builtin_amdgcn_wave_barrier();
+              bool there = lane < n;
+              double4 pj;
+              if (there) {
+                pj = S.posh[j];
+                there = (sx | sy | sz) == 0 || demImageExists(R, B, pj, sx, sy, sz);
+              }
+              const unsigned long long m = __ballot(there);
+              if (there) {
+                CplSphere& q = L[__builtin_amdgcn_mbcnt_hi(
+                    (unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u))];
+                const Img im = imagePos(pj, sx, sy, sz, B);
+                const double4 fdj = S.fdrag[j];
+                q.x = im.x;
+                q.y = im.y;
+                q.z = im.z;
+                q.s = S.vhm[j].w / S.fp[j].w;
+                q.fx = fdj.x;
+                q.fy = fdj.y;
+                q.fz = fdj.z;
+                q.c0 = demCell(R, im.x, 0);
+                q.c1 = demCell(R, im.y, 1);
+                q.c2 = demCell(R, im.z, 2);
+              }
+              __builtin_amdgcn_wave_barrier();
+              __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+              // the spheres within reach, then each lane its own ones
+              const int nk = __popcll(m);
+              unsigned long long mine = 0ull;
+              for (int k = 0; k < nk; k++) {
+                const double dx = pa.x - L[k].x, dy = pa.y - L[k].y, dz = pa.z - L[k].z;
+                if (dot3(dx, dy, dz, dx, dy, dz) <= R.skip2) mine |= 1ull << k;
+              }
+              if (!in) mine = 0ull;
+              for (; mine; mine &= mine - 1) {
+                const CplSphere& q = L[__builtin_ctzll(mine)];
+                const double dx = pa.x - q.x, dy = pa.y - q.y, dz = pa.z - q.z;
+                const double l2 = dot3(dx, dy, dz, dx, dy, dz);
+                if (!cellsAccept(R, q.c0 - ca[0], q.c1 - ca[1], q.c2 - ca[2], l2, false)) continue;
+                const double w = wendW(P.wcon, sqrt(l2) * (2.0 / Rc), Rc / 2.0);
+                por += P.porosity_incr * w;
+                const double t = q.s * rdens * w;
+                fd0 -= q.fx * t;
+                fd1 -= q.fy * t;
+                fd2 -= q.fz * t;
+              }
+            }
+          }
+        }
+      }
+    }
+  }
+  if (!act) return;
   S.fdrag[a] = make_double4(fd0, fd1, fd2, 0.0);
   double4 f = S.frc[a];
   f.x += fd0;
@@ -1107,7 +1300,7 @@ __global__ void k_coupling_sph(Store S, int ns, int nd, Grid gc, const int* __re
 // One wavefront per DEM particle: the lanes test the candidates, the accepted
 // ones are compacted and summed on full wavefronts, and the partial sums meet
 // in a fixed butterfly.
-__global__ void __launch_bounds__(256) k_fpi(Store S, int ns, int nd, Grid gs,
+__global__ void __launch_bounds__(256, 4) k_fpi(Store S, int ns, int nd, Grid gs,
                                              const int* __restrict__ start, Box B,
                                              sphdem_params P) {
   __shared__ int lbuf[4][kCompactCap], lcode[4][kCompactCap];
@@ -1125,16 +1318,19 @@ __global__ void __launch_bounds__(256) k_fpi(Store S, int ns, int nd, Grid gs,
     return dot3(dx, dy, dz, dx, dy, dz);
   };
   auto ranges = [&](auto&& visit) {
-    forCellRanges(gs, start, B, pj.x, pj.y, pj.z, 1, [&](int j0, int j1, int sx, int sy, int sz) {
-      visit(j0, j1, imageCode(sx, sy, sz));
-    });
+    waveCellRanges(gs, start, B, pj.x, pj.y, pj.z, 1, lane, visit);
   };
-  compactedPairs(lbuf[w], lcode[w], lane, ranges, [&](int b, int code) {
+  struct Cand {
+    double4 p;
+    int t;
+  };
+  compactedPairs(lbuf[w], lcode[w], lane, ranges, [&](int b) {
+    return Cand{S.posh[b], S.iam[b]};
+  }, [&](const Cand& c, int, int code) {
     int sx, sy, sz;
     imageShift(code, sx, sy, sz);
-    const double4 pb = S.posh[b];
-    const double lim = 2.0 * dmax2(pj.w, pb.w);
-    return dist2(pb, sx, sy, sz) <= lim * lim && S.iam[b] != T_BOUNDARY;
+    const double lim = 2.0 * dmax2(pj.w, c.p.w);
+    return dist2(c.p, sx, sy, sz) <= lim * lim && c.t != T_BOUNDARY;
   }, [&](int b, int code) {
     int sx, sy, sz;
     imageShift(code, sx, sy, sz);
