@@ -19,6 +19,7 @@
 #include <thread>
 #include <vector>
 
+#include "sphdem_hostcopy.h"
 #include "sphdem_kernels.hip"
 #include "sphdem_tiles.hip"
 #include "sphdem_mixed.hip"
@@ -45,6 +46,7 @@ struct sphdem_ctx {
   sphdem_params P;
   int device = 0;
   hipStream_t stream = nullptr;
+  sphdem::HostCopy hostCopy;  // fields into the caller's memory
   // second stream for passes that run beside the main chain, and its events
   hipStream_t side = nullptr;
   hipEvent_t evFork = nullptr, evJoin = nullptr;
@@ -1389,6 +1391,7 @@ void freeAll(sphdem_ctx* ctx) {
     if (p) (void)hipFree(p);
   for (hipEvent_t e : ctx->evPool) (void)hipEventDestroy(e);
   ctx->evPool.clear();
+  ctx->hostCopy.release();
   if (ctx->hostG) (void)hipHostFree(ctx->hostG);
   ctx->hostG = nullptr;
   if (ctx->gateHost) (void)hipHostFree(ctx->gateHost);
@@ -1456,6 +1459,7 @@ int sphdem_create(const sphdem_params* params, int device, int64_t capacity, sph
     HIPC(hipMalloc(&ctx->dg, sizeof(DevGlobals)));
     HIPC(hipMemset(ctx->dg, 0, sizeof(DevGlobals)));
     HIPC(hipHostMalloc((void**)&ctx->hostG, sizeof(DevGlobals), hipHostMallocDefault));
+    ctx->hostCopy.prepare(sizeof(double) * 3 * (size_t)capacity);
     return 0;
   };
   rc = setup();
@@ -1822,8 +1826,7 @@ int sphdem_get_field(sphdem_ctx* ctx, int field, void* host) {
                        field == SPHDEM_FIELD_IAM ? ctx->cur.iam : ctx->cur.orig,
                        field == SPHDEM_FIELD_IAM ? 0 : 1, ctx->cur.orig, n, buf);
     LAUNCHED();
-    HIPC(hipMemcpyAsync(host, buf, sizeof(int) * n, hipMemcpyDeviceToHost, ctx->stream));
-    HIPC(hipStreamSynchronize(ctx->stream));
+    HIPC(ctx->hostCopy.copy(ctx->device, ctx->stream, host, buf, sizeof(int) * n));
     return 0;
   }
   FieldLoc L;
@@ -1832,9 +1835,8 @@ int sphdem_get_field(sphdem_ctx* ctx, int field, void* host) {
                      (const double*)storeArr(ctx->cur, L.arr), L.off, L.width, ctx->cur.orig, n,
                      ctx->fieldbuf);
   LAUNCHED();
-  HIPC(hipMemcpyAsync(host, ctx->fieldbuf, sizeof(double) * L.width * n, hipMemcpyDeviceToHost,
-                      ctx->stream));
-  HIPC(hipStreamSynchronize(ctx->stream));
+  HIPC(ctx->hostCopy.copy(ctx->device, ctx->stream, host, ctx->fieldbuf,
+                          sizeof(double) * L.width * n));
   return 0;
 }
 
