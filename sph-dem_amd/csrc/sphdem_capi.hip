@@ -62,6 +62,8 @@ struct sphdem_ctx {
   int* pairCnt = nullptr;
   long long* pairOff = nullptr;
   int pairCap = 0;
+  unsigned* found = nullptr;  // a search's pairs, kept between its count and its write
+  int foundCap = 0;
   // segments of the SPH grid (the wavefront work units of the pair passes)
   int *segCnt = nullptr, *segOff = nullptr;
   Segment* segs = nullptr;
@@ -1386,7 +1388,7 @@ void freeAll(sphdem_ctx* ctx) {
                   ctx->mixP,        ctx->mixV,        ctx->mixD,    ctx->okey,
                   ctx->posm,        ctx->pairCnt,     ctx->pairOff, ctx->lrec,
                   ctx->lflag,       ctx->demNear,     ctx->nearGen, ctx->gate,
-                  ctx->keepMem,     ctx->dgKeep,      ctx->hList};
+                  ctx->keepMem,     ctx->dgKeep,      ctx->hList,   ctx->found};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
   for (hipEvent_t e : ctx->evPool) (void)hipEventDestroy(e);
@@ -2643,6 +2645,19 @@ static int getPairs(sphdem_ctx* ctx, int kind, int64_t* count, int32_t* a, int32
     HIPC(hipMalloc(&ctx->pairOff, sizeof(long long) * (cap + 1)));
     ctx->pairCap = cap;
   }
+  // up to 256 MB of kept pairs (their 27 bits of an entry allowing)
+  unsigned* found = nullptr;
+  if (kind != SPHDEM_PAIRS_SPH && nq <= (1 << 19) && ctx->n < (1 << 27)) {
+    if (nq > ctx->foundCap) {
+      if (ctx->found) HIPC(hipFree(ctx->found));
+      ctx->found = nullptr;
+      ctx->foundCap = 0;
+      const int cap = std::min(nq + nq / 4, 1 << 19);
+      HIPC(hipMalloc(&ctx->found, sizeof(unsigned) * kPairsKept * (size_t)cap));
+      ctx->foundCap = cap;
+    }
+    found = ctx->found;
+  }
   long long* off = ctx->pairOff;
   const double half = (ctx->rule.nc + 2) * ctx->rule.e * (1.0 + 1e-6);
   auto enumerate = [&](int mode, int* da, int* db, int* di) -> int {
@@ -2655,7 +2670,7 @@ static int getPairs(sphdem_ctx* ctx, int kind, int64_t* count, int32_t* a, int32
         const int per = TPB / lanes;
         hipLaunchKernelGGL(kernel, dim3((nq + per - 1) / per), dim3(TPB), 0, ctx->stream, ctx->cur,
                            ctx->ns, ctx->nd, kind, ctx->gs, ctx->gc, ctx->start, ctx->box,
-                           ctx->rule, half, mode, ctx->pairCnt, off, da, db, di);
+                           ctx->rule, half, mode, ctx->pairCnt, found, off, da, db, di);
       };
       if (kind == SPHDEM_PAIRS_DEM2SPH)
         launch(k_pairs<64>, 64);

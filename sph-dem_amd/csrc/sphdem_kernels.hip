@@ -2020,14 +2020,20 @@ __global__ void k_cell_coords(Store S, int n, Grid gs, CouplingRule R, int* __re
 // 464-495 and 135-145 us (G = 16: columns of about 25; the narrower range of
 // cells, 49 in place of 343, is part of it), DEM 89-93 and 23 us (G = 16).
 //
+// found (optional): the count keeps a query's first kPairsKept pairs there, and
+// the write copies them: 16, 20 and 3 us in place of the second walk's 145, 46
+// and 23 (the count 135 -> 155, 43 -> 46, 23 -> 25).  A query with more walks again.
+//
 // half (SPH2DEM): no sphere farther than this along an axis is accepted: an
 // accepted image lies within nc sphere cells of edge e, i.e. nc + 1 of them (and
 // one more where the cells around 0 truncate to one).
+constexpr int kPairsKept = 128;
 template <int G>
 __global__ void __launch_bounds__(256) k_pairs(Store S, int ns, int nd, int kind, Grid gs, Grid gc,
                                                const int* __restrict__ start, Box B,
                                                CouplingRule R, double half, int mode,
                                                int* __restrict__ cnt,
+                                               unsigned* __restrict__ found,
                                                const long long* __restrict__ off,
                                                int* __restrict__ oa, int* __restrict__ ob,
                                                int* __restrict__ oimg) {
@@ -2044,6 +2050,16 @@ __global__ void __launch_bounds__(256) k_pairs(Store S, int ns, int nd, int kind
   const int oaId = S.orig[a];
   const int ca[3] = {demCell(R, pa.x, 0), demCell(R, pa.y, 1), demCell(R, pa.z, 2)};
   long long w = (mode == 1) ? off[i] : 0;
+  unsigned* const keep = found ? found + (size_t)i * kPairsKept : nullptr;
+  if (mode == 1 && found && cnt[i] <= kPairsKept) {  // the count pass kept them all
+    for (int k = gl, n = cnt[i]; k < n; k += G) {
+      const unsigned f = keep[k];
+      oa[w + k] = oaId;
+      ob[w + k] = S.orig[f & 0x7ffffff];
+      oimg[w + k] = (int)(f >> 27);
+    }
+    return;
+  }
   auto accept = [&](int b, int sx, int sy, int sz) {
     if (b == a && (sx | sy | sz) == 0) return false;
     const double4 pb = S.posh[b];
@@ -2062,8 +2078,10 @@ __global__ void __launch_bounds__(256) k_pairs(Store S, int ns, int nd, int kind
       const bool ok = b < j1 && accept(b, sx, sy, sz);
       unsigned long long m = __ballot(ok);
       if (G < 64) m = (m >> (threadIdx.x & 63 & ~(G - 1))) & ((1ull << (G & 63)) - 1);
+      const long long at = w + __popcll(m & ((1ull << gl) - 1));
+      if (mode == 0 && ok && keep && at < kPairsKept)
+        keep[at] = (unsigned)b | (unsigned)imageCode(sx, sy, sz) << 27;
       if (mode == 1 && ok) {
-        const long long at = w + __popcll(m & ((1ull << gl) - 1));
         oa[at] = oaId;
         ob[at] = S.orig[b];
         oimg[at] = imageCode(sx, sy, sz);

@@ -57,3 +57,18 @@ def test_spheres_in_a_corner_across_the_periodic_faces():
     p[:, :2] = np.mod(p[:, :2], L[:2])
     c.r[dem] = lo + p
     same_sets(c)
+
+
+@pytest.mark.parametrize("n_dem", [120, 128, 129, 300])
+def test_queries_with_more_pairs_than_the_count_keeps(n_dem):
+    """All spheres within a coupling radius of one fluid particle: queries with
+    fewer pairs than the 128 the count keeps, that many, and more."""
+    c = sd.sediment_case(nf=12, n_dem=n_dem, seed=4)
+    dem = np.flatnonzero(c.iam == sd.DEM)
+    rng = np.random.default_rng(n_dem)
+    c.r[dem] = np.array([0.5, 0.5, 0.5]) + rng.normal(scale=0.01, size=(n_dem, 3))
+    sim = sd.Sim(c)
+    most = max(np.unique(np.asarray(sim.pairs(sd.PAIRS_SPH2DEM))[:, 0], return_counts=True)[1])
+    assert most == n_dem
+    sim.close()
+    same_sets(c)
