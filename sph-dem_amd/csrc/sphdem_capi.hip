@@ -1239,7 +1239,16 @@ int stepStart(sphdem_ctx* ctx, uint32_t bodyMask = 0, const double* accel = null
   }
   if (reinitDue(ctx, ctx->sphStep)) {
     CHECK(doReset(ctx));
-    for (int i = 0; i < 10; i++) CHECK(passDensity(ctx));
+    CHECK(passDensity(ctx));
+    if (mixed(ctx) && ctx->ns > 0) {  // the P records of that pass hold: only h has changed since
+      hipLaunchKernelGGL(k_reinit_m, dim3(blocks(ctx->ns)), dim3(TPB), 0, ctx->stream, ctx->cur,
+                         ctx->ns, ctx->nbl, ctx->nbcnt, ctx->mixP, ctx->mixRes, ctx->P.wcon,
+                         ctx->P.hfac, 9);
+      LAUNCHED();
+      markStale(ctx, GS_POSH | GS_DPO);
+    } else {
+      for (int i = 1; i < 10; i++) CHECK(passDensity(ctx));
+    }
   }
   return 0;
 }

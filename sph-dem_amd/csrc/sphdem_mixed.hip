@@ -138,6 +138,93 @@ __global__ void __launch_bounds__(256) k_density_m(Store S, int ns, const int* _
   S.dpo[a].x = rho;
 }
 
+// A re-initialisation's further iterations (sphIncompress.cpp:29-34) after the
+// first density pass: each sets h from the density and sums it again over the
+// same list, and a particle's sums read of its neighbours only their positions
+// and masses.  So a particle iterates by itself over its distances, kept in
+// registers: kReinitKept of them, of neighbours of one mass (else, or with more,
+// the records are gathered again).
+//
+// What bounds it: the vector arithmetic (13 instructions an entry and
+// iteration); a pass by itself waits for the L1's lines of its gathers.  The 48^3
+// dam break: a pass with its h and packing 65 us, the nine after the first 585;
+// this kernel 135.
+constexpr int kReinitKept = 160;
+__global__ void __launch_bounds__(256) k_reinit_m(Store S, int ns, const int* __restrict__ nbl,
+                                                  const int* __restrict__ nbcnt,
+                                                  const uint4* __restrict__ P, float res,
+                                                  double wcon, double hfac, int iterations) {
+  const int t = xcdThread();
+  const int a = min(t, ns - 1);  // every lane of a wavefront stays
+  const uint4 qa = P[a];
+  const float wc = (float)wcon;
+  const double mass = S.vhm[a].w;
+  const bool sets = isSphT(S.iam[a]);  // h is set from the density
+  double ha = S.posh[a].w, rho = S.dpo[a].x;
+  const int n = t < ns ? nbcnt[a] : 0;
+  int most = n;  // of the wavefront
+  for (int d = 32; d > 0; d >>= 1) most = max(most, __shfl_xor(most, d, 64));
+  most = __builtin_amdgcn_readfirstlane(most);
+  float r[kReinitKept];
+  unsigned m0 = 0u;
+  bool same = true;
+#pragma unroll
+  for (int c = 0; c < kReinitKept; c += 8) {
+#pragma unroll
+    for (int u = 0; u < 8; u++) r[c + u] = 1e30f;  // no entry: no term
+    if (c < most) {
+      const int k0 = c;
+      constexpr int U = 8;
+      SPHDEM_FETCH_ENTRIES(U)
+      uint4 q[U];
+#pragma unroll
+      for (int u = 0; u < U; u++) q[u] = P[e[u]];
+      if (c == 0) m0 = q[0].w;
+#pragma unroll
+      for (int u = 0; u < U; u++) {
+        const float x = fsqrt(dxq(qa, q[u], res).r2);
+        if (c + u < n) {
+          r[c + u] = x;
+          same = same && q[u].w == m0;
+        }
+      }
+    }
+  }
+  const bool kept = __all(same) && most <= kReinitKept;
+  const double mb = (double)__uint_as_float(m0);
+  for (int it = 0; it < iterations; it++) {
+    if (sets) ha = hfac * pow_third(mass / rho);
+    const float rha = (float)(1.0 / ha);
+    const double i3 = 1.0 / cube(ha);
+    rho = mass * (i3 * (double)wendK_m(wc, 0.0f));
+    if (kept) {
+#pragma unroll
+      for (int c = 0; c < kReinitKept; c += 8)
+        if (c < most) {
+#pragma unroll
+          for (int u = 0; u < 8; u++) rho += mb * (i3 * (double)wendK_m(wc, r[c + u] * rha));
+        }
+    } else {
+      constexpr int U = 8;
+      for (int k0 = 0; k0 < n; k0 += U) {
+        SPHDEM_FETCH_ENTRIES(U)
+        uint4 q[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) q[u] = P[e[u]];
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+          if (k0 + u >= n) break;
+          const float qq = fsqrt(dxq(qa, q[u], res).r2) * rha;
+          rho += (double)__uint_as_float(q[u].w) * (i3 * (double)wendK_m(wc, qq));
+        }
+      }
+    }
+  }
+  if (t >= ns) return;
+  if (sets) S.posh[a].w = ha;
+  S.dpo[a].x = rho;
+}
+
 // ---- calcDddtDudt, mixed -----------------------------------------------------------
 // OMG (VAR_H only): calcOmega fused into the walk (the k_omega_m sum, in list
 // order); the dddt terms are summed without 1/omega_a and scaled once in FP64.
