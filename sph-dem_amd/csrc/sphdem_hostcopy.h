@@ -4,8 +4,9 @@
 // What bounds them: the host.  The runtime stages such a copy through pinned
 // memory and moves it on by one thread, which also takes the page faults of
 // memory that was just allocated.  Here the caller's thread and helpers that
-// live for the copy (kWays together) each take every kWays-th piece, with a piece of their
-// own on its way from the device while they copy the one before.  One field,
+// live for the copy (kWays together) each take every kWays-th piece, with a
+// piece of their own on its way from the device while they copy the one before.
+// One field,
 // the runtime's copy and this one: 4.5 MB 288 and 215 us, 9.5 MB 575 and 378,
 // 28 MB 1615 and 960 (29 GB/s; eight threads the same, pieces of 0.5 MB 1330).
 // Threads kept for the context's life save some 20 us a copy.
