@@ -33,7 +33,7 @@ struct HostFields {
   long long sphStep;
   int ng, ns, nd, K, lgen, countsClean, gcntZeroAt;
   unsigned gstale;
-  bool listsValid, listsNear, hKept, segsValid, gridValid, pvFresh, dFresh;
+  bool listsValid, listsNear, hKept, posKept, segsValid, gridValid, pvFresh, dFresh;
   int recFresh;
   double ssr;
   Grid gs, gc;
@@ -90,6 +90,10 @@ struct sphdem_ctx {
   // built, its value then kept in hList
   bool listsNear = false, hKept = false;
   double* hList = nullptr;  // per SPH-group particle
+  // and r and h are about to change from outside a step: both kept in listPos
+  bool posKept = false;
+  double4* listPos = nullptr;
+  int64_t listPosCap = 0;
   // a search's records (recFresh, REC_*) and the mixed form's P and V records
   // (pvFresh) were written by the last reset's permutation and no position,
   // h or vhat changed since
@@ -882,7 +886,7 @@ int doReset(sphdem_ctx* ctx, bool keepSsr = false, bool midInit = false,
   ctx->gstale = 0;  // the permutation copied every ghost from its origin
   std::swap(ctx->cur, ctx->alt);
   std::swap(ctx->storeMem[0], ctx->storeMem[1]);
-  ctx->listsNear = ctx->hKept = false;
+  ctx->listsNear = ctx->hKept = ctx->posKept = false;
   ctx->listsValid = false;  // updateDomain clears every neighbour list (dataLL.cpp:374)
   ctx->recFresh = R.lists;
   ctx->pvFresh = R.mixed != 0;
@@ -898,7 +902,9 @@ int ensureLists(sphdem_ctx* ctx) {
   Timed tm(ctx, KID_LISTS);
   CHECK(refreshGhosts(ctx, GS_POSH));
   const double4* pos = ctx->cur.posh;
-  if (ctx->listsValid && ctx->hKept && ctx->ns > 0) {
+  if (ctx->listsValid && ctx->posKept) {
+    pos = ctx->listPos;
+  } else if (ctx->listsValid && ctx->hKept && ctx->ns > 0) {
     hipLaunchKernelGGL(k_list_pos, dim3(blocks(ctx->ns + ctx->ng)), dim3(TPB), 0, ctx->stream,
                        ctx->cur.posh, ctx->hList, ctx->ns, ctx->n, ctx->ng, ctx->gorig,
                        ctx->alt.posh);
@@ -907,7 +913,26 @@ int ensureLists(sphdem_ctx* ctx) {
   }
   CHECK(launchLists(ctx, pos));
   ctx->listsValid = true;
-  ctx->listsNear = ctx->hKept = false;
+  ctx->listsNear = ctx->hKept = ctx->posKept = false;
+  return 0;
+}
+// Before r or h change from outside a step: what the exact lists in near lists'
+// place are made from, should a caller still ask for them.
+int keepLists(sphdem_ctx* ctx) {
+  if (!ctx->listsNear || ctx->posKept || ctx->ns == 0) return 0;
+  const int64_t need = ctx->cap + ctx->ghostCap;
+  if (need > ctx->listPosCap) {
+    if (ctx->listPos) HIPC(hipFree(ctx->listPos));
+    ctx->listPos = nullptr;
+    ctx->listPosCap = 0;
+    HIPC(hipMalloc(&ctx->listPos, sizeof(double4) * need));
+    ctx->listPosCap = need;
+  }
+  hipLaunchKernelGGL(k_list_pos, dim3(blocks(ctx->ns + ctx->ng)), dim3(TPB), 0, ctx->stream,
+                     ctx->cur.posh, ctx->hKept ? ctx->hList : (const double*)nullptr, ctx->ns,
+                     ctx->n, ctx->ng, ctx->gorig, ctx->listPos);
+  LAUNCHED();
+  ctx->posKept = true;
   return 0;
 }
 // The step's lists, right after a reset.
@@ -1397,7 +1422,8 @@ void freeAll(sphdem_ctx* ctx) {
                   ctx->mixP,        ctx->mixV,        ctx->mixD,    ctx->okey,
                   ctx->posm,        ctx->pairCnt,     ctx->pairOff, ctx->lrec,
                   ctx->lflag,       ctx->demNear,     ctx->nearGen, ctx->gate,
-                  ctx->keepMem,     ctx->dgKeep,      ctx->hList,   ctx->found};
+                  ctx->keepMem,     ctx->dgKeep,      ctx->hList,   ctx->found,
+                  ctx->listPos};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
   for (hipEvent_t e : ctx->evPool) (void)hipEventDestroy(e);
@@ -1736,7 +1762,7 @@ int sphdem_checkpoint_restore(sphdem_ctx* ctx, const void* host, int64_t bytes) 
   ctx->ssr = h.ssr;
   ctx->ng = 0;
   ctx->gridValid = false;
-  ctx->listsValid = ctx->listsNear = ctx->hKept = false;
+  ctx->listsValid = ctx->listsNear = ctx->hKept = ctx->posKept = false;
   ctx->loaded = true;
   // the store is in original-index order: sort it with the saved search
   // radius (the grid of the saved state)
@@ -1869,9 +1895,7 @@ static int setField(sphdem_ctx* ctx, int field, const void* src, bool device) {
   }
   FieldLoc L;
   if (!fieldLoc(field, &L)) return fail(ctx, SPHDEM_E_ARG, "unknown or read-only field %d", field);
-  // near lists hold no value of their own: the exact ones, before r or h change
-  if (ctx->listsNear && (field == SPHDEM_FIELD_R || field == SPHDEM_FIELD_H))
-    CHECK(ensureLists(ctx));
+  if (field == SPHDEM_FIELD_R || field == SPHDEM_FIELD_H) CHECK(keepLists(ctx));
   const double* from = (const double*)src;
   if (!device) {
     HIPC(hipMemcpyAsync(ctx->fieldbuf, src, sizeof(double) * L.width * n, hipMemcpyHostToDevice,
@@ -1937,7 +1961,7 @@ int sphdem_sync(sphdem_ctx* ctx) {
 int sphdem_step_start(sphdem_ctx* ctx) {
   CHECK(checkLoaded(ctx));
   HIPC(hipSetDevice(ctx->device));
-  if (ctx->listsNear) CHECK(ensureLists(ctx));  // before r and h change
+  CHECK(keepLists(ctx));
   CHECK(stepStart(ctx));
   return checkFlags(ctx);
 }
@@ -2058,6 +2082,7 @@ HostFields saveHost(const sphdem_ctx* c) {
   h.listsValid = c->listsValid;
   h.listsNear = c->listsNear;
   h.hKept = c->hKept;
+  h.posKept = c->posKept;
   h.recFresh = c->recFresh;
   h.pvFresh = c->pvFresh;
   h.dFresh = c->dFresh;
@@ -2086,6 +2111,7 @@ void loadHost(sphdem_ctx* c, const HostFields& h) {
   c->listsValid = h.listsValid;
   c->listsNear = h.listsNear;
   c->hKept = h.hKept;
+  c->posKept = h.posKept;
   c->recFresh = h.recFresh;
   c->pvFresh = h.pvFresh;
   c->dFresh = h.dFresh;
@@ -2220,7 +2246,7 @@ int finishReplays(sphdem_ctx* ctx, int count, int* done, bool* stopped) {
                       ctx->stream));
   HIPC(hipMemcpyAsync(ctx->dg, ctx->dgKeep, sizeof(DevGlobals), hipMemcpyDeviceToDevice,
                       ctx->stream));
-  ctx->listsValid = ctx->listsNear = ctx->hKept = false;
+  ctx->listsValid = ctx->listsNear = ctx->hKept = ctx->posKept = false;
   ctx->ng = 0;
   dropGraph(ctx);
   return 0;

@@ -836,9 +836,9 @@ __global__ void __launch_bounds__(64 * W, W == 3 ? 4 : 3)
   }
 }
 
-// Positions with another h (hList, of real entries) for a list search: the
-// SPH-group entries [0, ns) and the ghosts [n, n + ng), whose h is their
-// origin's.
+// Positions with another h (hList, of real entries; null: their own) for a list
+// search: the SPH-group entries [0, ns) and the ghosts [n, n + ng), whose h is
+// their origin's.
 __global__ void k_list_pos(const double4* __restrict__ posh, const double* __restrict__ hList,
                            int ns, int n, int ng, const int* __restrict__ gorig,
                            double4* __restrict__ out) {
@@ -846,7 +846,7 @@ __global__ void k_list_pos(const double4* __restrict__ posh, const double* __res
   if (i >= ns + ng) return;
   const int e = i < ns ? i : n + (i - ns);
   const double4 p = posh[e];
-  out[e] = make_double4(p.x, p.y, p.z, hList[i < ns ? i : gorig[i - ns]]);
+  out[e] = make_double4(p.x, p.y, p.z, hList ? hList[i < ns ? i : gorig[i - ns]] : p.w);
 }
 
 // The cached lists as (a, b, image) triples of original indices, for the

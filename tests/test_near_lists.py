@@ -116,3 +116,31 @@ def test_an_h_of_zero_leaves_every_target_to_the_exact_search(precision):
 @pytest.mark.parametrize("flag", [sd.F_VISC_MONAGHAN, sd.F_VISC_CLEARY])
 def test_the_dt_conditions_take_pairs_only(flag, precision):
     check(viscosity(SIZES["closed17"], flag), spread(0.3), precision)
+
+
+@pytest.mark.parametrize("change", ["r", "h", "both", "start", "h then start"])
+@pytest.mark.parametrize("size", ["periodic13", "closed17"])
+def test_pairs_after_a_step_are_those_of_its_lists(size, change):
+    """r or h set, or a half-step started, after a run: the pairs stay those of the
+    last reset's lists, whichever search made them."""
+    got = []
+    for seg in (64, 0):
+        sim = sd.Sim(SIZES[size]())
+        sim.set_tile_shape(seg, 256)
+        spread(0.2)(sim, np.random.default_rng(3).random)
+        sim.run(2)
+        d = np.random.default_rng(4)
+        if change in ("r", "both"):
+            r = sim.get("r")
+            sim.set("r", r + 1e-3 * (d.random(r.shape) - 0.5))
+        if change in ("h", "both", "h then start"):
+            h = sim.get("h")
+            sim.set("h", h * (0.8 + 0.1 * d.random(h.shape)))
+        if "start" in change:
+            sim.start()
+        p = sim.pairs(sd.PAIRS_SPH)
+        sim.run(1)
+        got.append((p, sim.get("dens"), sim.get("r"), sim.pairs(sd.PAIRS_SPH)))
+        sim.close()
+    for a, b in zip(*got):
+        assert np.array_equal(a, b)
