@@ -1059,7 +1059,8 @@ int computeHinv(sphdem_ctx* ctx) {
 }
 // calcForce instantiated per flag combination (bit 0 VAR_H_CORRECTION, 1 VISC_ARTIFICIAL,
 // 2 LIQ_DEM, bits 3-4 the viscosity variant); OMG: the walkers with calcOmega fused
-// in (VAR_H only: the OMG entries without VAR_H are empty and never selected)
+// in (VAR_H only: the OMG entries without VAR_H are empty and never selected); NEAR:
+// those of near lists
 // The mixed walkers run faster below the occupancy their registers allow
 // (four wavefronts per SIMD): the force walker at two (2.83 against 3.10 ms
 // per launch at 160^3), the dddt walker at three (1.71 against 1.73 ms); their
@@ -1073,26 +1074,27 @@ unsigned walkerLds(const sphdem_ctx* ctx, unsigned waves) {
   return std::min(65536u, (163840u / (blocks + 1u) / 1024u + 1u) * 1024u);
 }
 constexpr unsigned kForceWaves = 2, kDddtWaves = 3;
-template <int F, bool OMG>
+// (near lists are walked by steps only, whose walk sums omega under VAR_H)
+template <int F, bool OMG, bool NEAR>
 void launchForce(sphdem_ctx* ctx) {
   constexpr bool V = (F & 1) != 0, A = (F & 2) != 0, L = (F & 4) != 0;
   constexpr int M = F >> 3;
-  if constexpr (!OMG || V) {
+  if constexpr (OMG ? V : !(NEAR && V)) {
     if (mixed(ctx))
-      hipLaunchKernelGGL((k_force_m<V, M, A, L, OMG>), dim3(walkBlocks(ctx, ctx->ns)), dim3(ctx->walkTPB),
+      hipLaunchKernelGGL((k_force_m<V, M, A, L, OMG, NEAR>), dim3(walkBlocks(ctx, ctx->ns)), dim3(ctx->walkTPB),
                          walkerLds(ctx, kForceWaves),
                          ctx->stream, ctx->cur, ctx->ns, ctx->nbl, ctx->nbcnt, ctx->mixP, ctx->mixV,
                          ctx->mixD, ctx->mixRes, ctx->P, ctx->dg);
     else
-      hipLaunchKernelGGL((k_force_l<V, M, A, L, OMG>), dim3(walkBlocks(ctx, ctx->ns)), dim3(ctx->walkTPB), 0,
+      hipLaunchKernelGGL((k_force_l<V, M, A, L, OMG, NEAR>), dim3(walkBlocks(ctx, ctx->ns)), dim3(ctx->walkTPB), 0,
                          ctx->stream, ctx->cur, ctx->ns, ctx->box, ctx->nbl, ctx->nbcnt, ctx->hinv,
                          ctx->P, ctx->dg);
   }
 }
-template <bool OMG, int... F>
+template <bool OMG, bool NEAR, int... F>
 constexpr std::array<void (*)(sphdem_ctx*), sizeof...(F)> forceTable(
     std::integer_sequence<int, F...>) {
-  return {launchForce<F, OMG>...};
+  return {launchForce<F, OMG, NEAR>...};
 }
 // hinvReady: the 1/h table is already current (made beside the list build);
 // withOmega (VAR_H only): calcOmega summed in the same walk and omega stored --
@@ -1105,15 +1107,19 @@ int passForce(sphdem_ctx* ctx, bool hinvReady = false, bool withOmega = false,
   if (!inStep) CHECK(ensureLists(ctx));
   CHECK(refreshGhosts(ctx, GS_ALL));
   if (!mixed(ctx) && !hinvReady) CHECK(computeHinv(ctx));
-  static constexpr auto table = forceTable<false>(std::make_integer_sequence<int, 32>{});
-  static constexpr auto tableOmega = forceTable<true>(std::make_integer_sequence<int, 32>{});
+  constexpr std::make_integer_sequence<int, 32> flags{};
+  static constexpr std::array<void (*)(sphdem_ctx*), 32> tables[2][2] = {
+      {forceTable<false, false>(flags), forceTable<false, true>(flags)},
+      {forceTable<true, false>(flags), forceTable<true, true>(flags)}};
+  if (ctx->listsNear && varH(ctx) && !withOmega)
+    return fail(ctx, SPHDEM_E_STATE, "near lists are walked with omega in the same walk");
   const uint32_t f = ctx->P.flags;
   const int sel = ((f & SPHDEM_F_VAR_H_CORRECTION) ? 1 : 0) |
                   ((f & SPHDEM_F_VISC_ARTIFICIAL) ? 2 : 0) | ((f & SPHDEM_F_LIQ_DEM) ? 4 : 0) |
                   (viscVariant(f) << 3);
   Timed tm(ctx, KID_FORCE);
   if (mixed(ctx)) CHECK(packMix(ctx, MIX_P | MIX_V | MIX_D));
-  (withOmega ? tableOmega : table)[sel](ctx);
+  tables[withOmega][ctx->listsNear][sel](ctx);
   LAUNCHED();
   if (withOmega) markStale(ctx, GS_DPO);
   return 0;

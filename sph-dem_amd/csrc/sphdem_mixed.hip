@@ -289,7 +289,11 @@ __global__ void __launch_bounds__(256) k_dddt_m(Store S, int ns, const int* __re
 // ---- calcForce, mixed --------------------------------------------------------------
 // OMG (VAR_H only): calcOmega fused into the walk, as in k_dddt_m; the force
 // sums are taken without 1/omega_a and scaled once in FP64.
-template <bool VARH, int VISC, bool ARTIF, bool LIQDEM, bool OMG = false>
+//
+// NEAR: the list is a near list, as in k_force_l.  Its entries that are pairs
+// within the rounding of their FP32 distance ("sure") set their conditions at
+// once; the others are put to the FP64 test where theirs would lower the result.
+template <bool VARH, int VISC, bool ARTIF, bool LIQDEM, bool OMG, bool NEAR>
 __global__ void __launch_bounds__(256) k_force_m(Store S, int ns, const int* __restrict__ nbl,
                                                  const int* __restrict__ nbcnt,
                                                  const uint4* __restrict__ Pq,
@@ -302,11 +306,12 @@ __global__ void __launch_bounds__(256) k_force_m(Store S, int ns, const int* __r
   constexpr bool perPair = ARTIF || VISC == VISC_MON;  // the signal speed is the pair's
   // the least condition so far, by any particle: a bound below which only few
   // pairs lie (an older value serves as well)
-  double newDt = perPair ? __longlong_as_double((long long)g->newDt_bits) : inf;
+  double newDt = NEAR && perPair ? __longlong_as_double((long long)g->newDt_bits) : inf;
   // the dt conditions 0.6 hav and cdiff hav^2 and their rounded values increase
   // with h_b: their minima are those of the smallest h_b over the pairs.  minHb
   // is that of the certain pairs, anyHb of all entries.
   float minHb = __builtin_inff(), anyHb = __builtin_inff();
+  const double vsigC = (VISC == VISC_MOR || VISC == VISC_CLE) ? 2.0 * P.spsound : 0.0;
   if (a < ns) {
     const bool fluid = S.iam[a] == T_SPH;
     const uint4 qa = Pq[a];
@@ -323,7 +328,6 @@ __global__ void __launch_bounds__(256) k_force_m(Store S, int ns, const int* __r
     const float nu = (float)P.viscosity, viscLiq = (float)(2.0 * P.viscosity * P.dens);
     const float cs2 = (float)(2.0 * P.spsound), alpha = (float)P.alpha_artificial;
     const float nu198 = (float)(19.8 * P.viscosity), alphaM = (float)monaghanAlpha(P);
-    const double vsigC = (VISC == VISC_MOR || VISC == VISC_CLE) ? 2.0 * P.spsound : 0.0;
     // certainly a pair of is_neighbr (particle.h:236-238), within 2 ha: the
     // fixed-point positions move r by less than sqrt(3) res, r2 by less than
     // 7 ha res, and FP32 rounding r2 by less than 1e-6 of it
@@ -368,7 +372,7 @@ __global__ void __launch_bounds__(256) k_force_m(Store S, int ns, const int* __r
           const float Gbar = 0.5f * (Ga + Gb);
           const double hav = 0.5 * (ha + (double)v[u].w);
           const float havf = (float)hav;
-          const bool sure = dx.r2 < sure2;
+          const bool sure = !NEAR || dx.r2 < sure2;
           float fvs = 0.0f;  // fv = dv * fvs (Morris)
           float fvr = 0.0f;  // fv = dx * fvr (Cleary, Monaghan)
           float vsig = (float)vsigC;
@@ -407,10 +411,12 @@ __global__ void __launch_bounds__(256) k_force_m(Store S, int ns, const int* __r
           if (perPair) {
             const double lim = 0.6 * hav / (double)vsig;
             newDt = dmin2(newDt, sure ? lim : inf);
-            low = dmin2(low, lim);
-            vs[u] = sure ? 0.0f : vsig;
+            if (NEAR) {
+              low = dmin2(low, lim);
+              vs[u] = sure ? 0.0f : vsig;
+            }
           }
-          anyHb = fminf(anyHb, v[u].w);
+          if (NEAR) anyHb = fminf(anyHb, v[u].w);
           minHb = fminf(minHb, sure ? v[u].w : __builtin_inff());
           constexpr bool alongDr = VISC == VISC_CLE || VISC == VISC_MON;
           const double f0 = (double)(alongDr ? dx.x * fvr : dv0 * fvs);
@@ -426,7 +432,7 @@ __global__ void __launch_bounds__(256) k_force_m(Store S, int ns, const int* __r
         py += q1;
         pz += q2;
       }
-      if (perPair && low < newDt)  // by an entry that may be no pair
+      if (NEAR && perPair && low < newDt)  // by an entry that may be no pair
 #pragma unroll
         for (int u = 0; u < U; u++) {
           const double lim = 0.6 * (0.5 * (ha + (double)v[u].w)) / (double)vs[u];
@@ -464,11 +470,6 @@ __global__ void __launch_bounds__(256) k_force_m(Store S, int ns, const int* __r
     S.fp[a] = fpa;
     S.fv[a] = fva;
   }
-  // a particle whose smallest entry may be no pair and would set the wavefront's
-  // condition: the wavefront goes through its list by the FP64 test, a lane per
-  // entry
-  const int lane = threadIdx.x & 63;
-  const double vsigC = (VISC == VISC_MOR || VISC == VISC_CLE) ? 2.0 * P.spsound : 0.0;
   const double cdiff = VISC == VISC_MON ? 0.06 : 0.125;  // viscDiffusionCondition
   const double ha = a < ns ? S.posh[a].w : 0.0;
   auto lower = [&](float hb) {  // the conditions of the smallest h_b
@@ -478,17 +479,23 @@ __global__ void __launch_bounds__(256) k_force_m(Store S, int ns, const int* __r
     return perPair ? m : dmin2((0.6 * hav) / vsigC, m);
   };
   newDt = dmin2(newDt, lower(minHb));
-  const double sureDt = waveMin(newDt), lowDt = lower(anyHb);
-  for (unsigned long long todo = __ballot(lowDt < sureDt); todo; todo &= todo - 1) {
-    const int s = __builtin_ctzll(todo), as = __builtin_amdgcn_readlane(a, s);
-    const double4 pa = S.posh[as];
-    double x = inf;
-    for (int k = lane, n = nbcnt[as]; k < n; k += 64) {
-      const int j = nbl[nbEntry(k, as, ns)];
-      if (pairWithin(pa, S.posh[j])) x = dmin2(x, (double)V[j].w);
+  if (NEAR) {
+    // a particle whose smallest entry may be no pair and would set the
+    // wavefront's condition: the wavefront goes through its list by the FP64
+    // test, a lane per entry
+    const int lane = threadIdx.x & 63;
+    const double sureDt = waveMin(newDt), lowDt = lower(anyHb);
+    for (unsigned long long todo = __ballot(lowDt < sureDt); todo; todo &= todo - 1) {
+      const int s = __builtin_ctzll(todo), as = __builtin_amdgcn_readlane(a, s);
+      const double4 pa = S.posh[as];
+      double x = inf;
+      for (int k = lane, n = nbcnt[as]; k < n; k += 64) {
+        const int j = nbl[nbEntry(k, as, ns)];
+        if (pairWithin(pa, S.posh[j])) x = dmin2(x, (double)V[j].w);
+      }
+      x = waveMin(x);
+      if (lane == s) newDt = dmin2(newDt, lower((float)x));
     }
-    x = waveMin(x);
-    if (lane == s) newDt = dmin2(newDt, lower((float)x));
   }
   atomicMinPos(&g->newDt_bits, newDt);
 }

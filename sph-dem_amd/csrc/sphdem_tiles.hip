@@ -1054,7 +1054,11 @@ __device__ __forceinline__ bool pairWithin(const double4& pa, const double4& pb)
 // arithmetic (VISC: the viscosity variant, VISC_NONE..VISC_MON).  The per-pair
 // dt conditions (sph.h:545-560) are min-reduced into newDt_bits: those of the
 // artificial and Monaghan viscosities pair by pair, the others, whose signal
-// speed is constant, through the smallest neighbour h.
+// speed is constant, through the smallest numerators.
+//
+// NEAR: the list is a near list, whose entries beyond the radius set no
+// condition.  An exact list's pairs all set theirs, as calcForce over the cached
+// neighbours does, also where r or h has changed since the list was made.
 //
 // OMG (VAR_H only): calcOmega fused into the same walk.  Under VAR_H every
 // force term of a is linear in 1/omega_a and in nothing else of omega
@@ -1062,7 +1066,7 @@ __device__ __forceinline__ bool pairWithin(const double4& pa, const double4& pb)
 // so the walk sums the omega terms (in list order, as k_omega_l) beside the
 // force terms taken without 1/omega_a, stores omega_a, and adds the force
 // sums times 1/omega_a to the incoming f, fp, fv.
-template <bool VARH, int VISC, bool ARTIF, bool LIQDEM, bool OMG = false>
+template <bool VARH, int VISC, bool ARTIF, bool LIQDEM, bool OMG, bool NEAR>
 __global__ void __launch_bounds__(256) k_force_l(Store S, int ns, Box B,
                                                  const int* __restrict__ nbl,
                                                  const int* __restrict__ nbcnt,
@@ -1090,9 +1094,7 @@ __global__ void __launch_bounds__(256) k_force_l(Store S, int ns, Box B,
     const double vsigC = (VISC == VISC_MOR || VISC == VISC_CLE) ? 2.0 * P.spsound : 0.0;
     const double cdiff = VISC == VISC_MON ? 0.06 : 0.125;  // viscDiffusionCondition
     const double alphaM = monaghanAlpha(P);
-    // 0.6 hav and cdiff hav^2 and their rounded values increase with h_b: their
-    // minima are those of the smallest h_b, formed once at the end
-    double minHb = inf;
+    double minA = inf, minB = inf;  // min over pairs of 0.6 hav and cdiff hav^2
     const double4 zero4 = make_double4(0.0, 0.0, 0.0, 0.0);
     double4 f = OMG ? zero4 : S.frc[a], fpa = OMG ? zero4 : S.fp[a], fva = OMG ? zero4 : S.fv[a];
     const int n = nbcnt[a];
@@ -1127,10 +1129,9 @@ __global__ void __launch_bounds__(256) k_force_l(Store S, int ns, Box B,
           const double dv0 = va.x - v[u].x, dv1 = va.y - v[u].y, dv2 = va.z - v[u].z;
           const double Gbar = 0.5 * (Ga + Gb);  // gradW-bar = dr * Gbar
           const double hav = 0.5 * (ha + hb);
-          // the dt conditions are those of the pairs of is_neighbr
-          // (particle.h:236-238): a near list also holds others
+          // is_neighbr (particle.h:236-238)
           const double lim = 2.0 * dmax2(fabs(ha), fabs(hb));
-          const bool isPair = l2 <= lim * lim;
+          const bool isPair = !NEAR || l2 <= lim * lim;
           double fvs = 0.0;  // fv = dv * fvs (Morris)
           double fvr = 0.0;  // fv = dr * fvr (Cleary, Monaghan: m_b visc gradW-bar)
           double vsig = vsigC;
@@ -1167,8 +1168,11 @@ __global__ void __launch_bounds__(256) k_force_l(Store S, int ns, Box B,
             f.z += sg * dz;
             vsig = dmax2(vsig, avsig);
           }
-          if (ARTIF || VISC == VISC_MON) newDt = dmin2(newDt, isPair ? 0.6 * hav / vsig : inf);
-          minHb = dmin2(minHb, isPair ? hb : inf);
+          if (ARTIF || VISC == VISC_MON)
+            newDt = dmin2(newDt, isPair ? 0.6 * hav / vsig : inf);
+          else
+            minA = dmin2(minA, isPair ? 0.6 * hav : inf);
+          minB = dmin2(minB, isPair ? cdiff * (hav * hav) : inf);
           constexpr bool alongDr = VISC == VISC_CLE || VISC == VISC_MON;
           const double fv0 = alongDr ? dx * fvr : dv0 * fvs;
           const double fv1 = alongDr ? dy * fvr : dv1 * fvs;
@@ -1192,11 +1196,8 @@ __global__ void __launch_bounds__(256) k_force_l(Store S, int ns, Box B,
         f.z += p2;
       }
     }
-    if (minHb != inf) {
-      const double hav = 0.5 * (ha + minHb);
-      if (!ARTIF && VISC != VISC_MON) newDt = dmin2(newDt, 0.6 * hav / vsigC);
-      newDt = dmin2(newDt, cdiff * (hav * hav) / P.viscosity);
-    }
+    if (!ARTIF && VISC != VISC_MON && minA != inf) newDt = dmin2(newDt, minA / vsigC);
+    if (minB != inf) newDt = dmin2(newDt, minB / P.viscosity);
     if (OMG) {
       const double omega = 1 + ha * om / (da.x * 3);
       S.dpo[a].z = omega;
