@@ -1129,37 +1129,37 @@ int passDddt(sphdem_ctx* ctx, bool withOmega = false, bool inStep = false) {
   if (withOmega && !varH(ctx)) return fail(ctx, SPHDEM_E_STATE, "fused omega needs VAR_H");
   if (!inStep) CHECK(ensureLists(ctx));
   CHECK(refreshGhosts(ctx, GS_POSH | GS_VHM));
+  const bool near = ctx->listsNear, omega = varH(ctx) && withOmega;
+  if (near && varH(ctx) && !withOmega)
+    return fail(ctx, SPHDEM_E_STATE, "near lists are walked with omega in the same walk");
+  const dim3 grid(walkBlocks(ctx, ctx->ns)), block(ctx->walkTPB);
   if (mixed(ctx)) {
     Timed tm(ctx, KID_DDDT);
     CHECK(packMix(ctx, MIX_P | MIX_V));
-    if (varH(ctx) && withOmega)
-      hipLaunchKernelGGL((k_dddt_m<true, true>), dim3(walkBlocks(ctx, ctx->ns)), dim3(ctx->walkTPB),
-                         walkerLds(ctx, kDddtWaves),
-                         ctx->stream, ctx->cur, ctx->ns, ctx->nbl, ctx->nbcnt, ctx->mixP, ctx->mixV,
+    auto launch = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, grid, block, omega ? walkerLds(ctx, kDddtWaves) : 0u, ctx->stream,
+                         ctx->cur, ctx->ns, ctx->nbl, ctx->nbcnt, ctx->mixP, ctx->mixV,
                          ctx->mixRes, ctx->P.wcon);
+    };
+    if (omega)
+      launch(near ? k_dddt_m<true, true, true> : k_dddt_m<true, true, false>);
     else if (varH(ctx))
-      hipLaunchKernelGGL(k_dddt_m<true>, dim3(walkBlocks(ctx, ctx->ns)), dim3(ctx->walkTPB), 0, ctx->stream,
-                         ctx->cur, ctx->ns, ctx->nbl, ctx->nbcnt, ctx->mixP, ctx->mixV,
-                         ctx->mixRes, ctx->P.wcon);
+      launch(k_dddt_m<true, false, false>);
     else
-      hipLaunchKernelGGL(k_dddt_m<false>, dim3(walkBlocks(ctx, ctx->ns)), dim3(ctx->walkTPB), 0, ctx->stream,
-                         ctx->cur, ctx->ns, ctx->nbl, ctx->nbcnt, ctx->mixP, ctx->mixV,
-                         ctx->mixRes, ctx->P.wcon);
-  } else if (varH(ctx)) {
-    Timed tm(ctx, KID_DDDT);
-    if (withOmega)
-      hipLaunchKernelGGL((k_dddt_l<true, true>), dim3(walkBlocks(ctx, ctx->ns)), dim3(ctx->walkTPB), 0,
-                         ctx->stream, ctx->cur, ctx->ns, ctx->box, ctx->nbl, ctx->nbcnt,
-                         (const double2*)nullptr, ctx->P.wcon);
-    else
-      hipLaunchKernelGGL(k_dddt_l<true>, dim3(walkBlocks(ctx, ctx->ns)), dim3(ctx->walkTPB), 0, ctx->stream, ctx->cur,
-                         ctx->ns, ctx->box, ctx->nbl, ctx->nbcnt, (const double2*)nullptr,
-                         ctx->P.wcon);
+      launch(near ? k_dddt_m<false, false, true> : k_dddt_m<false, false, false>);
   } else {
-    CHECK(computeHinv(ctx));
+    if (!varH(ctx)) CHECK(computeHinv(ctx));
     Timed tm(ctx, KID_DDDT);
-    hipLaunchKernelGGL(k_dddt_l<false>, dim3(walkBlocks(ctx, ctx->ns)), dim3(ctx->walkTPB), 0, ctx->stream, ctx->cur,
-                       ctx->ns, ctx->box, ctx->nbl, ctx->nbcnt, ctx->hinv, ctx->P.wcon);
+    auto launch = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, grid, block, 0, ctx->stream, ctx->cur, ctx->ns, ctx->box, ctx->nbl,
+                         ctx->nbcnt, varH(ctx) ? (const double2*)nullptr : ctx->hinv, ctx->P.wcon);
+    };
+    if (omega)
+      launch(near ? k_dddt_l<true, true, true> : k_dddt_l<true, true, false>);
+    else if (varH(ctx))
+      launch(k_dddt_l<true, false, false>);
+    else
+      launch(near ? k_dddt_l<false, false, true> : k_dddt_l<false, false, false>);
   }
   LAUNCHED();
   if (withOmega) markStale(ctx, GS_DPO);

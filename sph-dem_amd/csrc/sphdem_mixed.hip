@@ -228,15 +228,14 @@ __global__ void __launch_bounds__(256) k_reinit_m(Store S, int ns, const int* __
 // ---- calcDddtDudt, mixed -----------------------------------------------------------
 // OMG (VAR_H only): calcOmega fused into the walk (the k_omega_m sum, in list
 // order); the dddt terms are summed without 1/omega_a and scaled once in FP64.
-template <bool VARH, bool OMG = false>
-__global__ void __launch_bounds__(256) k_dddt_m(Store S, int ns, const int* __restrict__ nbl,
-                                                const int* __restrict__ nbcnt,
-                                                const uint4* __restrict__ P,
-                                                const float4* __restrict__ V, float res,
-                                                double wcon) {
+// NEAR: the list is a near list (true: walk again).  An entry just beyond the
+// radius whose rounded distance falls below 2 h adds less than 1e-20 of a usual
+// pair's term.
+template <bool VARH, bool OMG, bool NEAR>
+__device__ __forceinline__ bool walkDddtM(const Store& S, int a, int ns, int* __restrict__ nbl,
+                                          int* __restrict__ nbcnt, const uint4* __restrict__ P,
+                                          const float4* __restrict__ V, float res, double wcon) {
   static_assert(VARH || !OMG, "omega is only fused under VAR_H");
-  const int a = xcdThread();
-  if (a >= ns) return;
   const uint4 qa = P[a];
   const float4 va = V[a];
   const double ha = S.posh[a].w;
@@ -278,12 +277,24 @@ __global__ void __launch_bounds__(256) k_dddt_m(Store S, int ns, const int* __re
       dddt += (double)__uint_as_float(q[u].w) * (double)(gF * (dv0 * d.x + dv1 * d.y + dv2 * d.z));
     }
   }
+  if (NEAR && walkAgain(dddt + om, S.posh, a, ns, nbl, nbcnt)) return true;
   if (OMG) {
     const double omega = 1 + ha * om / (S.dpo[a].x * 3);
     S.dpo[a].z = omega;
     dddt = S.vh0d[a].w + (1.0 / omega) * dddt;
   }
   S.vh0d[a].w = dddt;
+  return false;
+}
+template <bool VARH, bool OMG, bool NEAR>
+__global__ void __launch_bounds__(256) k_dddt_m(Store S, int ns, int* __restrict__ nbl,
+                                                int* __restrict__ nbcnt,
+                                                const uint4* __restrict__ P,
+                                                const float4* __restrict__ V, float res,
+                                                double wcon) {
+  int a = xcdThread();
+  if (a >= ns) return;
+  while (walkDddtM<VARH, OMG, NEAR>(S, a, ns, nbl, nbcnt, P, V, res, wcon)) a = anew(a);
 }
 
 // ---- calcForce, mixed --------------------------------------------------------------
@@ -293,183 +304,200 @@ __global__ void __launch_bounds__(256) k_dddt_m(Store S, int ns, const int* __re
 // NEAR: the list is a near list, as in k_force_l.  Its entries that are pairs
 // within the rounding of their FP32 distance ("sure") set their conditions at
 // once; the others are put to the FP64 test where theirs would lower the result.
+//
+// The dt conditions 0.6 hav and cdiff hav^2 and their rounded values increase
+// with h_b: their minima are those of the smallest h_b over the pairs.  minHb is
+// that of the certain pairs, anyHb of all entries.
 template <bool VARH, int VISC, bool ARTIF, bool LIQDEM, bool OMG, bool NEAR>
-__global__ void __launch_bounds__(256) k_force_m(Store S, int ns, const int* __restrict__ nbl,
-                                                 const int* __restrict__ nbcnt,
+__device__ __forceinline__ bool walkForceM(const Store& S, int a, int ns, int* __restrict__ nbl,
+                                           int* __restrict__ nbcnt, const uint4* __restrict__ Pq,
+                                           const float4* __restrict__ V,
+                                           const float4* __restrict__ D, float res,
+                                           const sphdem_params& P, double vsigC, double& newDt,
+                                           float& minHb, float& anyHb) {
+  static_assert(VARH || !OMG, "omega is only fused under VAR_H");
+  const double inf = __longlong_as_double(0x7ff0000000000000ll);
+  constexpr bool perPair = ARTIF || VISC == VISC_MON;  // the signal speed is the pair's
+  const bool fluid = S.iam[a] == T_SPH;
+  const uint4 qa = Pq[a];
+  const float4 va = V[a];
+  const double4 da = S.dpo[a];
+  const double ha = S.posh[a].w;
+  const float wc10 = (float)(10.0 * P.wcon);
+  const float rha = (float)(1.0 / ha), i5a = (float)(1.0 / pow5(ha));
+  const float rom = (VARH && !OMG) ? (float)(1.0 / da.z) : 1.0f;
+  const float wc = (float)P.wcon;
+  const float i3 = OMG ? (float)(1.0 / cube(ha)) : 0.0f, c3 = OMG ? (float)(3.0 / pow4(ha)) : 0.0f;
+  double om = OMG ? S.vhm[a].w * (double)wendPdWh_m(wc, 0.0f, rha, i3, c3) : 0.0;
+  const float rhoa = (float)da.x, pdr2a = (float)da.y;
+  const float nu = (float)P.viscosity, viscLiq = (float)(2.0 * P.viscosity * P.dens);
+  const float cs2 = (float)(2.0 * P.spsound), alpha = (float)P.alpha_artificial;
+  const float nu198 = (float)(19.8 * P.viscosity), alphaM = (float)monaghanAlpha(P);
+  // certainly a pair of is_neighbr (particle.h:236-238), within 2 ha: the
+  // fixed-point positions move r by less than sqrt(3) res, r2 by less than
+  // 7 ha res, and FP32 rounding r2 by less than 1e-6 of it
+  const float haf = fabsf((float)ha), sure2 = haf * (3.99998f * haf - 8.0f * res);
+  // f is the sum of the pressure, viscous and artificial-viscosity parts,
+  // added once at the end
+  double ax = 0.0, ay = 0.0, az = 0.0, px = 0.0, py = 0.0, pz = 0.0, vx = 0.0, vy = 0.0,
+         vz = 0.0;
+  const int n = nbcnt[a];
+  constexpr int U = 8;
+  for (int k0 = 0; k0 < n; k0 += U) {
+    SPHDEM_FETCH_ENTRIES(U)
+    uint4 q[U];
+    float4 v[U], d[U];
+    float vs[U] = {};   // the signal speeds of entries that may be no pairs
+    double low = inf;  // the batch's smallest Courant condition
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      q[u] = Pq[e[u]];
+      v[u] = V[e[u]];
+      d[u] = D[e[u]];
+    }
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      if (k0 + u >= n) break;
+      const DxF dx = dxq(qa, q[u], res);
+      const float mb = __uint_as_float(q[u].w), rhob = d[u].x, pdr2b = d[u].y;
+      const float r = fsqrt(dx.r2);
+      if (OMG) om += (double)mb * (double)wendPdWh_m(wc, r * rha, rha, i3, c3);
+      const float Fa = wendF_m(wc10, r * rha, i5a);
+      const float Fb = wendF_m(wc10, r * d[u].z, d[u].w);
+      // gradients are dx * G; under VAR_H both divide by pa.omega (sph.h:331-332)
+      float Ga, Gb;
+      if (VARH) {
+        Ga = Fa * rom;
+        Gb = Fb * rom;
+      } else {
+        Ga = Gb = 0.5f * (Fa + Fb);
+      }
+      if (fluid) {
+        const float dv0 = va.x - v[u].x, dv1 = va.y - v[u].y, dv2 = va.z - v[u].z;
+        const float Gbar = 0.5f * (Ga + Gb);
+        const double hav = 0.5 * (ha + (double)v[u].w);
+        const float havf = (float)hav;
+        const bool sure = !NEAR || dx.r2 < sure2;
+        float fvs = 0.0f;  // fv = dv * fvs (Morris)
+        float fvr = 0.0f;  // fv = dx * fvr (Cleary, Monaghan)
+        float vsig = (float)vsigC;
+        const float vdr = (ARTIF || VISC == VISC_CLE || VISC == VISC_MON)
+                              ? dx.x * dv0 + dx.y * dv1 + dx.z * dv2
+                              : 0.0f;
+        if (VISC == VISC_MOR) {
+          const float rr = frcp(rhoa * rhob);
+          const float visc = LIQDEM ? viscLiq * rr : nu * (rhoa + rhob) * rr;
+          const float dd = Gbar * dx.r2;  // dot(dx, dx * Gbar)
+          const float den = dx.r2 + 0.01f * (havf * havf);
+          fvs = mb * visc * dd * frcp(den);
+        }
+        if (VISC == VISC_CLE) {
+          const float den = dx.r2 + 0.01f * (havf * havf);
+          fvr = mb * (nu198 * vdr * frcp((rhoa + rhob) * den)) * Gbar;
+        }
+        if (VISC == VISC_MON) {
+          const float viss = r != 0.0f ? vdr * frcp(r) : 0.0f;
+          if (!LIQDEM) vsig = cs2 + 2.0f * fabsf(viss);
+          fvr = mb * (viss * vsig * alphaM * frcp(rhoa + rhob)) * Gbar;
+        }
+        if (ARTIF) {
+          float avsig = 0.0f, avisc = 0.0f;
+          if (vdr < 0.0f) {
+            const float viss = r != 0.0f ? vdr * frcp(r) : 0.0f;
+            avsig = cs2 - 4.0f * viss;
+            avisc = viss * avsig * alpha * frcp(rhoa + rhob);
+          }
+          const float s = mb * avisc * Gbar;
+          ax += (double)(s * dx.x);
+          ay += (double)(s * dx.y);
+          az += (double)(s * dx.z);
+          vsig = fmaxf(vsig, avsig);
+        }
+        if (perPair) {
+          const double lim = 0.6 * hav / (double)vsig;
+          newDt = dmin2(newDt, sure ? lim : inf);
+          if (NEAR) {
+            low = dmin2(low, lim);
+            vs[u] = sure ? 0.0f : vsig;
+          }
+        }
+        if (NEAR) anyHb = fminf(anyHb, v[u].w);
+        minHb = fminf(minHb, sure ? v[u].w : __builtin_inff());
+        constexpr bool alongDr = VISC == VISC_CLE || VISC == VISC_MON;
+        const double f0 = (double)(alongDr ? dx.x * fvr : dv0 * fvs);
+        const double f1 = (double)(alongDr ? dx.y * fvr : dv1 * fvs);
+        const double f2 = (double)(alongDr ? dx.z * fvr : dv2 * fvs);
+        vx += f0;
+        vy += f1;
+        vz += f2;
+      }
+      const float pp = -mb * (pdr2a * Ga + pdr2b * Gb);  // pressure force = dx * pp
+      const double q0 = (double)(pp * dx.x), q1 = (double)(pp * dx.y), q2 = (double)(pp * dx.z);
+      px += q0;
+      py += q1;
+      pz += q2;
+    }
+    if (NEAR && perPair && low < newDt)  // by an entry that may be no pair
+#pragma unroll
+      for (int u = 0; u < U; u++) {
+        const double lim = 0.6 * (0.5 * (ha + (double)v[u].w)) / (double)vs[u];
+        if (vs[u] > 0.0f && lim < newDt &&
+            pairWithin(S.posh[a], S.posh[nbl[nbEntry(k0 + u, a, ns)]]))
+          newDt = lim;
+      }
+  }
+  if (NEAR &&
+      walkAgain(om + ax + ay + az + px + py + pz + vx + vy + vz, S.posh, a, ns, nbl, nbcnt))
+    return true;
+  double fx = px + vx + ax, fy = py + vy + ay, fz = pz + vz + az;
+  if (OMG) {
+    const double omega = 1 + ha * om / (da.x * 3);
+    S.dpo[a].z = omega;
+    const double rw = 1.0 / omega;
+    fx *= rw;
+    fy *= rw;
+    fz *= rw;
+    px *= rw;
+    py *= rw;
+    pz *= rw;
+    vx *= rw;
+    vy *= rw;
+    vz *= rw;
+  }
+  double4 f = S.frc[a], fpa = S.fp[a], fva = S.fv[a];
+  f.x += fx;
+  f.y += fy;
+  f.z += fz;
+  fpa.x += px;
+  fpa.y += py;
+  fpa.z += pz;
+  fva.x += vx;
+  fva.y += vy;
+  fva.z += vz;
+  S.frc[a] = f;
+  S.fp[a] = fpa;
+  S.fv[a] = fva;
+  return false;
+}
+template <bool VARH, int VISC, bool ARTIF, bool LIQDEM, bool OMG, bool NEAR>
+__global__ void __launch_bounds__(256) k_force_m(Store S, int ns, int* __restrict__ nbl,
+                                                 int* __restrict__ nbcnt,
                                                  const uint4* __restrict__ Pq,
                                                  const float4* __restrict__ V,
                                                  const float4* __restrict__ D, float res,
                                                  sphdem_params P, DevGlobals* g) {
-  static_assert(VARH || !OMG, "omega is only fused under VAR_H");
-  const int a = xcdThread();
+  int a = xcdThread();
   const double inf = __longlong_as_double(0x7ff0000000000000ll);
-  constexpr bool perPair = ARTIF || VISC == VISC_MON;  // the signal speed is the pair's
+  constexpr bool perPair = ARTIF || VISC == VISC_MON;
   // the least condition so far, by any particle: a bound below which only few
   // pairs lie (an older value serves as well)
   double newDt = NEAR && perPair ? __longlong_as_double((long long)g->newDt_bits) : inf;
-  // the dt conditions 0.6 hav and cdiff hav^2 and their rounded values increase
-  // with h_b: their minima are those of the smallest h_b over the pairs.  minHb
-  // is that of the certain pairs, anyHb of all entries.
   float minHb = __builtin_inff(), anyHb = __builtin_inff();
   const double vsigC = (VISC == VISC_MOR || VISC == VISC_CLE) ? 2.0 * P.spsound : 0.0;
-  if (a < ns) {
-    const bool fluid = S.iam[a] == T_SPH;
-    const uint4 qa = Pq[a];
-    const float4 va = V[a];
-    const double4 da = S.dpo[a];
-    const double ha = S.posh[a].w;
-    const float wc10 = (float)(10.0 * P.wcon);
-    const float rha = (float)(1.0 / ha), i5a = (float)(1.0 / pow5(ha));
-    const float rom = (VARH && !OMG) ? (float)(1.0 / da.z) : 1.0f;
-    const float wc = (float)P.wcon;
-    const float i3 = OMG ? (float)(1.0 / cube(ha)) : 0.0f, c3 = OMG ? (float)(3.0 / pow4(ha)) : 0.0f;
-    double om = OMG ? S.vhm[a].w * (double)wendPdWh_m(wc, 0.0f, rha, i3, c3) : 0.0;
-    const float rhoa = (float)da.x, pdr2a = (float)da.y;
-    const float nu = (float)P.viscosity, viscLiq = (float)(2.0 * P.viscosity * P.dens);
-    const float cs2 = (float)(2.0 * P.spsound), alpha = (float)P.alpha_artificial;
-    const float nu198 = (float)(19.8 * P.viscosity), alphaM = (float)monaghanAlpha(P);
-    // certainly a pair of is_neighbr (particle.h:236-238), within 2 ha: the
-    // fixed-point positions move r by less than sqrt(3) res, r2 by less than
-    // 7 ha res, and FP32 rounding r2 by less than 1e-6 of it
-    const float haf = fabsf((float)ha), sure2 = haf * (3.99998f * haf - 8.0f * res);
-    // f is the sum of the pressure, viscous and artificial-viscosity parts,
-    // added once at the end
-    double ax = 0.0, ay = 0.0, az = 0.0, px = 0.0, py = 0.0, pz = 0.0, vx = 0.0, vy = 0.0,
-           vz = 0.0;
-    const int n = nbcnt[a];
-    constexpr int U = 8;
-    for (int k0 = 0; k0 < n; k0 += U) {
-      SPHDEM_FETCH_ENTRIES(U)
-      uint4 q[U];
-      float4 v[U], d[U];
-      float vs[U] = {};   // the signal speeds of entries that may be no pairs
-      double low = inf;  // the batch's smallest Courant condition
-#pragma unroll
-      for (int u = 0; u < U; u++) {
-        q[u] = Pq[e[u]];
-        v[u] = V[e[u]];
-        d[u] = D[e[u]];
-      }
-#pragma unroll
-      for (int u = 0; u < U; u++) {
-        if (k0 + u >= n) break;
-        const DxF dx = dxq(qa, q[u], res);
-        const float mb = __uint_as_float(q[u].w), rhob = d[u].x, pdr2b = d[u].y;
-        const float r = fsqrt(dx.r2);
-        if (OMG) om += (double)mb * (double)wendPdWh_m(wc, r * rha, rha, i3, c3);
-        const float Fa = wendF_m(wc10, r * rha, i5a);
-        const float Fb = wendF_m(wc10, r * d[u].z, d[u].w);
-        // gradients are dx * G; under VAR_H both divide by pa.omega (sph.h:331-332)
-        float Ga, Gb;
-        if (VARH) {
-          Ga = Fa * rom;
-          Gb = Fb * rom;
-        } else {
-          Ga = Gb = 0.5f * (Fa + Fb);
-        }
-        if (fluid) {
-          const float dv0 = va.x - v[u].x, dv1 = va.y - v[u].y, dv2 = va.z - v[u].z;
-          const float Gbar = 0.5f * (Ga + Gb);
-          const double hav = 0.5 * (ha + (double)v[u].w);
-          const float havf = (float)hav;
-          const bool sure = !NEAR || dx.r2 < sure2;
-          float fvs = 0.0f;  // fv = dv * fvs (Morris)
-          float fvr = 0.0f;  // fv = dx * fvr (Cleary, Monaghan)
-          float vsig = (float)vsigC;
-          const float vdr = (ARTIF || VISC == VISC_CLE || VISC == VISC_MON)
-                                ? dx.x * dv0 + dx.y * dv1 + dx.z * dv2
-                                : 0.0f;
-          if (VISC == VISC_MOR) {
-            const float rr = frcp(rhoa * rhob);
-            const float visc = LIQDEM ? viscLiq * rr : nu * (rhoa + rhob) * rr;
-            const float dd = Gbar * dx.r2;  // dot(dx, dx * Gbar)
-            const float den = dx.r2 + 0.01f * (havf * havf);
-            fvs = mb * visc * dd * frcp(den);
-          }
-          if (VISC == VISC_CLE) {
-            const float den = dx.r2 + 0.01f * (havf * havf);
-            fvr = mb * (nu198 * vdr * frcp((rhoa + rhob) * den)) * Gbar;
-          }
-          if (VISC == VISC_MON) {
-            const float viss = r != 0.0f ? vdr * frcp(r) : 0.0f;
-            if (!LIQDEM) vsig = cs2 + 2.0f * fabsf(viss);
-            fvr = mb * (viss * vsig * alphaM * frcp(rhoa + rhob)) * Gbar;
-          }
-          if (ARTIF) {
-            float avsig = 0.0f, avisc = 0.0f;
-            if (vdr < 0.0f) {
-              const float viss = r != 0.0f ? vdr * frcp(r) : 0.0f;
-              avsig = cs2 - 4.0f * viss;
-              avisc = viss * avsig * alpha * frcp(rhoa + rhob);
-            }
-            const float s = mb * avisc * Gbar;
-            ax += (double)(s * dx.x);
-            ay += (double)(s * dx.y);
-            az += (double)(s * dx.z);
-            vsig = fmaxf(vsig, avsig);
-          }
-          if (perPair) {
-            const double lim = 0.6 * hav / (double)vsig;
-            newDt = dmin2(newDt, sure ? lim : inf);
-            if (NEAR) {
-              low = dmin2(low, lim);
-              vs[u] = sure ? 0.0f : vsig;
-            }
-          }
-          if (NEAR) anyHb = fminf(anyHb, v[u].w);
-          minHb = fminf(minHb, sure ? v[u].w : __builtin_inff());
-          constexpr bool alongDr = VISC == VISC_CLE || VISC == VISC_MON;
-          const double f0 = (double)(alongDr ? dx.x * fvr : dv0 * fvs);
-          const double f1 = (double)(alongDr ? dx.y * fvr : dv1 * fvs);
-          const double f2 = (double)(alongDr ? dx.z * fvr : dv2 * fvs);
-          vx += f0;
-          vy += f1;
-          vz += f2;
-        }
-        const float pp = -mb * (pdr2a * Ga + pdr2b * Gb);  // pressure force = dx * pp
-        const double q0 = (double)(pp * dx.x), q1 = (double)(pp * dx.y), q2 = (double)(pp * dx.z);
-        px += q0;
-        py += q1;
-        pz += q2;
-      }
-      if (NEAR && perPair && low < newDt)  // by an entry that may be no pair
-#pragma unroll
-        for (int u = 0; u < U; u++) {
-          const double lim = 0.6 * (0.5 * (ha + (double)v[u].w)) / (double)vs[u];
-          if (vs[u] > 0.0f && lim < newDt &&
-              pairWithin(S.posh[a], S.posh[nbl[nbEntry(k0 + u, a, ns)]]))
-            newDt = lim;
-        }
-    }
-    double fx = px + vx + ax, fy = py + vy + ay, fz = pz + vz + az;
-    if (OMG) {
-      const double omega = 1 + ha * om / (da.x * 3);
-      S.dpo[a].z = omega;
-      const double rw = 1.0 / omega;
-      fx *= rw;
-      fy *= rw;
-      fz *= rw;
-      px *= rw;
-      py *= rw;
-      pz *= rw;
-      vx *= rw;
-      vy *= rw;
-      vz *= rw;
-    }
-    double4 f = S.frc[a], fpa = S.fp[a], fva = S.fv[a];
-    f.x += fx;
-    f.y += fy;
-    f.z += fz;
-    fpa.x += px;
-    fpa.y += py;
-    fpa.z += pz;
-    fva.x += vx;
-    fva.y += vy;
-    fva.z += vz;
-    S.frc[a] = f;
-    S.fp[a] = fpa;
-    S.fv[a] = fva;
-  }
+  if (a < ns)
+    while (walkForceM<VARH, VISC, ARTIF, LIQDEM, OMG, NEAR>(S, a, ns, nbl, nbcnt, Pq, V, D, res, P,
+                                                            vsigC, newDt, minHb, anyHb))
+      a = anew(a);
   const double cdiff = VISC == VISC_MON ? 0.06 : 0.125;  // viscDiffusionCondition
   const double ha = a < ns ? S.posh[a].w : 0.0;
   auto lower = [&](float hb) {  // the conditions of the smallest h_b

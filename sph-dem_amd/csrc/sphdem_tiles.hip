@@ -444,10 +444,12 @@ __global__ void __launch_bounds__(256) k_lists_t(const double4* __restrict__ pos
 
 // ---- near lists: the step's own search -----------------------------------------------
 // A superset of the lists above for the step's pair walks, in the same order:
-// every SPH neighbour within 2 max(h) and a few just beyond, whose kernel
-// terms are exactly zero (the walks take the pairs of the dt conditions by the
-// FP64 test).  So no candidate needs the FP64 test here, and the distance
-// tests run on the matrix cores.
+// every SPH neighbour within 2 max(h) and some beyond (just beyond where all h
+// are equal, up to sqrt(T_a + T_b - T_0) below where they differ), whose kernel
+// terms are zero in FP64.  The walks take the pairs of the dt conditions by the
+// FP64 test, and leave the others out where their values are not finite
+// (walkAgain).  So no candidate needs the FP64 test here, and the distance tests
+// run on the matrix cores.
 //
 // A workgroup takes a tile of 64 consecutive targets of the cell-sorted store,
 // lane l of every wavefront owning target l.  Its W = 3 wavefronts take the
@@ -979,19 +981,48 @@ __global__ void __launch_bounds__(256) k_density_l(Store S, int ns, Box B,
     S.dpo[a].x = rho;
 }
 
+// is_neighbr (particle.h:236-238) of two entries
+__device__ __forceinline__ bool pairWithin(const double4& pa, const double4& pb) {
+  const double x = pa.x - pb.x, y = pa.y - pb.y, z = pa.z - pb.z;
+  const double l = 2.0 * dmax2(fabs(pa.w), fabs(pb.w));
+  return dot3(x, y, z, x, y, z) <= l * l;
+}
+// A near list's entries beyond the radius add exact zeros, or, where such an
+// entry's mass, density, pressure or velocity is not finite, NaN.  So a particle
+// whose sums do not come out finite keeps the pairs of its list only and is
+// walked again (walkAgain; the walks below store nothing before).
+__device__ __forceinline__ bool walkAgain(double sums, const double4* posh, int a, int ns,
+                                          int* nbl, int* nbcnt) {
+  if (fabs(sums) < __longlong_as_double(0x7ff0000000000000ll)) return false;
+  const double4 pa = posh[a];
+  const int n = nbcnt[a];
+  int m = 0;
+  for (int k = 0; k < n; k++) {
+    const int j = nbl[nbEntry(k, a, ns)];
+    if (pairWithin(pa, posh[j])) nbl[nbEntry(m++, a, ns)] = j;
+  }
+  if (m == n) return false;
+  nbcnt[a] = m;
+  return true;
+}
+// a, as a value the compiler knows nothing of: a second walk reads its particle
+// afresh, and the first keeps no registers for it.
+__device__ __forceinline__ int anew(int a) {
+  asm volatile("" : "+v"(a));
+  return a;
+}
+
 // ---- calcDddtDudt (sphIncompress.h:783-851) over the cached list ----------------
 // OMG (VAR_H only): calcOmega fused into the walk, as in k_force_l -- every
 // dddt term of a is linear in 1/omega_a, so the terms are summed without it
-// beside the omega sum and scaled once.  Three wavefronts per SIMD: 168 VGPRs
-// without spills (170 would allow two), 2 % faster.
-template <bool VARH, bool OMG = false>
-__global__ void __launch_bounds__(256, 3) k_dddt_l(Store S, int ns, Box B,
-                                                const int* __restrict__ nbl,
-                                                const int* __restrict__ nbcnt,
-                                                const double2* __restrict__ hinv, double wcon) {
+// beside the omega sum and scaled once.  NEAR: the list is a near list (true:
+// walk again).  Three wavefronts per SIMD: 168 VGPRs without spills (170 would
+// allow two), 2 % faster.
+template <bool VARH, bool OMG, bool NEAR>
+__device__ __forceinline__ bool walkDddt(const Store& S, int a, int ns, int* __restrict__ nbl,
+                                         int* __restrict__ nbcnt,
+                                         const double2* __restrict__ hinv, double wcon) {
   static_assert(VARH || !OMG, "omega is only fused under VAR_H");
-  const int a = xcdThread();
-  if (a >= ns) return;
   const double4 pa = S.posh[a];
   const double4 va = S.vhm[a];
   const double ha = pa.w;
@@ -1035,20 +1066,24 @@ __global__ void __launch_bounds__(256, 3) k_dddt_l(Store S, int ns, Box B,
       dddt += v[u].w * (dot3(dv0, dv1, dv2, dx, dy, dz) * G);
     }
   }
+  if (NEAR && walkAgain(dddt + om, S.posh, a, ns, nbl, nbcnt)) return true;
   if (OMG) {
     const double omega = 1 + ha * om / (S.dpo[a].x * 3);
     S.dpo[a].z = omega;
     dddt = S.vh0d[a].w + (1.0 / omega) * dddt;
   }
   S.vh0d[a].w = dddt;
+  return false;
+}
+template <bool VARH, bool OMG, bool NEAR>
+__global__ void __launch_bounds__(256, 3) k_dddt_l(Store S, int ns, Box B, int* __restrict__ nbl,
+                                                   int* __restrict__ nbcnt,
+                                                   const double2* __restrict__ hinv, double wcon) {
+  int a = xcdThread();
+  if (a >= ns) return;
+  while (walkDddt<VARH, OMG, NEAR>(S, a, ns, nbl, nbcnt, hinv, wcon)) a = anew(a);
 }
 
-// is_neighbr (particle.h:236-238) of two entries
-__device__ __forceinline__ bool pairWithin(const double4& pa, const double4& pb) {
-  const double x = pa.x - pb.x, y = pa.y - pb.y, z = pa.z - pb.z;
-  const double l = 2.0 * dmax2(fabs(pa.w), fabs(pb.w));
-  return dot3(x, y, z, x, y, z) <= l * l;
-}
 // ---- calcForce (sphIncompress.h:899-972; sph.h:579-666, 692-734) over the list --
 // One instantiation per combination of the flags that change the pair
 // arithmetic (VISC: the viscosity variant, VISC_NONE..VISC_MON).  The per-pair
@@ -1057,8 +1092,9 @@ __device__ __forceinline__ bool pairWithin(const double4& pa, const double4& pb)
 // speed is constant, through the smallest numerators.
 //
 // NEAR: the list is a near list, whose entries beyond the radius set no
-// condition.  An exact list's pairs all set theirs, as calcForce over the cached
-// neighbours does, also where r or h has changed since the list was made.
+// condition (true: walk again).  An exact list's pairs all set theirs, as
+// calcForce over the cached neighbours does, also where r or h has changed since
+// the list was made.
 //
 // OMG (VAR_H only): calcOmega fused into the same walk.  Under VAR_H every
 // force term of a is linear in 1/omega_a and in nothing else of omega
@@ -1067,150 +1103,160 @@ __device__ __forceinline__ bool pairWithin(const double4& pa, const double4& pb)
 // force terms taken without 1/omega_a, stores omega_a, and adds the force
 // sums times 1/omega_a to the incoming f, fp, fv.
 template <bool VARH, int VISC, bool ARTIF, bool LIQDEM, bool OMG, bool NEAR>
-__global__ void __launch_bounds__(256) k_force_l(Store S, int ns, Box B,
-                                                 const int* __restrict__ nbl,
-                                                 const int* __restrict__ nbcnt,
+__device__ __forceinline__ bool walkForce(const Store& S, int a, int ns, int* __restrict__ nbl,
+                                          int* __restrict__ nbcnt,
+                                          const double2* __restrict__ hinv, const sphdem_params& P,
+                                          double& newDt) {
+  static_assert(VARH || !OMG, "omega is only fused under VAR_H");
+  const double inf = __longlong_as_double(0x7ff0000000000000ll);
+  const bool fluid = S.iam[a] == T_SPH;  // viscosity only acts on sph (sphIncompress.h:927)
+  const double4 pa = S.posh[a];
+  const double4 va = S.vhm[a];
+  const double4 da = S.dpo[a];
+  const double ha = pa.w;
+  const double rha = 1.0 / ha;
+  const double rom = (VARH && !OMG) ? 1.0 / da.z : 1.0;
+  const double i3 = OMG ? 1.0 / cube(ha) : 0.0, c3 = OMG ? 3.0 / pow4(ha) : 0.0;
+  double om = OMG ? va.w * wendPdWhi(P.wcon, 0, ha, rha, i3, c3) : 0.0;
+  // gradW = dr * F(q, h) (/ omega_a under VAR_H), F = WCON poly(q) / (q h^5)
+  // = dr * poly(q) * K(h) / r with K(h) = WCON h^-4 (/ omega_a)
+  const double Ka = P.wcon * (rha * rha) * (rha * rha) * rom;
+  const double wrom = P.wcon * rom;
+  const double viscLiq = 2.0 * P.viscosity * P.dens;  // numerator under LIQ_DEM
+  const double vsigC = (VISC == VISC_MOR || VISC == VISC_CLE) ? 2.0 * P.spsound : 0.0;
+  const double cdiff = VISC == VISC_MON ? 0.06 : 0.125;  // viscDiffusionCondition
+  const double alphaM = monaghanAlpha(P);
+  double minA = inf, minB = inf;  // min over pairs of 0.6 hav and cdiff hav^2
+  const double4 zero4 = make_double4(0.0, 0.0, 0.0, 0.0);
+  double4 f = OMG ? zero4 : S.frc[a], fpa = OMG ? zero4 : S.fp[a], fva = OMG ? zero4 : S.fv[a];
+  const int n = nbcnt[a];
+  constexpr int U = 4;
+  for (int k0 = 0; k0 < n; k0 += U) {
+    SPHDEM_FETCH_ENTRIES(U)
+    double4 p[U], v[U];
+    double2 d[U], hi[U];
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const int j = e[u];
+      p[u] = S.posh[j];
+      v[u] = S.vhm[j];
+      d[u] = *reinterpret_cast<const double2*>(&S.dpo[j]);  // dens, pdr2
+      hi[u] = hinv[j];
+    }
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      if (k0 + u >= n) break;
+      const double hb = p[u].w, mb = v[u].w, rhob = d[u].x, pdr2b = d[u].y;
+      const double dx = pa.x - p[u].x, dy = pa.y - p[u].y, dz = pa.z - p[u].z;
+      const double l2 = dot3(dx, dy, dz, dx, dy, dz);
+      const double r = sqrt(l2);
+      const double rinv = r > 0.0 ? 1.0 / r : 0.0;  // r = 0: dr = 0, gradW = 0
+      const double qa = divr(r, ha, rha), qb = divr(r, hb, hi[u].x);
+      if (OMG) om += mb * wendPdWhi(P.wcon, qa, ha, rha, i3, c3);
+      const double Kb = wrom * (hi[u].y * hb);  // WCON hb^-4 (/ omega_a)
+      double Ga = qa <= 2.0 ? wendPoly(qa) * Ka * rinv : 0.0;
+      double Gb = qb <= 2.0 ? wendPoly(qb) * Kb * rinv : 0.0;
+      if (!VARH) Ga = Gb = 0.5 * (Ga + Gb);  // the average gradient
+      if (fluid) {
+        const double dv0 = va.x - v[u].x, dv1 = va.y - v[u].y, dv2 = va.z - v[u].z;
+        const double Gbar = 0.5 * (Ga + Gb);  // gradW-bar = dr * Gbar
+        const double hav = 0.5 * (ha + hb);
+        // is_neighbr (particle.h:236-238)
+        const double lim = 2.0 * dmax2(fabs(ha), fabs(hb));
+        const bool isPair = !NEAR || l2 <= lim * lim;
+        double fvs = 0.0;  // fv = dv * fvs (Morris)
+        double fvr = 0.0;  // fv = dr * fvr (Cleary, Monaghan: m_b visc gradW-bar)
+        double vsig = vsigC;
+        const double vdr = (ARTIF || VISC == VISC_CLE || VISC == VISC_MON)
+                               ? dot3(dx, dy, dz, dv0, dv1, dv2)
+                               : 0.0;
+        if (VISC == VISC_MOR) {
+          const double rab = 1.0 / (da.x * rhob);
+          const double visc = LIQDEM ? viscLiq * rab : P.viscosity * (da.x + rhob) * rab;
+          const double den = l2 + 0.01 * (hav * hav);
+          fvs = mb * visc * (Gbar * l2) / den;  // dr . gradW-bar = Gbar |dr|^2
+        }
+        if (VISC == VISC_CLE) {  // sph.h:598-604
+          const double den = l2 + 0.01 * (hav * hav);
+          const double visc = 19.8 * P.viscosity * vdr / ((da.x + rhob) * den);
+          fvr = mb * visc * Gbar;
+        }
+        if (VISC == VISC_MON) {  // sph.h:606-630, no SLK
+          const double viss = vdr * rinv;
+          if (!LIQDEM) vsig = 2.0 * P.spsound + 2.0 * fabs(viss);
+          const double visc = viss * vsig * alphaM / (da.x + rhob);
+          fvr = mb * visc * Gbar;
+        }
+        if (ARTIF) {
+          double avsig = 0, avisc = 0.0;
+          if (vdr < 0) {
+            const double viss = vdr * rinv;
+            avsig = 2.0 * P.spsound - 4.0 * viss;
+            avisc = viss * avsig * P.alpha_artificial / (da.x + rhob);
+          }
+          const double sg = mb * avisc * Gbar;
+          f.x += sg * dx;
+          f.y += sg * dy;
+          f.z += sg * dz;
+          vsig = dmax2(vsig, avsig);
+        }
+        if (ARTIF || VISC == VISC_MON)
+          newDt = dmin2(newDt, isPair ? 0.6 * hav / vsig : inf);
+        else
+          minA = dmin2(minA, isPair ? 0.6 * hav : inf);
+        minB = dmin2(minB, isPair ? cdiff * (hav * hav) : inf);
+        constexpr bool alongDr = VISC == VISC_CLE || VISC == VISC_MON;
+        const double fv0 = alongDr ? dx * fvr : dv0 * fvs;
+        const double fv1 = alongDr ? dy * fvr : dv1 * fvs;
+        const double fv2 = alongDr ? dz * fvr : dv2 * fvs;
+        fva.x += fv0;
+        fva.y += fv1;
+        fva.z += fv2;
+        f.x += fv0;
+        f.y += fv1;
+        f.z += fv2;
+      }
+      // calcPressForce (sph.h:698-710), antic = 0 under NO_ANTICLUMPING:
+      // -mb (pdr2a gradWa + pdr2b gradWb) = dr * pp
+      const double pp = -mb * (da.y * Ga + pdr2b * Gb);
+      const double p0 = pp * dx, p1 = pp * dy, p2 = pp * dz;
+      fpa.x += p0;
+      fpa.y += p1;
+      fpa.z += p2;
+      f.x += p0;
+      f.y += p1;
+      f.z += p2;
+    }
+  }
+  if (NEAR && walkAgain(om + f.x + f.y + f.z + fpa.x + fpa.y + fpa.z + fva.x + fva.y + fva.z,
+                        S.posh, a, ns, nbl, nbcnt))
+    return true;
+  if (!ARTIF && VISC != VISC_MON && minA != inf) newDt = dmin2(newDt, minA / vsigC);
+  if (minB != inf) newDt = dmin2(newDt, minB / P.viscosity);
+  if (OMG) {
+    const double omega = 1 + ha * om / (da.x * 3);
+    S.dpo[a].z = omega;
+    const double rw = 1.0 / omega;
+    const double4 f0 = S.frc[a], fp0 = S.fp[a], fv0 = S.fv[a];
+    f = make_double4(f0.x + rw * f.x, f0.y + rw * f.y, f0.z + rw * f.z, f0.w);
+    fpa = make_double4(fp0.x + rw * fpa.x, fp0.y + rw * fpa.y, fp0.z + rw * fpa.z, fp0.w);
+    fva = make_double4(fv0.x + rw * fva.x, fv0.y + rw * fva.y, fv0.z + rw * fva.z, fv0.w);
+  }
+  S.frc[a] = f;
+  S.fp[a] = fpa;
+  S.fv[a] = fva;
+  return false;
+}
+template <bool VARH, int VISC, bool ARTIF, bool LIQDEM, bool OMG, bool NEAR>
+__global__ void __launch_bounds__(256) k_force_l(Store S, int ns, Box B, int* __restrict__ nbl,
+                                                 int* __restrict__ nbcnt,
                                                  const double2* __restrict__ hinv,
                                                  sphdem_params P, DevGlobals* g) {
-  static_assert(VARH || !OMG, "omega is only fused under VAR_H");
-  const int a = xcdThread();
-  const double inf = __longlong_as_double(0x7ff0000000000000ll);
-  double newDt = inf;
-  if (a < ns) {
-    const bool fluid = S.iam[a] == T_SPH;  // viscosity only acts on sph (sphIncompress.h:927)
-    const double4 pa = S.posh[a];
-    const double4 va = S.vhm[a];
-    const double4 da = S.dpo[a];
-    const double ha = pa.w;
-    const double rha = 1.0 / ha;
-    const double rom = (VARH && !OMG) ? 1.0 / da.z : 1.0;
-    const double i3 = OMG ? 1.0 / cube(ha) : 0.0, c3 = OMG ? 3.0 / pow4(ha) : 0.0;
-    double om = OMG ? va.w * wendPdWhi(P.wcon, 0, ha, rha, i3, c3) : 0.0;
-    // gradW = dr * F(q, h) (/ omega_a under VAR_H), F = WCON poly(q) / (q h^5)
-    // = dr * poly(q) * K(h) / r with K(h) = WCON h^-4 (/ omega_a)
-    const double Ka = P.wcon * (rha * rha) * (rha * rha) * rom;
-    const double wrom = P.wcon * rom;
-    const double viscLiq = 2.0 * P.viscosity * P.dens;  // numerator under LIQ_DEM
-    const double vsigC = (VISC == VISC_MOR || VISC == VISC_CLE) ? 2.0 * P.spsound : 0.0;
-    const double cdiff = VISC == VISC_MON ? 0.06 : 0.125;  // viscDiffusionCondition
-    const double alphaM = monaghanAlpha(P);
-    double minA = inf, minB = inf;  // min over pairs of 0.6 hav and cdiff hav^2
-    const double4 zero4 = make_double4(0.0, 0.0, 0.0, 0.0);
-    double4 f = OMG ? zero4 : S.frc[a], fpa = OMG ? zero4 : S.fp[a], fva = OMG ? zero4 : S.fv[a];
-    const int n = nbcnt[a];
-    constexpr int U = 4;
-    for (int k0 = 0; k0 < n; k0 += U) {
-      SPHDEM_FETCH_ENTRIES(U)
-      double4 p[U], v[U];
-      double2 d[U], hi[U];
-#pragma unroll
-      for (int u = 0; u < U; u++) {
-        const int j = e[u];
-        p[u] = S.posh[j];
-        v[u] = S.vhm[j];
-        d[u] = *reinterpret_cast<const double2*>(&S.dpo[j]);  // dens, pdr2
-        hi[u] = hinv[j];
-      }
-#pragma unroll
-      for (int u = 0; u < U; u++) {
-        if (k0 + u >= n) break;
-        const double hb = p[u].w, mb = v[u].w, rhob = d[u].x, pdr2b = d[u].y;
-        const double dx = pa.x - p[u].x, dy = pa.y - p[u].y, dz = pa.z - p[u].z;
-        const double l2 = dot3(dx, dy, dz, dx, dy, dz);
-        const double r = sqrt(l2);
-        const double rinv = r > 0.0 ? 1.0 / r : 0.0;  // r = 0: dr = 0, gradW = 0
-        const double qa = divr(r, ha, rha), qb = divr(r, hb, hi[u].x);
-        if (OMG) om += mb * wendPdWhi(P.wcon, qa, ha, rha, i3, c3);
-        const double Kb = wrom * (hi[u].y * hb);  // WCON hb^-4 (/ omega_a)
-        double Ga = qa <= 2.0 ? wendPoly(qa) * Ka * rinv : 0.0;
-        double Gb = qb <= 2.0 ? wendPoly(qb) * Kb * rinv : 0.0;
-        if (!VARH) Ga = Gb = 0.5 * (Ga + Gb);  // the average gradient
-        if (fluid) {
-          const double dv0 = va.x - v[u].x, dv1 = va.y - v[u].y, dv2 = va.z - v[u].z;
-          const double Gbar = 0.5 * (Ga + Gb);  // gradW-bar = dr * Gbar
-          const double hav = 0.5 * (ha + hb);
-          // is_neighbr (particle.h:236-238)
-          const double lim = 2.0 * dmax2(fabs(ha), fabs(hb));
-          const bool isPair = !NEAR || l2 <= lim * lim;
-          double fvs = 0.0;  // fv = dv * fvs (Morris)
-          double fvr = 0.0;  // fv = dr * fvr (Cleary, Monaghan: m_b visc gradW-bar)
-          double vsig = vsigC;
-          const double vdr = (ARTIF || VISC == VISC_CLE || VISC == VISC_MON)
-                                 ? dot3(dx, dy, dz, dv0, dv1, dv2)
-                                 : 0.0;
-          if (VISC == VISC_MOR) {
-            const double rab = 1.0 / (da.x * rhob);
-            const double visc = LIQDEM ? viscLiq * rab : P.viscosity * (da.x + rhob) * rab;
-            const double den = l2 + 0.01 * (hav * hav);
-            fvs = mb * visc * (Gbar * l2) / den;  // dr . gradW-bar = Gbar |dr|^2
-          }
-          if (VISC == VISC_CLE) {  // sph.h:598-604
-            const double den = l2 + 0.01 * (hav * hav);
-            const double visc = 19.8 * P.viscosity * vdr / ((da.x + rhob) * den);
-            fvr = mb * visc * Gbar;
-          }
-          if (VISC == VISC_MON) {  // sph.h:606-630, no SLK
-            const double viss = vdr * rinv;
-            if (!LIQDEM) vsig = 2.0 * P.spsound + 2.0 * fabs(viss);
-            const double visc = viss * vsig * alphaM / (da.x + rhob);
-            fvr = mb * visc * Gbar;
-          }
-          if (ARTIF) {
-            double avsig = 0, avisc = 0.0;
-            if (vdr < 0) {
-              const double viss = vdr * rinv;
-              avsig = 2.0 * P.spsound - 4.0 * viss;
-              avisc = viss * avsig * P.alpha_artificial / (da.x + rhob);
-            }
-            const double sg = mb * avisc * Gbar;
-            f.x += sg * dx;
-            f.y += sg * dy;
-            f.z += sg * dz;
-            vsig = dmax2(vsig, avsig);
-          }
-          if (ARTIF || VISC == VISC_MON)
-            newDt = dmin2(newDt, isPair ? 0.6 * hav / vsig : inf);
-          else
-            minA = dmin2(minA, isPair ? 0.6 * hav : inf);
-          minB = dmin2(minB, isPair ? cdiff * (hav * hav) : inf);
-          constexpr bool alongDr = VISC == VISC_CLE || VISC == VISC_MON;
-          const double fv0 = alongDr ? dx * fvr : dv0 * fvs;
-          const double fv1 = alongDr ? dy * fvr : dv1 * fvs;
-          const double fv2 = alongDr ? dz * fvr : dv2 * fvs;
-          fva.x += fv0;
-          fva.y += fv1;
-          fva.z += fv2;
-          f.x += fv0;
-          f.y += fv1;
-          f.z += fv2;
-        }
-        // calcPressForce (sph.h:698-710), antic = 0 under NO_ANTICLUMPING:
-        // -mb (pdr2a gradWa + pdr2b gradWb) = dr * pp
-        const double pp = -mb * (da.y * Ga + pdr2b * Gb);
-        const double p0 = pp * dx, p1 = pp * dy, p2 = pp * dz;
-        fpa.x += p0;
-        fpa.y += p1;
-        fpa.z += p2;
-        f.x += p0;
-        f.y += p1;
-        f.z += p2;
-      }
-    }
-    if (!ARTIF && VISC != VISC_MON && minA != inf) newDt = dmin2(newDt, minA / vsigC);
-    if (minB != inf) newDt = dmin2(newDt, minB / P.viscosity);
-    if (OMG) {
-      const double omega = 1 + ha * om / (da.x * 3);
-      S.dpo[a].z = omega;
-      const double rw = 1.0 / omega;
-      const double4 f0 = S.frc[a], fp0 = S.fp[a], fv0 = S.fv[a];
-      f = make_double4(f0.x + rw * f.x, f0.y + rw * f.y, f0.z + rw * f.z, f0.w);
-      fpa = make_double4(fp0.x + rw * fpa.x, fp0.y + rw * fpa.y, fp0.z + rw * fpa.z, fp0.w);
-      fva = make_double4(fv0.x + rw * fva.x, fv0.y + rw * fva.y, fv0.z + rw * fva.z, fv0.w);
-    }
-    S.frc[a] = f;
-    S.fp[a] = fpa;
-    S.fv[a] = fva;
-  }
+  int a = xcdThread();
+  double newDt = __longlong_as_double(0x7ff0000000000000ll);
+  if (a < ns)
+    while (walkForce<VARH, VISC, ARTIF, LIQDEM, OMG, NEAR>(S, a, ns, nbl, nbcnt, hinv, P, newDt))
+      a = anew(a);
   atomicMinPos(&g->newDt_bits, newDt);
 }
 
