@@ -10,7 +10,7 @@
 // output adjoints to every differentiable input by the chain rule written out
 // by hand (derivations in the comments).  Sums over pairs go through hardware
 // FP64 atomics on global memory; the parameter adjoints are reduced per block
-// first, so one atomic per block lands on each.
+// first, and those of many blocks by way of partial sums (SumCells).
 //
 // Wendland C2 (3D, support 2h) in the closed forms used below, with q = r/h,
 // t = 2 - q and c = WCON:
@@ -138,10 +138,27 @@ __device__ __forceinline__ void wendW(double c, double r, double h, double& W, d
   }
 }
 
-// Sums NV per-thread values over the block and adds each total to dst[k]
-// with one atomic.  Every thread of the block must call it.
+// Partial sums of one launch's parameter adjoints.  A group of lanes per query
+// makes a block of 256 threads' share small (4 to 16 queries), and thousands of
+// blocks that each round one running total leave 3 to 9 times the error of the
+// few blocks of a thread per query.  So block b adds to cell b % 64 of its
+// launch's own cells, and the last block adds these up: 64 totals of 1/64 the
+// size, each rounded 1/64 as often.  The rms error against the exact sum, in
+// units of its last place, with a thread per query, with all blocks adding to
+// the result, and now: drag_a over 131072 spheres 3.1, 48 and 0.4, over 8192
+// 1.2, 8.2 and 0.3; viscosity (force) over 131072 particles 4.7, 6.0 and below
+// 0.1, over 8192 0.7, 3.8 and below 0.1.
+constexpr int kSumCells = 64;
+struct SumCells {
+  double part[3][kSumCells];
+  unsigned done;  // blocks that have added; zero between launches, as the cells
+};
+
+// Sums NV per-thread values over the block and adds each total to dst[k], by way
+// of the launch's cells if it has any.  Every thread of the block must call it.
 template <int NV>
-__device__ void blockAdd(double (&v)[NV], double* dst) {
+__device__ void blockAdd(double (&v)[NV], double* dst, SumCells* cells = nullptr) {
+  static_assert(NV <= 3, "SumCells holds three sums");
   __shared__ double part[NV][kTPB / 64];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
 #pragma unroll
@@ -151,11 +168,30 @@ __device__ void blockAdd(double (&v)[NV], double* dst) {
     if (lane == 0) part[k][w] = x;
   }
   __syncthreads();
-  if (threadIdx.x < NV) {
+  if (w != 0) return;
+  if (lane < NV) {
     double s = 0.0;
-    for (int j = 0; j < kTPB / 64; j++) s += part[threadIdx.x][j];
-    if (s != 0.0) unsafeAtomicAdd(dst + threadIdx.x, s);
+    for (int j = 0; j < kTPB / 64; j++) s += part[lane][j];
+    double* const to = cells ? &cells->part[lane][blockIdx.x % kSumCells] : dst + lane;
+    if (s != 0.0) unsafeAtomicAdd(to, s);
   }
+  if (!cells) return;
+  // the additions have reached the memory all XCDs share before the count does
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  unsigned before = 0;
+  if (lane == 0)
+    before = __hip_atomic_fetch_add(&cells->done, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if ((unsigned)__builtin_amdgcn_readfirstlane((int)before) != gridDim.x - 1) return;
+#pragma unroll
+  for (int k = 0; k < NV; k++) {
+    double x = __longlong_as_double((long long)__hip_atomic_exchange(
+        (unsigned long long*)&cells->part[k][lane], 0ull, __ATOMIC_RELAXED,
+        __HIP_MEMORY_SCOPE_AGENT));
+    for (int o = 32; o > 0; o >>= 1) x += __shfl_down(x, o, 64);
+    if (lane == 0 && x != 0.0) unsafeAtomicAdd(dst + k, x);
+  }
+  if (lane == 0)
+    __hip_atomic_store(&cells->done, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // ---------------------------------------------------------------- SPH force
@@ -224,7 +260,8 @@ __global__ void __launch_bounds__(kTPB) k_force_bwd(int32_t nq, const int32_t* _
                             const int64_t* __restrict__ off, const int32_t* __restrict__ pb,
                             const int32_t* __restrict__ pimg, sphdem_adj_fields in,
                             sphdem_adj_consts C, const double* __restrict__ gfv,
-                            const double* __restrict__ gfp, sphdem_adj_grads g) {
+                            const double* __restrict__ gfp, sphdem_adj_grads g,
+                            SumCells* cells) {
   const int i = queryIndex<kSphLanes>(), gl = queryLane<kSphLanes>();
   double gnu[1] = {0.0};
   if (i < nq) {
@@ -340,7 +377,7 @@ __global__ void __launch_bounds__(kTPB) k_force_bwd(int32_t nq, const int32_t* _
       g.pdr2[a] += gpa;
     }
   }
-  blockAdd<1>(gnu, g.params);
+  blockAdd<1>(gnu, g.params, cells);
 }
 
 // ---------------------------------------------------------------- omega
@@ -784,7 +821,7 @@ __global__ void __launch_bounds__(kTPB) k_fpi_bwd(int32_t nq, const int32_t* __r
                           const int64_t* __restrict__ off, const int32_t* __restrict__ pb,
                           const int32_t* __restrict__ pimg, sphdem_adj_fields in,
                           sphdem_adj_consts C, const double* __restrict__ gfd,
-                          sphdem_adj_grads g) {
+                          sphdem_adj_grads g, SumCells* cells) {
   const int i = queryIndex<kFpiLanes>(), gl = queryLane<kFpiLanes>();
   __shared__ Add3Stage stage[kTPB / 64];
   double gpar[3] = {0.0, 0.0, 0.0};  // nu, drag_a, drag_b
@@ -900,7 +937,7 @@ __global__ void __launch_bounds__(kTPB) k_fpi_bwd(int32_t nq, const int32_t* __r
     if (gl == 0) add3(g.r, p, rpx, rpy, rpz);
   }
   if (gl != 0) gpar[0] = gpar[1] = gpar[2] = 0.0;  // every lane holds the query's
-  blockAdd<3>(gpar, g.params);
+  blockAdd<3>(gpar, g.params, cells);
 }
 
 // -------------------------------------------------------------- DEM contacts
@@ -1010,6 +1047,106 @@ int scratchOfCurrentDevice(double** out) {
   return 0;
 }
 
+// ---- the launches' partial sums
+// A launch has its SumCells to itself until it has ended (an event after it
+// says so), whatever streams and threads launch beside it; where all are in use
+// it takes those of an earlier launch on its own stream, behind which it runs.
+// A captured launch keeps its cells: it may be replayed at any time (two replays
+// of one captured launch at once would race on its outputs as well).  With none
+// left, or on a device past the kept ones, the blocks add to the result directly.
+constexpr int kSumLaunches = 32, kSumCaptured = 64;
+__device__ sphdem_adj::SumCells sumCells[kSumLaunches + kSumCaptured];
+
+struct SumPool {
+  sphdem_adj::SumCells* base = nullptr;
+  hipEvent_t ended[kSumLaunches] = {};
+  hipStream_t stream[kSumLaunches] = {};  // of its last launch
+  bool taken[kSumLaunches] = {};  // until its event is recorded
+  bool used[kSumLaunches] = {};
+  int next = 0, captured = 0;
+};
+std::mutex g_sumMu;
+SumPool g_sumPool[kScratchDevices];
+
+// The cells of one launch on `stream`: taken here, given back when destroyed,
+// right after the launch.
+class LaunchSums {
+ public:
+  LaunchSums(hipStream_t stream, unsigned blocks) : stream_(stream) {
+    int dev = -1;
+    if (blocks < 2 || hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kScratchDevices) return;
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(stream, &cap) != hipSuccess) {
+      (void)hipGetLastError();
+      return;
+    }
+    std::lock_guard<std::mutex> lock(g_sumMu);
+    SumPool& p = g_sumPool[dev];
+    if (!p.base) {
+      void* q = nullptr;
+      if (hipGetSymbolAddress(&q, HIP_SYMBOL(sumCells)) != hipSuccess) {
+        (void)hipGetLastError();
+        return;
+      }
+      p.base = (sphdem_adj::SumCells*)q;
+    }
+    if (cap != hipStreamCaptureStatusNone) {
+      if (p.captured < kSumCaptured) cells_ = p.base + kSumLaunches + p.captured++;
+      return;
+    }
+    // another thread's capture is none of these calls' concern
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+    for (int i = 0; i < 2 * kSumLaunches && !pool_; i++) {
+      const int k = (p.next + i) % kSumLaunches;
+      if (p.taken[k]) continue;
+      if (i >= kSumLaunches) {  // all in use
+        if (p.stream[k] != stream || hipStreamWaitEvent(stream, p.ended[k], 0) != hipSuccess)
+          continue;
+        take(p, k, stream);
+        break;
+      }
+      if (!p.ended[k] &&
+          hipEventCreateWithFlags(&p.ended[k], hipEventDisableTiming) != hipSuccess) {
+        p.ended[k] = nullptr;
+        (void)hipGetLastError();
+        break;
+      }
+      if (p.used[k] && hipEventQuery(p.ended[k]) != hipSuccess) {
+        (void)hipGetLastError();
+        continue;
+      }
+      take(p, k, stream);
+    }
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+  }
+  ~LaunchSums() {
+    if (!pool_) return;
+    const bool ok = hipEventRecord(pool_->ended[k_], stream_) == hipSuccess;
+    if (!ok) (void)hipGetLastError();  // these cells are not used again
+    std::lock_guard<std::mutex> lock(g_sumMu);
+    pool_->taken[k_] = !ok;
+  }
+  LaunchSums(const LaunchSums&) = delete;
+  LaunchSums& operator=(const LaunchSums&) = delete;
+  sphdem_adj::SumCells* cells() const { return cells_; }
+
+ private:
+  void take(SumPool& p, int k, hipStream_t stream) {
+    p.taken[k] = p.used[k] = true;
+    p.stream[k] = stream;
+    p.next = k + 1;
+    pool_ = &p;
+    k_ = k;
+    cells_ = p.base + k;
+  }
+
+  hipStream_t stream_;
+  SumPool* pool_ = nullptr;
+  int k_ = 0;
+  sphdem_adj::SumCells* cells_ = nullptr;
+};
+
 // zero fill (a kernel, not a memset: the call stays a plain kernel sequence)
 __global__ void __launch_bounds__(sphdem_adj::kTPB) k_zero_doubles(double* __restrict__ p, int64_t n) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -1045,9 +1182,11 @@ int sphdem_adj_force_bwd(int32_t nquery, const int32_t* query, const int64_t* of
   if (!SPHDEM_ADJ_CSR_OK(in) || !in->h || !in->vhat || !in->dens || !in->omega || !in->pdr2 ||
       !in->iam || !g->r || !g->vhat || !g->h || !g->dens || !g->omega || !g->pdr2 || !g->params)
     return SPHDEM_E_ARG;
-  hipLaunchKernelGGL(sphdem_adj::k_force_bwd, dim3(sphdem_adj::gridFor(nquery, sphdem_adj::kSphLanes)),
-                     dim3(sphdem_adj::kTPB), 0, (hipStream_t)stream, nquery, query, off, b, img,
-                     *in, *c, gfv, gfp, *g);
+  const unsigned grid = sphdem_adj::gridFor(nquery, sphdem_adj::kSphLanes);
+  const LaunchSums sums((hipStream_t)stream, grid);
+  hipLaunchKernelGGL(sphdem_adj::k_force_bwd, dim3(grid), dim3(sphdem_adj::kTPB), 0,
+                     (hipStream_t)stream, nquery, query, off, b, img, *in, *c, gfv, gfp, *g,
+                     sums.cells());
   return adjLaunched();
 }
 
@@ -1196,9 +1335,11 @@ int sphdem_adj_fpi_bwd(int32_t nquery, const int32_t* query, const int64_t* off,
       !in->mass || !in->fpfb || !in->fv || !in->por || !g->r || !g->vhat || !g->h ||
       !g->dens || !g->fpfb || !g->fv || !g->por || !g->params)
     return SPHDEM_E_ARG;
-  hipLaunchKernelGGL(sphdem_adj::k_fpi_bwd, dim3(sphdem_adj::gridFor(nquery, sphdem_adj::kFpiLanes)),
-                     dim3(sphdem_adj::kTPB), 0, (hipStream_t)stream, nquery, query, off, b, img,
-                     *in, *c, gfdrag, *g);
+  const unsigned grid = sphdem_adj::gridFor(nquery, sphdem_adj::kFpiLanes);
+  const LaunchSums sums((hipStream_t)stream, grid);
+  hipLaunchKernelGGL(sphdem_adj::k_fpi_bwd, dim3(grid), dim3(sphdem_adj::kTPB), 0,
+                     (hipStream_t)stream, nquery, query, off, b, img, *in, *c, gfdrag, *g,
+                     sums.cells());
   return adjLaunched();
 }
 
