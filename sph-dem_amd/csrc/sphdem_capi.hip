@@ -378,12 +378,11 @@ int ensureKeys(sphdem_ctx* ctx, int K) {
   return 0;
 }
 
-// exclusive scan of in[0..nin), then zeros, into out[0..m) (m <= SCAN_TILE^2);
-// copyLast (device, optional) also receives out[m - 1]
+// exclusive scan of in[0..nin), then zeros, into out[0..m); copyLast (device,
+// optional) also receives out[m - 1]
 template <class T>
 int scanItems(sphdem_ctx* ctx, const int* in, int nin, T* out, int m, T* copyLast = nullptr) {
   const int tiles = (m + SCAN_TILE - 1) / SCAN_TILE;
-  if (tiles > SCAN_TILE) return fail(ctx, SPHDEM_E_CAPACITY, "scan of %d items", m);
   if (tiles + 1 > ctx->tileCap) {
     if (ctx->tiles) HIPC(hipFree(ctx->tiles));
     ctx->tileCap = tiles + 1 + (tiles + 1) / 4;
@@ -401,7 +400,9 @@ int scanItems(sphdem_ctx* ctx, const int* in, int nin, T* out, int m, T* copyLas
   }
   return 0;
 }
+// a reset's counts: at most SCAN_TILE^2 cells or particles with ghosts
 int scanInts(sphdem_ctx* ctx, const int* in, int* out, int m, int* copyLast = nullptr) {
+  if (m > SCAN_TILE * SCAN_TILE) return fail(ctx, SPHDEM_E_CAPACITY, "scan of %d items", m);
   return scanItems<int>(ctx, in, m, out, m, copyLast);
 }
 int scanCounts(sphdem_ctx* ctx, int m) { return scanInts(ctx, ctx->counts, ctx->start, m); }
