@@ -2687,16 +2687,22 @@ static int getPairs(sphdem_ctx* ctx, int kind, int64_t* count, int32_t* a, int32
     HIPC(hipMalloc(&ctx->pairOff, sizeof(long long) * (cap + 1)));
     ctx->pairCap = cap;
   }
-  // up to 256 MB of kept pairs (their 27 bits of an entry allowing)
+  // up to 256 MB of kept pairs (their 27 bits of an entry allowing), where a
+  // write follows the count; without the memory the write searches again
+  const bool write = a && b && image;
   unsigned* found = nullptr;
-  if (kind != SPHDEM_PAIRS_SPH && nq <= (1 << 19) && ctx->n < (1 << 27)) {
+  if (write && kind != SPHDEM_PAIRS_SPH && nq <= (1 << 19) && ctx->n < (1 << 27)) {
     if (nq > ctx->foundCap) {
       if (ctx->found) HIPC(hipFree(ctx->found));
       ctx->found = nullptr;
       ctx->foundCap = 0;
       const int cap = std::min(nq + nq / 4, 1 << 19);
-      HIPC(hipMalloc(&ctx->found, sizeof(unsigned) * kPairsKept * (size_t)cap));
-      ctx->foundCap = cap;
+      if (hipMalloc(&ctx->found, sizeof(unsigned) * kPairsKept * (size_t)cap) == hipSuccess) {
+        ctx->foundCap = cap;
+      } else {
+        (void)hipGetLastError();
+        ctx->found = nullptr;
+      }
     }
     found = ctx->found;
   }
@@ -2729,7 +2735,7 @@ static int getPairs(sphdem_ctx* ctx, int kind, int64_t* count, int32_t* a, int32
   HIPC(hipMemcpyAsync(&tot, off + nq, sizeof(long long), hipMemcpyDeviceToHost, ctx->stream));
   HIPC(hipStreamSynchronize(ctx->stream));
   *count = tot;
-  if (a && b && image && tot > 0) {
+  if (write && tot > 0) {
     if (tot > capacity)
       return fail(ctx, SPHDEM_E_CAPACITY, "pair buffer of %lld < %lld", (long long)capacity, tot);
     int *da = nullptr, *db = nullptr, *di = nullptr;

@@ -1,5 +1,6 @@
-"""Pair searches of more targets than one tile of scanned tiles holds (16,777,216)
-hand out their pairs, as the list build does."""
+"""Pair searches: more targets than one tile of scanned tiles holds (16,777,216)
+hand out their pairs, as the list build does; and a search that only counts takes
+no memory for the pairs."""
 import ctypes
 
 import numpy as np
@@ -43,4 +44,19 @@ def test_more_targets_than_a_tile_of_tiles():
     step = (a - b).abs()
     assert bool(((step == 1) | (step == N) | (step == N * N)).all())
     assert bool((im == 13).all())
+    sim.close()
+
+
+def test_a_count_keeps_no_pairs():
+    """The room for pairs kept between the count and the write (128 a query) is
+    taken by a search that writes."""
+    sim = sd.Sim(sd.sediment_case(nf=32, n_dem=64, seed=1))
+    sim.reset()
+    sim.pair_count(sd.PAIRS_DEM2SPH)
+    torch.cuda.synchronize()
+    kept = 4 * 128 * sim.case.n
+    before = torch.cuda.mem_get_info()[0]
+    cnt = sim.pair_count(sd.PAIRS_SPH2DEM)
+    assert before - torch.cuda.mem_get_info()[0] < kept // 4  # counts and offsets
+    assert len(sim.pairs(sd.PAIRS_SPH2DEM)) == cnt
     sim.close()
