@@ -90,10 +90,9 @@ struct sphdem_ctx {
   // built, its value then kept in hList
   bool listsNear = false, hKept = false;
   double* hList = nullptr;  // per SPH-group particle
-  // and r and h are about to change from outside a step: both kept in listPos
+  // and r and h are about to change from outside a step: both kept in alt.posh
+  // (until the next reset, which writes alt, nothing else does)
   bool posKept = false;
-  double4* listPos = nullptr;
-  int64_t listPosCap = 0;
   // a search's records (recFresh, REC_*) and the mixed form's P and V records
   // (pvFresh) were written by the last reset's permutation and no position,
   // h or vhat changed since
@@ -904,7 +903,7 @@ int ensureLists(sphdem_ctx* ctx) {
   CHECK(refreshGhosts(ctx, GS_POSH));
   const double4* pos = ctx->cur.posh;
   if (ctx->listsValid && ctx->posKept) {
-    pos = ctx->listPos;
+    pos = ctx->alt.posh;
   } else if (ctx->listsValid && ctx->hKept && ctx->ns > 0) {
     hipLaunchKernelGGL(k_list_pos, dim3(blocks(ctx->ns + ctx->ng)), dim3(TPB), 0, ctx->stream,
                        ctx->cur.posh, ctx->hList, ctx->ns, ctx->n, ctx->ng, ctx->gorig,
@@ -921,17 +920,9 @@ int ensureLists(sphdem_ctx* ctx) {
 // place are made from, should a caller still ask for them.
 int keepLists(sphdem_ctx* ctx) {
   if (!ctx->listsNear || ctx->posKept || ctx->ns == 0) return 0;
-  const int64_t need = ctx->cap + ctx->ghostCap;
-  if (need > ctx->listPosCap) {
-    if (ctx->listPos) HIPC(hipFree(ctx->listPos));
-    ctx->listPos = nullptr;
-    ctx->listPosCap = 0;
-    HIPC(hipMalloc(&ctx->listPos, sizeof(double4) * need));
-    ctx->listPosCap = need;
-  }
   hipLaunchKernelGGL(k_list_pos, dim3(blocks(ctx->ns + ctx->ng)), dim3(TPB), 0, ctx->stream,
                      ctx->cur.posh, ctx->hKept ? ctx->hList : (const double*)nullptr, ctx->ns,
-                     ctx->n, ctx->ng, ctx->gorig, ctx->listPos);
+                     ctx->n, ctx->ng, ctx->gorig, ctx->alt.posh);
   LAUNCHED();
   ctx->posKept = true;
   return 0;
@@ -1429,8 +1420,7 @@ void freeAll(sphdem_ctx* ctx) {
                   ctx->mixP,        ctx->mixV,        ctx->mixD,    ctx->okey,
                   ctx->posm,        ctx->pairCnt,     ctx->pairOff, ctx->lrec,
                   ctx->lflag,       ctx->demNear,     ctx->nearGen, ctx->gate,
-                  ctx->keepMem,     ctx->dgKeep,      ctx->hList,   ctx->found,
-                  ctx->listPos};
+                  ctx->keepMem,     ctx->dgKeep,      ctx->hList,   ctx->found};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
   for (hipEvent_t e : ctx->evPool) (void)hipEventDestroy(e);
@@ -1709,7 +1699,7 @@ int sphdem_checkpoint_save(sphdem_ctx* ctx, void* host, int64_t capacity) {
   HIPC(hipMemcpyAsync(p, ctx->dg, sizeof(DevGlobals), hipMemcpyDeviceToHost, ctx->stream));
   p += sizeof(DevGlobals);
   // each stream in original-index order, staged through the other store buffer
-  double4* stage = ctx->alt.posh;
+  double4* stage = ctx->alt.vhm;  // alt.posh may hold the lists' positions
   for (int k = 0; k < kNumVec; k++) {
     hipLaunchKernelGGL(k_gather_orig, dim3(blocks(n)), dim3(TPB), 0, ctx->stream,
                        storeArr(ctx->cur, k), ctx->cur.orig, n, stage);
