@@ -361,6 +361,10 @@ int sphdem_num_deleted(const sphdem_ctx* ctx, int64_t* n);
  * launches, so "omega" times only sphdem_pass_omega. */
 int sphdem_timing_begin(sphdem_ctx* ctx, const char* kernel);
 int sphdem_timing_end(sphdem_ctx* ctx, double* total_ms, int64_t* launches);
+/* The near searches (the steps' own list build) since the context was created,
+ * replayed ones included, and the targets that they left to the exact search:
+ * all where some h is not positive, those of crowded cells. */
+int sphdem_near_searches(sphdem_ctx* ctx, int64_t* searches, int64_t* exact_targets);
 
 #ifdef __cplusplus
 }

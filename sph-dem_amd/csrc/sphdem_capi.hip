@@ -69,7 +69,7 @@ struct sphdem_ctx {
   Segment* segs = nullptr;
   int segColCap = 0, segCap = 0;
   bool segsValid = false;  // the segments partition the current store
-  DevGlobals* hostG = nullptr;  // pinned host copy of dg for the reset's readback
+  DevState* hostG = nullptr;  // pinned host copy for the reset's readback
   // tile shape: particles per list-build segment (<= 64, one wavefront; 0 for
   // the per-target search) and threads per workgroup of the SPH pair walkers
   // (sphdem_set_tile_shape)
@@ -93,6 +93,10 @@ struct sphdem_ctx {
   // and r and h are about to change from outside a step: both kept in alt.posh
   // (until the next reset, which writes alt, nothing else does)
   bool posKept = false;
+  // the near searches read back so far, the resets left for which the steps'
+  // searches are exact ones, and the last number of those
+  NearCount nearSeen{};
+  int nearWait = 0, nearBackoff = 0;
   // a search's records (recFresh, REC_*) and the mixed form's P and V records
   // (pvFresh) were written by the last reset's permutation and no position,
   // h or vhat changed since
@@ -127,7 +131,7 @@ struct sphdem_ctx {
   int partialCap = 0;
   double* fieldbuf = nullptr;
   int* errflag = nullptr;
-  DevGlobals* dg = nullptr;
+  DevGlobals* dg = nullptr;  // the first member of a DevState
   long long sphStep = 0;
   double ssr = 0.0;
   Grid gs{}, gc{};
@@ -509,6 +513,12 @@ int launchLists(sphdem_ctx* ctx, const double4* pos) {
   LAUNCHED();
   return 0;
 }
+// Up to this many targets (two tiles a CU) a tile's columns are searched by nine
+// wavefronts side by side instead of three after one another: a build is then a
+// chain of latencies.  Sedimentation boxes, one build, nine against three:
+// 12^3 23 / 37 us, 16^3 44 / 68, 20^3 27 / 42, 24^3 35 / 38, 28^3 52 / 64;
+// past it the wavefronts queue: 32^3 64 / 52, 64^3 265 / 125.
+constexpr int kNearSmall = 64 * 512;
 // Whether a step's walks take near lists: not with a segmented tile shape, and
 // not where a cell holds over kNearOccupancy particles at
 // the initial spacing (h grown at a free surface by a density
@@ -517,17 +527,34 @@ int launchLists(sphdem_ctx* ctx, const double4* pos) {
 // of the 48^3 dam break re-initialised every step (216 a cell), while at the
 // usual 27 a cell it takes 44 against 125 us (16^3 box), 125 against 199 us
 // (64^3) and 1.89 against 2.71 ms (160^3).
+// And not for a while (nearWait, set by countNear) after near searches that left
+// many of their targets to the exact part of k_near, as in crowded cells that
+// psep does not tell of or with a particle whose h is zero.
 constexpr double kNearOccupancy = 45.0;
 bool nearSearch(const sphdem_ctx* ctx) {
   const double e = ctx->P.psep > 0.0 ? ctx->gs.edge / ctx->P.psep : 0.0;
-  return ctx->tileSeg == 0 && e * e * e <= kNearOccupancy;
+  return ctx->tileSeg == 0 && e * e * e <= kNearOccupancy && ctx->nearWait == 0;
 }
-// Up to this many targets (two tiles a CU) a tile's columns are searched by nine
-// wavefronts side by side instead of three after one another: a build is then a
-// chain of latencies.  Sedimentation boxes, one build, nine against three:
-// 12^3 23 / 37 us, 16^3 44 / 68, 20^3 27 / 42, 24^3 35 / 38, 28^3 52 / 64;
-// past it the wavefronts queue: 32^3 64 / 52, 64^3 265 / 125.
-constexpr int kNearSmall = 64 * 512;
+// From a reset's readback: where over an eighth of the targets were left to the
+// exact part since the last one (it then costs as much as the near part saves),
+// the next 16 resets search exactly, and twice as many each time that a new
+// attempt ends the same way, up to 1024 (one slow search in a thousand).  Only
+// beyond kNearSmall: all targets in the exact part, one build by it and by the
+// exact search, with a zero h 127 and 325 us (16^3 box), 228 and 341 (28^3), 567
+// and 308 (48^3), 1229 and 586 (64^3), and with cells of 216 particles 216 and
+// 211 (16^3 dam break), 246 and 230 (20^3), 636 and 235 (24^3, 34776 targets),
+// 816 and 341 (36^3).
+void countNear(sphdem_ctx* ctx, const NearCount& now) {
+  const unsigned long long builds = now.builds - ctx->nearSeen.builds;
+  const unsigned long long exact = now.exact - ctx->nearSeen.exact;
+  ctx->nearSeen = now;
+  if (ctx->nearWait > 0) ctx->nearWait--;
+  if (builds == 0) return;
+  const bool bad =
+      ctx->ns > kNearSmall && exact * 8 > builds * (unsigned long long)ctx->ns;
+  ctx->nearBackoff = bad ? std::min(std::max(2 * ctx->nearBackoff, 16), 1024) : 0;
+  ctx->nearWait = ctx->nearBackoff;
+}
 // the near lists, right after a reset (positions in their cells)
 int launchNear(sphdem_ctx* ctx) {
   if (ctx->ns == 0) return 0;
@@ -543,7 +570,8 @@ int launchNear(sphdem_ctx* ctx) {
   auto launch = [&](auto kernel, int waves) {
     hipLaunchKernelGGL(kernel, dim3(8 * ((ctx->ns + 511) / 512)), dim3(64 * waves), 0,
                        ctx->stream, ctx->cur.posh, ctx->lrec, ctx->cur.cell, ctx->gs, ctx->gbase,
-                       ctx->start, ctx->ns, Q.inv, ctx->lflag, gen, ctx->nbl, ctx->nbcnt, ctx->dg);
+                       ctx->start, ctx->ns, Q.inv, ctx->lflag, gen, ctx->nbl, ctx->nbcnt,
+                       (DevState*)ctx->dg);
   };
   if (ctx->ns <= kNearSmall)
     launch(k_near<9>, 9);
@@ -705,10 +733,10 @@ int flagError(sphdem_ctx* ctx, unsigned flags) {
 // the end of every entry point that builds neighbour lists, so that no call
 // returns 0 after a pass used a clipped list.
 int checkFlags(sphdem_ctx* ctx) {
-  HIPC(hipMemcpyAsync(&ctx->hostG->errflags, &ctx->dg->errflags, sizeof(unsigned),
+  HIPC(hipMemcpyAsync(&ctx->hostG->g.errflags, &ctx->dg->errflags, sizeof(unsigned),
                       hipMemcpyDeviceToHost, ctx->stream));
   HIPC(hipStreamSynchronize(ctx->stream));
-  return flagError(ctx, ctx->hostG->errflags);
+  return flagError(ctx, ctx->hostG->g.errflags);
 }
 
 bool mixed(const sphdem_ctx* c);
@@ -770,15 +798,16 @@ int doReset(sphdem_ctx* ctx, bool keepSsr = false, bool midInit = false,
     LAUNCHED();
   } else {
     // into pinned memory: a direct copy, no staging through a runtime buffer
-    HIPC(hipMemcpyAsync(ctx->hostG, ctx->dg, sizeof(DevGlobals), hipMemcpyDeviceToHost,
+    HIPC(hipMemcpyAsync(ctx->hostG, ctx->dg, sizeof(DevState), hipMemcpyDeviceToHost,
                         ctx->stream));
-    const DevGlobals& hg = *ctx->hostG;
+    const DevGlobals& hg = ctx->hostG->g;
     HIPC(hipStreamSynchronize(ctx->stream));
     if (pre) ngPre = hg.ghostTotal;
     const double oldSsr = ctx->ssr;
     CHECK(flagError(ctx, hg.errflags));
     ctx->ns = ctx->ns0 - (int)hg.ndel_sph;
     ctx->nd = ctx->nd0 - (int)hg.ndel_dem;
+    countNear(ctx, ctx->hostG->near);
     double hmax;
     unsigned long long hb = hg.hmax_bits;
     memcpy(&hmax, &hb, sizeof(hmax));
@@ -1490,9 +1519,9 @@ int sphdem_create(const sphdem_params* params, int device, int64_t capacity, sph
     HIPC(hipMalloc(&ctx->gate, sizeof(int) * 4));
     HIPC(hipMemset(ctx->gate, 0, sizeof(int) * 4));
     HIPC(hipHostMalloc((void**)&ctx->gateHost, sizeof(int) * 4, hipHostMallocDefault));
-    HIPC(hipMalloc(&ctx->dg, sizeof(DevGlobals)));
-    HIPC(hipMemset(ctx->dg, 0, sizeof(DevGlobals)));
-    HIPC(hipHostMalloc((void**)&ctx->hostG, sizeof(DevGlobals), hipHostMallocDefault));
+    HIPC(hipMalloc((void**)&ctx->dg, sizeof(DevState)));
+    HIPC(hipMemset(ctx->dg, 0, sizeof(DevState)));
+    HIPC(hipHostMalloc((void**)&ctx->hostG, sizeof(DevState), hipHostMallocDefault));
     ctx->hostCopy.prepare(sizeof(double) * 3 * (size_t)capacity);
     return 0;
   };
@@ -1574,6 +1603,7 @@ int sphdem_upload(sphdem_ctx* ctx, int64_t n, const double* r, const double* v, 
   g.maxdt = ctx->P.maxdt;
   HIPC(hipMemcpy(ctx->dg, &g, sizeof(g), hipMemcpyHostToDevice));
   ctx->sphStep = 0;
+  ctx->nearWait = ctx->nearBackoff = 0;
   // CdataLL::CdataLL (dataLL.cpp:8-40): hmax = sph_search_radius = H, then reset()
   ctx->ssr = ctx->P.h;
   ctx->gridValid = false;
@@ -2136,7 +2166,7 @@ std::vector<unsigned char> graphKeyOf(const sphdem_ctx* c, int hookset) {
   putBytes(v, c->storeMem[1]);
   putBytes(v, c->cur.posh);
   const int ints[] = {c->n, c->ns, c->nd, c->ns0, c->nd0, c->K, c->gbase, hookset, c->tileSeg,
-                      c->walkTPB, c->reachShep, c->overlap ? 1 : 0};
+                      c->walkTPB, c->reachShep, c->overlap ? 1 : 0, nearSearch(c) ? 1 : 0};
   putBytes(v, ints);
   putBytes(v, c->ghostCap);
   putBytes(v, c->ssr);
@@ -2848,6 +2878,18 @@ int sphdem_reduce_dt(sphdem_ctx* ctx, double* newdt) {
   HIPC(hipMemcpyAsync(&d, ctx->dg, sizeof(d), hipMemcpyDeviceToHost, ctx->stream));
   HIPC(hipStreamSynchronize(ctx->stream));
   memcpy(newdt, &d.newDt_bits, sizeof(double));
+  return 0;
+}
+
+int sphdem_near_searches(sphdem_ctx* ctx, int64_t* searches, int64_t* exact_targets) {
+  if (!ctx || !searches || !exact_targets) return SPHDEM_E_ARG;
+  HIPC(hipSetDevice(ctx->device));
+  NearCount c;
+  HIPC(hipMemcpyAsync(&c, &((DevState*)ctx->dg)->near, sizeof(c), hipMemcpyDeviceToHost,
+                      ctx->stream));
+  HIPC(hipStreamSynchronize(ctx->stream));
+  *searches = (int64_t)c.builds;
+  *exact_targets = (int64_t)c.exact;
   return 0;
 }
 

@@ -76,6 +76,16 @@ struct DevGlobals {
   int ghostTotal;         // ghost entries counted by the last reset's scan
 };
 
+// The near searches run so far and the targets they left to their exact part.
+struct NearCount {
+  unsigned long long builds, exact;
+};
+// What a context holds on the device; a checkpoint keeps g alone.
+struct DevState {
+  DevGlobals g;
+  NearCount near;
+};
+
 // Cells (per axis) a ghost may occupy: one beyond the cells real particles of
 // a periodic axis can hold, [cellOf(min) - 1, cellOf(max) + 1] of the domain.
 struct GhostBand {

@@ -557,7 +557,7 @@ __global__ void __launch_bounds__(64 * W, W == 3 ? 4 : 3)
     k_near(const double4* __restrict__ pos, const uint4* __restrict__ rec,
            const int* __restrict__ cellc, Grid g, int gbase, const int* __restrict__ start, int ns,
            double qinv, const int* __restrict__ lflag, int gen, int* __restrict__ nbl,
-           int* __restrict__ nbcnt, DevGlobals* dg) {
+           int* __restrict__ nbcnt, DevState* dev) {
   constexpr int kNearSlots = nearSlots(W);
   __shared__ NearWave<kNearSlots> lds[W];
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
@@ -798,6 +798,10 @@ __global__ void __launch_bounds__(64 * W, W == 3 ? 4 : 3)
     __syncthreads();
   }
 
+  if (threadIdx.x == 0) {
+    if (t0 == 0) dev->near.builds++;
+    if (exact) atomicAdd(&dev->near.exact, (unsigned long long)__popcll(exact));
+  }
   // ---- exact lists: the FP64 test of is_neighbr (particle.h:236-238) over the
   // 27 cells, a lane per candidate; the wavefronts take the targets in turn
   for (; exact; exact &= exact - 1) {
@@ -832,7 +836,7 @@ __global__ void __launch_bounds__(64 * W, W == 3 ? 4 : 3)
             }
           }
     if (lane == 0) {
-      if (c > kMaxNb) atomicOr(&dg->errflags, 2u);
+      if (c > kMaxNb) atomicOr(&dev->g.errflags, 2u);
       nbcnt[st] = min(c, kMaxNb);
     }
   }

@@ -646,6 +646,7 @@ def load_library(path: str = LIB_PATH):
                                            ctypes.POINTER(ctypes.c_int), dp]
     lib.sphdem_timing_begin.argtypes = [vp, ctypes.c_char_p]
     lib.sphdem_timing_end.argtypes = [vp, dp, ctypes.POINTER(i64)]
+    lib.sphdem_near_searches.argtypes = [vp, ctypes.POINTER(i64), ctypes.POINTER(i64)]
     _lib = lib
     return lib
 
@@ -882,6 +883,12 @@ class Sim:
         return s.value, b.value, ms.value
 
     # ---- measurement: HIP events around each launch of one kernel
+    def near_searches(self) -> tuple[int, int]:
+        """(near searches run, targets they left to the exact search)."""
+        n, x = ctypes.c_int64(), ctypes.c_int64()
+        self._check(self.lib.sphdem_near_searches(self.ctx, ctypes.byref(n), ctypes.byref(x)))
+        return n.value, x.value
+
     def timing_begin(self, kernel: str):
         self._check(self.lib.sphdem_timing_begin(self.ctx, kernel.encode()))
 
