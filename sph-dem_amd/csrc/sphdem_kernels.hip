@@ -86,15 +86,10 @@ __device__ __forceinline__ void atomicMaxPos(unsigned long long* p, double v) {
 // point q, for each periodic image shift s (s = 0 first): the candidates b are
 // real particles whose image r_b + s*L may lie near q.  Cells along z of one
 // (x,y) column are contiguous in the sorted store, so each column is one range.
-// `first`/`stride` split each contiguous range over the lanes of a wavefront.
-struct KeepAll {
-  __device__ bool operator()(int, int, int) const { return true; }
-};
-template <class V, class K = KeepAll>
+template <class V>
 __device__ __forceinline__ void forCells(const Grid& g, const int* __restrict__ start,
                                          const Box& B, double qx, double qy, double qz,
-                                         int reach, V&& visit, int first = 0, int stride = 1,
-                                         K&& keep = K()) {
+                                         int reach, V&& visit) {
   const int nsx = B.periodic[0] ? 3 : 1, nsy = B.periodic[1] ? 3 : 1, nsz = B.periodic[2] ? 3 : 1;
   const double q[3] = {qx, qy, qz};
   for (int ix = 0; ix < nsx; ix++) {
@@ -114,12 +109,12 @@ __device__ __forceinline__ void forCells(const Grid& g, const int* __restrict__ 
         const double tz = sz == 0 ? q[2] : (sz == 1 ? q[2] - B.Lp[2] : q[2] - B.Lm[2]);
         const int cz = cellOf(tz, g, 2);
         const int z0 = max(cz - reach, 0), z1 = min(cz + reach, g.dim[2] - 1);
-        if (z0 > z1 || !keep(cx, cy, cz)) continue;
+        if (z0 > z1) continue;
         for (int a = x0; a <= x1; a++)
           for (int b = y0; b <= y1; b++) {
             const int k0 = g.base + (a * g.dim[1] + b) * g.dim[2];
             const int j0 = start[k0 + z0], j1 = start[k0 + z1 + 1];
-            for (int j = j0 + first; j < j1; j += stride) visit(j, sx, sy, sz);
+            for (int j = j0; j < j1; j++) visit(j, sx, sy, sz);
           }
       }
     }
@@ -822,10 +817,12 @@ __device__ __forceinline__ CellSpan cellSpan(double t, const Grid& g, int d, int
   }
   return CellSpan{max(lo, 0), min(hi, g.dim[d] - 1)};
 }
-// The candidate ranges of forCells for a wave-uniform query point: visit(j0,
-// j1, sx, sy, sz) once per column range, in forCells' order.  half > 0: only the
-// cells of the coordinates within half of the query's (cellOf is monotone: they
-// hold every particle that near).
+// The candidate ranges of forCells: visit(j0, j1, sx, sy, sz) once per column
+// range, in forCells' order.  Lanes that take a query together give the same
+// point; a wavefront may hold several such groups, which then part ways here (a
+// ballot in visit is to be masked to the group).  half > 0: only the cells of the
+// coordinates within half of the query's (cellOf is monotone: they hold every
+// particle that near).
 template <class V>
 __device__ __forceinline__ void forCellRanges(const Grid& g, const int* __restrict__ start,
                                               const Box& B, double qx, double qy, double qz,
