@@ -565,7 +565,8 @@ int launchNear(sphdem_ctx* ctx) {
   const int gen = ctx->lgen++ & 1;
   if (ctx->recFresh != REC_NEAR) {  // else the reset's permutation wrote them
     hipLaunchKernelGGL(k_near_rec, dim3(blocks(ctx->ns + ctx->ng)), dim3(TPB), 0, ctx->stream,
-                       ctx->cur.posh, ctx->ns, ctx->n, ctx->ng, Q, ctx->lrec, ctx->lflag, gen,
+                       ctx->cur.posh, ctx->cur.vhm, ctx->ns, ctx->n, ctx->ng, Q, ctx->lrec,
+                       ctx->lflag, gen,
                        ctx->graphMode ? &ctx->dg->ghostTotal : (const int*)nullptr);
     LAUNCHED();
   }
@@ -1065,7 +1066,7 @@ int passEos(sphdem_ctx* ctx) {
                   ? ctx->mixD
                   : nullptr;
   hipLaunchKernelGGL(k_eos, dim3(blocks(ctx->ns)), dim3(TPB), 0, ctx->stream, ctx->cur, ctx->ns,
-                     ctx->P, D);
+                     ctx->P, D, ctx->lflag + (ctx->lgen & 1));
   LAUNCHED();
   markStale(ctx, GS_DPO);
   ctx->dFresh = D != nullptr;
@@ -1098,6 +1099,8 @@ unsigned walkerLds(const sphdem_ctx* ctx, unsigned waves) {
   return std::min(65536u, (163840u / (blocks + 1u) / 1024u + 1u) * 1024u);
 }
 constexpr unsigned kForceWaves = 2, kDddtWaves = 3;
+// the flag word of the lists in place
+const int* listFlags(const sphdem_ctx* ctx) { return ctx->lflag + ((ctx->lgen + 1) & 1); }
 // (near lists are walked by steps only, whose walk sums omega under VAR_H)
 template <int F, bool OMG, bool NEAR>
 void launchForce(sphdem_ctx* ctx) {
@@ -1111,8 +1114,8 @@ void launchForce(sphdem_ctx* ctx) {
                          ctx->mixD, ctx->mixRes, ctx->P, ctx->dg);
     else
       hipLaunchKernelGGL((k_force_l<V, M, A, L, OMG, NEAR>), dim3(walkBlocks(ctx, ctx->ns)), dim3(ctx->walkTPB), 0,
-                         ctx->stream, ctx->cur, ctx->ns, ctx->box, ctx->nbl, ctx->nbcnt, ctx->hinv,
-                         ctx->P, ctx->dg);
+                         ctx->stream, ctx->cur, ctx->ns, ctx->box, ctx->nbl, ctx->nbcnt,
+                         listFlags(ctx), ctx->hinv, ctx->P, ctx->dg);
   }
 }
 template <bool OMG, bool NEAR, int... F>
@@ -1162,8 +1165,8 @@ int passDddt(sphdem_ctx* ctx, bool withOmega = false, bool inStep = false) {
     CHECK(packMix(ctx, MIX_P | MIX_V));
     auto launch = [&](auto kernel) {
       hipLaunchKernelGGL(kernel, grid, block, omega ? walkerLds(ctx, kDddtWaves) : 0u, ctx->stream,
-                         ctx->cur, ctx->ns, ctx->nbl, ctx->nbcnt, ctx->mixP, ctx->mixV,
-                         ctx->mixRes, ctx->P.wcon);
+                         ctx->cur, ctx->ns, ctx->nbl, ctx->nbcnt, listFlags(ctx), ctx->mixP,
+                         ctx->mixV, ctx->mixRes, ctx->P.wcon);
     };
     if (omega)
       launch(near ? k_dddt_m<true, true, true> : k_dddt_m<true, true, false>);
@@ -1176,7 +1179,8 @@ int passDddt(sphdem_ctx* ctx, bool withOmega = false, bool inStep = false) {
     Timed tm(ctx, KID_DDDT);
     auto launch = [&](auto kernel) {
       hipLaunchKernelGGL(kernel, grid, block, 0, ctx->stream, ctx->cur, ctx->ns, ctx->box, ctx->nbl,
-                         ctx->nbcnt, varH(ctx) ? (const double2*)nullptr : ctx->hinv, ctx->P.wcon);
+                         ctx->nbcnt, listFlags(ctx),
+                         varH(ctx) ? (const double2*)nullptr : ctx->hinv, ctx->P.wcon);
     };
     if (omega)
       launch(near ? k_dddt_l<true, true, true> : k_dddt_l<true, true, false>);

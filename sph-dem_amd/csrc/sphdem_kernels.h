@@ -105,6 +105,14 @@ struct WrapFold {
   double ax, ay, az;
 };
 
+// What a list search and the walks of its lists ask of the generation's flag
+// word: a position or h that is no bound; a velocity, mass, density or pressure
+// term that is not finite, or so large or (density) small that a product of a few
+// of them might not be; an h of which 1/h^5 is not finite in FP32.
+enum { FLAG_BOUNDS = 1, FLAG_VALUES = 2 };
+constexpr double kLargeValue = 1e30, kSmallH = 3e-8;
+__device__ __forceinline__ bool usual(double x) { return fabs(x) < kLargeValue; }
+
 // The per-target list search's record of an SPH-group entry or ghost: its
 // position as 16-bit fixed point modulo 2^16 in the unit 1/uinv (a power of
 // two) from the origin o, and the bound code B16 = ceil(((2 h / u + kQBand)^2
@@ -155,24 +163,28 @@ __device__ __forceinline__ float4 mixRecordV(const double4& p, const double4& vh
 
 // The near search's record of an SPH-group entry or ghost: its position in
 // Quant's fixed point and, as FP32 rounded up, the square of 2 h in that unit.
-// False (and a zero record) for a non-finite position or a non-positive h.
-__device__ __forceinline__ bool nearRecord(const double4& p, const Quant& Q, uint4& r) {
+// Returns the entry's flags: FLAG_BOUNDS (and a zero record) for a non-finite
+// position or a non-positive h, FLAG_VALUES by its vhat and mass vh and its h.
+__device__ __forceinline__ int nearRecord(const double4& p, const double4& vh, const Quant& Q,
+                                          uint4& r) {
+  const bool ok = usual(vh.x) && usual(vh.y) && usual(vh.z) && usual(vh.w) && p.w >= kSmallH;
+  const int f = ok ? 0 : (int)FLAG_VALUES;
   if (!(isfinite(p.x) && isfinite(p.y) && isfinite(p.z) && isfinite(p.w) && p.w > 0.0)) {
     r = make_uint4(0u, 0u, 0u, 0u);
-    return false;
+    return f | FLAG_BOUNDS;
   }
   const double b = 2.0 * p.w * Q.inv;
   r = make_uint4(quant1(p.x, Q.o[0], Q.inv), quant1(p.y, Q.o[1], Q.inv),
                  quant1(p.z, Q.o[2], Q.inv),
                  __float_as_uint((float)fmin(b * b * (1.0 + 1e-6), 1e30)));
-  return true;
+  return f;
 }
 
 // Records a folded reset's permutation writes on the way (WrapFold): the
 // SPH-group entries [0, ns) and the ghosts, from the values it stores.
 enum { REC_NONE, REC_NEAR, REC_EXACT };  // none; k_near's (uint4); k_lists_t's (uint2)
 struct PermRecords {
-  int lists;  // a search's records (REC_*; non-finite input to lflag[gen & 1])
+  int lists;  // a search's records (REC_*; flags to lflag[gen & 1])
   int mixed;  // the mixed form's P and V records
   int ns;
   ListQuant lq;

@@ -573,11 +573,12 @@ __device__ __forceinline__ void permRecords(const PermRecords& R, int p, const d
                                             const double4& vh) {
   if (R.lists == REC_NEAR) {
     uint4 r;
-    if (!nearRecord(q, R.Q, r)) atomicOr(&R.lflag[R.gen & 1], 1);
+    const int f = nearRecord(q, vh, R.Q, r);
+    if (f) atomicOr(&R.lflag[R.gen & 1], f);
     R.rec[p] = r;
   } else if (R.lists == REC_EXACT) {
     uint2 r;
-    if (!listRecord(q, R.lq, r)) atomicOr(&R.lflag[R.gen & 1], 1);
+    if (!listRecord(q, R.lq, r)) atomicOr(&R.lflag[R.gen & 1], FLAG_BOUNDS);
     reinterpret_cast<uint2*>(R.rec)[p] = r;
   }
   if (R.mixed) {
@@ -741,8 +742,10 @@ __global__ void k_snapshot(Store src, Store dst, int n, const DevGlobals* __rest
 
 // CsphIncompress::calcPressSpsoundPdr2 sphIncompress.h:863-896
 // D (optional): also the mixed form's D record {dens, pdr2, 1/h, 1/h^5} of
-// each entry, as the mixed record packing would write it afterwards.
-__global__ void k_eos(Store S, int ns, sphdem_params P, float4* __restrict__ D) {
+// each entry, as the mixed record packing would write it afterwards.  flags: the
+// next list search's flag word (FLAG_VALUES by density and pdr2).
+__global__ void k_eos(Store S, int ns, sphdem_params P, float4* __restrict__ D,
+                      int* __restrict__ flags) {
   const int a = blockIdx.x * blockDim.x + threadIdx.x;
   if (a >= ns) return;
   if (!isSphT(S.iam[a])) return;
@@ -754,6 +757,7 @@ __global__ void k_eos(Store S, int ns, sphdem_params P, float4* __restrict__ D) 
     press = P.prb * (pow(d.x / P.refd, 7.0) - 1.0);
   // only pdr2 and press are stored (omega may be written beside this pass)
   const double pdr2 = press / (d.x * d.x);
+  if (!(d.x > 1.0 / kLargeValue && usual(d.x) && usual(pdr2))) atomicOr(flags, FLAG_VALUES);
   S.dpo[a].y = pdr2;
   S.v0p[a].w = press;
   if (D) {

@@ -228,14 +228,18 @@ __global__ void __launch_bounds__(256) k_reinit_m(Store S, int ns, const int* __
 // ---- calcDddtDudt, mixed -----------------------------------------------------------
 // OMG (VAR_H only): calcOmega fused into the walk (the k_omega_m sum, in list
 // order); the dddt terms are summed without 1/omega_a and scaled once in FP64.
-// NEAR: the list is a near list (true: walk again).  An entry just beyond the
-// radius whose rounded distance falls below 2 h adds less than 1e-20 of a usual
-// pair's term.
+// NEAR: the list is a near list.  An entry just beyond the radius whose rounded
+// distance falls below 2 h adds less than 1e-20 of a usual pair's term.
 template <bool VARH, bool OMG, bool NEAR>
-__device__ __forceinline__ bool walkDddtM(const Store& S, int a, int ns, int* __restrict__ nbl,
-                                          int* __restrict__ nbcnt, const uint4* __restrict__ P,
-                                          const float4* __restrict__ V, float res, double wcon) {
+__global__ void __launch_bounds__(256) k_dddt_m(Store S, int ns, int* __restrict__ nbl,
+                                                int* __restrict__ nbcnt,
+                                                const int* __restrict__ flags,
+                                                const uint4* __restrict__ P,
+                                                const float4* __restrict__ V, float res,
+                                                double wcon) {
   static_assert(VARH || !OMG, "omega is only fused under VAR_H");
+  const int a = xcdThread();
+  if (a >= ns) return;
   const uint4 qa = P[a];
   const float4 va = V[a];
   const double ha = S.posh[a].w;
@@ -246,7 +250,7 @@ __device__ __forceinline__ bool walkDddtM(const Store& S, int a, int ns, int* __
   const float i3 = OMG ? (float)(1.0 / cube(ha)) : 0.0f, c3 = OMG ? (float)(3.0 / pow4(ha)) : 0.0f;
   double om = OMG ? S.vhm[a].w * (double)wendPdWh_m(wc, 0.0f, rha, i3, c3) : 0.0;
   double dddt = OMG ? 0.0 : S.vh0d[a].w;
-  const int n = nbcnt[a];
+  const int n = walkLength<NEAR>(flags, S.posh, a, ns, nbl, nbcnt);
   constexpr int U = 8;
   for (int k0 = 0; k0 < n; k0 += U) {
     SPHDEM_FETCH_ENTRIES(U)
@@ -277,24 +281,12 @@ __device__ __forceinline__ bool walkDddtM(const Store& S, int a, int ns, int* __
       dddt += (double)__uint_as_float(q[u].w) * (double)(gF * (dv0 * d.x + dv1 * d.y + dv2 * d.z));
     }
   }
-  if (NEAR && walkAgain(dddt + om, S.posh, a, ns, nbl, nbcnt)) return true;
   if (OMG) {
     const double omega = 1 + ha * om / (S.dpo[a].x * 3);
     S.dpo[a].z = omega;
     dddt = S.vh0d[a].w + (1.0 / omega) * dddt;
   }
   S.vh0d[a].w = dddt;
-  return false;
-}
-template <bool VARH, bool OMG, bool NEAR>
-__global__ void __launch_bounds__(256) k_dddt_m(Store S, int ns, int* __restrict__ nbl,
-                                                int* __restrict__ nbcnt,
-                                                const uint4* __restrict__ P,
-                                                const float4* __restrict__ V, float res,
-                                                double wcon) {
-  int a = xcdThread();
-  if (a >= ns) return;
-  while (walkDddtM<VARH, OMG, NEAR>(S, a, ns, nbl, nbcnt, P, V, res, wcon)) a = anew(a);
 }
 
 // ---- calcForce, mixed --------------------------------------------------------------

@@ -320,7 +320,7 @@ __global__ void k_lrec(const double4* __restrict__ posh, int ns, int n, int ng, 
   if (i >= ns + (ngp ? min(*ngp, ng) : ng)) return;
   const int s = i < ns ? i : n + (i - ns);
   uint2 r;
-  if (!listRecord(posh[s], lq, r)) atomicOr(&lflag[gen & 1], 1);
+  if (!listRecord(posh[s], lq, r)) atomicOr(&lflag[gen & 1], FLAG_BOUNDS);
   rec[s] = r;
 }
 
@@ -357,7 +357,7 @@ __global__ void __launch_bounds__(256) k_lists_t(const double4* __restrict__ pos
   const uint2 own = rec[t];
   const short2v ownxy = asShort2(own.x);
   int aq = -1, bq = 0x7fffffff;
-  if (lflag[gen & 1] == 0) {
+  if ((lflag[gen & 1] & FLAG_BOUNDS) == 0) {
     const double a = 2.0 * p.w * uinv - kQBand;
     if (a > 0.0) aq = (int)floor(a * a) - 1;
     const double b = 2.0 * p.w * uinv + kQBand;
@@ -447,9 +447,9 @@ __global__ void __launch_bounds__(256) k_lists_t(const double4* __restrict__ pos
 // every SPH neighbour within 2 max(h) and some beyond (just beyond where all h
 // are equal, up to sqrt(T_a + T_b - T_0) below where they differ), whose kernel
 // terms are zero in FP64.  The walks take the pairs of the dt conditions by the
-// FP64 test, and leave the others out where their values are not finite
-// (walkAgain).  So no candidate needs the FP64 test here, and the distance tests
-// run on the matrix cores.
+// FP64 test, and leave the others out where values are not finite (pairsOnly).
+// So no candidate needs the FP64 test here, and the distance tests run on the
+// matrix cores.
 //
 // A workgroup takes a tile of 64 consecutive targets of the cell-sorted store,
 // lane l of every wavefront owning target l.  Its W = 3 wavefronts take the
@@ -518,15 +518,16 @@ __device__ __forceinline__ unsigned foldSigns(unsigned m, const float16v& v) {
 }
 // The near search's records of the SPH-group entries [0, ns) and the ghosts
 // [n, n + ng); flag slots as for k_lrec.
-__global__ void k_near_rec(const double4* __restrict__ posh, int ns, int n, int ng, Quant Q,
-                           uint4* __restrict__ rec, int* __restrict__ lflag, int gen,
+__global__ void k_near_rec(const double4* __restrict__ posh, const double4* __restrict__ vhm,
+                           int ns, int n, int ng, Quant Q, uint4* __restrict__ rec, int* __restrict__ lflag, int gen,
                            const int* __restrict__ ngp) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i == 0) lflag[(gen + 1) & 1] = 0;
   if (i >= ns + (ngp ? min(*ngp, ng) : ng)) return;
   const int s = i < ns ? i : n + (i - ns);
   uint4 r;
-  if (!nearRecord(posh[s], Q, r)) atomicOr(&lflag[gen & 1], 1);
+  const int f = nearRecord(posh[s], vhm[s], Q, r);
+  if (f) atomicOr(&lflag[gen & 1], f);
   rec[s] = r;
 }
 // bits [32 - k, 32) set: the first k of a word's candidates
@@ -581,7 +582,7 @@ __global__ void __launch_bounds__(64 * W, W == 3 ? 4 : 3)
 
   unsigned long long exact = 0ull;  // targets left to the exact search
   unsigned long long todo = __ballot(act);
-  if (lflag[gen & 1] != 0) {
+  if (lflag[gen & 1] & FLAG_BOUNDS) {
     exact = todo;
     todo = 0ull;
   }
@@ -992,12 +993,10 @@ __device__ __forceinline__ bool pairWithin(const double4& pa, const double4& pb)
   return dot3(x, y, z, x, y, z) <= l * l;
 }
 // A near list's entries beyond the radius add exact zeros, or, where such an
-// entry's mass, density, pressure or velocity is not finite, NaN.  So a particle
-// whose sums do not come out finite keeps the pairs of its list only and is
-// walked again (walkAgain; the walks below store nothing before).
-__device__ __forceinline__ bool walkAgain(double sums, const double4* posh, int a, int ns,
-                                          int* nbl, int* nbcnt) {
-  if (fabs(sums) < __longlong_as_double(0x7ff0000000000000ll)) return false;
+// entry's mass, density, pressure or velocity is not finite, NaN.  Then the list
+// is cut down to its pairs before the sums are taken: pairsOnly returns its
+// length.
+__device__ __forceinline__ int pairsOnly(const double4* posh, int a, int ns, int* nbl, int* nbcnt) {
   const double4 pa = posh[a];
   const int n = nbcnt[a];
   int m = 0;
@@ -1005,9 +1004,27 @@ __device__ __forceinline__ bool walkAgain(double sums, const double4* posh, int 
     const int j = nbl[nbEntry(k, a, ns)];
     if (pairWithin(pa, posh[j])) nbl[nbEntry(m++, a, ns)] = j;
   }
-  if (m == n) return false;
   nbcnt[a] = m;
-  return true;
+  return m;
+}
+// A walk's list length.  The FP64 walks and the mixed dddt walk ask beforehand, all
+// of them, whether any particle holds such a value (FLAG_VALUES, set where the
+// values are written).  Asked by each particle of its own sums at the end, FP64
+// force takes 5.91 ms at 160^3, in place of 5.79 without the question; asked here
+// 5.59.
+template <bool NEAR>
+__device__ __forceinline__ int walkLength(const int* __restrict__ flags, const double4* posh,
+                                          int a, int ns, int* nbl, int* nbcnt) {
+  if (NEAR && (*flags & FLAG_VALUES)) return pairsOnly(posh, a, ns, nbl, nbcnt);
+  return nbcnt[a];
+}
+// The mixed force walk asks of its sums whether to walk again, before it stores
+// anything (at no cost; in FP32 finite values may overflow on the way as well).
+__device__ __forceinline__ bool walkAgain(double sums, const double4* posh, int a, int ns,
+                                          int* nbl, int* nbcnt) {
+  if (fabs(sums) < __longlong_as_double(0x7ff0000000000000ll)) return false;
+  const int n = nbcnt[a];
+  return pairsOnly(posh, a, ns, nbl, nbcnt) < n;
 }
 // a, as a value the compiler knows nothing of: a second walk reads its particle
 // afresh, and the first keeps no registers for it.
@@ -1019,14 +1036,16 @@ __device__ __forceinline__ int anew(int a) {
 // ---- calcDddtDudt (sphIncompress.h:783-851) over the cached list ----------------
 // OMG (VAR_H only): calcOmega fused into the walk, as in k_force_l -- every
 // dddt term of a is linear in 1/omega_a, so the terms are summed without it
-// beside the omega sum and scaled once.  NEAR: the list is a near list (true:
-// walk again).  Three wavefronts per SIMD: 168 VGPRs without spills (170 would
-// allow two), 2 % faster.
+// beside the omega sum and scaled once.  NEAR: the list is a near list.  Three
+// wavefronts per SIMD: 168 VGPRs without spills (170 would allow two), 2 % faster.
 template <bool VARH, bool OMG, bool NEAR>
-__device__ __forceinline__ bool walkDddt(const Store& S, int a, int ns, int* __restrict__ nbl,
-                                         int* __restrict__ nbcnt,
-                                         const double2* __restrict__ hinv, double wcon) {
+__global__ void __launch_bounds__(256, 3) k_dddt_l(Store S, int ns, Box B, int* __restrict__ nbl,
+                                                   int* __restrict__ nbcnt,
+                                                   const int* __restrict__ flags,
+                                                   const double2* __restrict__ hinv, double wcon) {
   static_assert(VARH || !OMG, "omega is only fused under VAR_H");
+  const int a = xcdThread();
+  if (a >= ns) return;
   const double4 pa = S.posh[a];
   const double4 va = S.vhm[a];
   const double ha = pa.w;
@@ -1038,7 +1057,7 @@ __device__ __forceinline__ bool walkDddt(const Store& S, int a, int ns, int* __r
   // under VAR_H, sph.h:331-332): F(q, h) = WCON poly(q) / (q h^5) and 1/q = h/r
   const double Ka = wcon * (rha * rha) * (rha * rha) * rom;
   double dddt = OMG ? 0.0 : S.vh0d[a].w;
-  const int n = nbcnt[a];
+  const int n = walkLength<NEAR>(flags, S.posh, a, ns, nbl, nbcnt);
   constexpr int U = 8;
   for (int k0 = 0; k0 < n; k0 += U) {
     SPHDEM_FETCH_ENTRIES(U)
@@ -1070,22 +1089,12 @@ __device__ __forceinline__ bool walkDddt(const Store& S, int a, int ns, int* __r
       dddt += v[u].w * (dot3(dv0, dv1, dv2, dx, dy, dz) * G);
     }
   }
-  if (NEAR && walkAgain(dddt + om, S.posh, a, ns, nbl, nbcnt)) return true;
   if (OMG) {
     const double omega = 1 + ha * om / (S.dpo[a].x * 3);
     S.dpo[a].z = omega;
     dddt = S.vh0d[a].w + (1.0 / omega) * dddt;
   }
   S.vh0d[a].w = dddt;
-  return false;
-}
-template <bool VARH, bool OMG, bool NEAR>
-__global__ void __launch_bounds__(256, 3) k_dddt_l(Store S, int ns, Box B, int* __restrict__ nbl,
-                                                   int* __restrict__ nbcnt,
-                                                   const double2* __restrict__ hinv, double wcon) {
-  int a = xcdThread();
-  if (a >= ns) return;
-  while (walkDddt<VARH, OMG, NEAR>(S, a, ns, nbl, nbcnt, hinv, wcon)) a = anew(a);
 }
 
 // ---- calcForce (sphIncompress.h:899-972; sph.h:579-666, 692-734) over the list --
@@ -1096,9 +1105,8 @@ __global__ void __launch_bounds__(256, 3) k_dddt_l(Store S, int ns, Box B, int* 
 // speed is constant, through the smallest numerators.
 //
 // NEAR: the list is a near list, whose entries beyond the radius set no
-// condition (true: walk again).  An exact list's pairs all set theirs, as
-// calcForce over the cached neighbours does, also where r or h has changed since
-// the list was made.
+// condition.  An exact list's pairs all set theirs, as calcForce over the cached
+// neighbours does, also where r or h has changed since the list was made.
 //
 // OMG (VAR_H only): calcOmega fused into the same walk.  Under VAR_H every
 // force term of a is linear in 1/omega_a and in nothing else of omega
@@ -1107,160 +1115,161 @@ __global__ void __launch_bounds__(256, 3) k_dddt_l(Store S, int ns, Box B, int* 
 // force terms taken without 1/omega_a, stores omega_a, and adds the force
 // sums times 1/omega_a to the incoming f, fp, fv.
 template <bool VARH, int VISC, bool ARTIF, bool LIQDEM, bool OMG, bool NEAR>
-__device__ __forceinline__ bool walkForce(const Store& S, int a, int ns, int* __restrict__ nbl,
-                                          int* __restrict__ nbcnt,
-                                          const double2* __restrict__ hinv, const sphdem_params& P,
-                                          double& newDt) {
-  static_assert(VARH || !OMG, "omega is only fused under VAR_H");
-  const double inf = __longlong_as_double(0x7ff0000000000000ll);
-  const bool fluid = S.iam[a] == T_SPH;  // viscosity only acts on sph (sphIncompress.h:927)
-  const double4 pa = S.posh[a];
-  const double4 va = S.vhm[a];
-  const double4 da = S.dpo[a];
-  const double ha = pa.w;
-  const double rha = 1.0 / ha;
-  const double rom = (VARH && !OMG) ? 1.0 / da.z : 1.0;
-  const double i3 = OMG ? 1.0 / cube(ha) : 0.0, c3 = OMG ? 3.0 / pow4(ha) : 0.0;
-  double om = OMG ? va.w * wendPdWhi(P.wcon, 0, ha, rha, i3, c3) : 0.0;
-  // gradW = dr * F(q, h) (/ omega_a under VAR_H), F = WCON poly(q) / (q h^5)
-  // = dr * poly(q) * K(h) / r with K(h) = WCON h^-4 (/ omega_a)
-  const double Ka = P.wcon * (rha * rha) * (rha * rha) * rom;
-  const double wrom = P.wcon * rom;
-  const double viscLiq = 2.0 * P.viscosity * P.dens;  // numerator under LIQ_DEM
-  const double vsigC = (VISC == VISC_MOR || VISC == VISC_CLE) ? 2.0 * P.spsound : 0.0;
-  const double cdiff = VISC == VISC_MON ? 0.06 : 0.125;  // viscDiffusionCondition
-  const double alphaM = monaghanAlpha(P);
-  double minA = inf, minB = inf;  // min over pairs of 0.6 hav and cdiff hav^2
-  const double4 zero4 = make_double4(0.0, 0.0, 0.0, 0.0);
-  double4 f = OMG ? zero4 : S.frc[a], fpa = OMG ? zero4 : S.fp[a], fva = OMG ? zero4 : S.fv[a];
-  const int n = nbcnt[a];
-  constexpr int U = 4;
-  for (int k0 = 0; k0 < n; k0 += U) {
-    SPHDEM_FETCH_ENTRIES(U)
-    double4 p[U], v[U];
-    double2 d[U], hi[U];
-#pragma unroll
-    for (int u = 0; u < U; u++) {
-      const int j = e[u];
-      p[u] = S.posh[j];
-      v[u] = S.vhm[j];
-      d[u] = *reinterpret_cast<const double2*>(&S.dpo[j]);  // dens, pdr2
-      hi[u] = hinv[j];
-    }
-#pragma unroll
-    for (int u = 0; u < U; u++) {
-      if (k0 + u >= n) break;
-      const double hb = p[u].w, mb = v[u].w, rhob = d[u].x, pdr2b = d[u].y;
-      const double dx = pa.x - p[u].x, dy = pa.y - p[u].y, dz = pa.z - p[u].z;
-      const double l2 = dot3(dx, dy, dz, dx, dy, dz);
-      const double r = sqrt(l2);
-      const double rinv = r > 0.0 ? 1.0 / r : 0.0;  // r = 0: dr = 0, gradW = 0
-      const double qa = divr(r, ha, rha), qb = divr(r, hb, hi[u].x);
-      if (OMG) om += mb * wendPdWhi(P.wcon, qa, ha, rha, i3, c3);
-      const double Kb = wrom * (hi[u].y * hb);  // WCON hb^-4 (/ omega_a)
-      double Ga = qa <= 2.0 ? wendPoly(qa) * Ka * rinv : 0.0;
-      double Gb = qb <= 2.0 ? wendPoly(qb) * Kb * rinv : 0.0;
-      if (!VARH) Ga = Gb = 0.5 * (Ga + Gb);  // the average gradient
-      if (fluid) {
-        const double dv0 = va.x - v[u].x, dv1 = va.y - v[u].y, dv2 = va.z - v[u].z;
-        const double Gbar = 0.5 * (Ga + Gb);  // gradW-bar = dr * Gbar
-        const double hav = 0.5 * (ha + hb);
-        // is_neighbr (particle.h:236-238)
-        const double lim = 2.0 * dmax2(fabs(ha), fabs(hb));
-        const bool isPair = !NEAR || l2 <= lim * lim;
-        double fvs = 0.0;  // fv = dv * fvs (Morris)
-        double fvr = 0.0;  // fv = dr * fvr (Cleary, Monaghan: m_b visc gradW-bar)
-        double vsig = vsigC;
-        const double vdr = (ARTIF || VISC == VISC_CLE || VISC == VISC_MON)
-                               ? dot3(dx, dy, dz, dv0, dv1, dv2)
-                               : 0.0;
-        if (VISC == VISC_MOR) {
-          const double rab = 1.0 / (da.x * rhob);
-          const double visc = LIQDEM ? viscLiq * rab : P.viscosity * (da.x + rhob) * rab;
-          const double den = l2 + 0.01 * (hav * hav);
-          fvs = mb * visc * (Gbar * l2) / den;  // dr . gradW-bar = Gbar |dr|^2
-        }
-        if (VISC == VISC_CLE) {  // sph.h:598-604
-          const double den = l2 + 0.01 * (hav * hav);
-          const double visc = 19.8 * P.viscosity * vdr / ((da.x + rhob) * den);
-          fvr = mb * visc * Gbar;
-        }
-        if (VISC == VISC_MON) {  // sph.h:606-630, no SLK
-          const double viss = vdr * rinv;
-          if (!LIQDEM) vsig = 2.0 * P.spsound + 2.0 * fabs(viss);
-          const double visc = viss * vsig * alphaM / (da.x + rhob);
-          fvr = mb * visc * Gbar;
-        }
-        if (ARTIF) {
-          double avsig = 0, avisc = 0.0;
-          if (vdr < 0) {
-            const double viss = vdr * rinv;
-            avsig = 2.0 * P.spsound - 4.0 * viss;
-            avisc = viss * avsig * P.alpha_artificial / (da.x + rhob);
-          }
-          const double sg = mb * avisc * Gbar;
-          f.x += sg * dx;
-          f.y += sg * dy;
-          f.z += sg * dz;
-          vsig = dmax2(vsig, avsig);
-        }
-        if (ARTIF || VISC == VISC_MON)
-          newDt = dmin2(newDt, isPair ? 0.6 * hav / vsig : inf);
-        else
-          minA = dmin2(minA, isPair ? 0.6 * hav : inf);
-        minB = dmin2(minB, isPair ? cdiff * (hav * hav) : inf);
-        constexpr bool alongDr = VISC == VISC_CLE || VISC == VISC_MON;
-        const double fv0 = alongDr ? dx * fvr : dv0 * fvs;
-        const double fv1 = alongDr ? dy * fvr : dv1 * fvs;
-        const double fv2 = alongDr ? dz * fvr : dv2 * fvs;
-        fva.x += fv0;
-        fva.y += fv1;
-        fva.z += fv2;
-        f.x += fv0;
-        f.y += fv1;
-        f.z += fv2;
-      }
-      // calcPressForce (sph.h:698-710), antic = 0 under NO_ANTICLUMPING:
-      // -mb (pdr2a gradWa + pdr2b gradWb) = dr * pp
-      const double pp = -mb * (da.y * Ga + pdr2b * Gb);
-      const double p0 = pp * dx, p1 = pp * dy, p2 = pp * dz;
-      fpa.x += p0;
-      fpa.y += p1;
-      fpa.z += p2;
-      f.x += p0;
-      f.y += p1;
-      f.z += p2;
-    }
-  }
-  if (NEAR && walkAgain(om + f.x + f.y + f.z + fpa.x + fpa.y + fpa.z + fva.x + fva.y + fva.z,
-                        S.posh, a, ns, nbl, nbcnt))
-    return true;
-  if (!ARTIF && VISC != VISC_MON && minA != inf) newDt = dmin2(newDt, minA / vsigC);
-  if (minB != inf) newDt = dmin2(newDt, minB / P.viscosity);
-  if (OMG) {
-    const double omega = 1 + ha * om / (da.x * 3);
-    S.dpo[a].z = omega;
-    const double rw = 1.0 / omega;
-    const double4 f0 = S.frc[a], fp0 = S.fp[a], fv0 = S.fv[a];
-    f = make_double4(f0.x + rw * f.x, f0.y + rw * f.y, f0.z + rw * f.z, f0.w);
-    fpa = make_double4(fp0.x + rw * fpa.x, fp0.y + rw * fpa.y, fp0.z + rw * fpa.z, fp0.w);
-    fva = make_double4(fv0.x + rw * fva.x, fv0.y + rw * fva.y, fv0.z + rw * fva.z, fv0.w);
-  }
-  S.frc[a] = f;
-  S.fp[a] = fpa;
-  S.fv[a] = fva;
-  return false;
-}
-template <bool VARH, int VISC, bool ARTIF, bool LIQDEM, bool OMG, bool NEAR>
 __global__ void __launch_bounds__(256) k_force_l(Store S, int ns, Box B, int* __restrict__ nbl,
                                                  int* __restrict__ nbcnt,
+                                                 const int* __restrict__ flags,
                                                  const double2* __restrict__ hinv,
                                                  sphdem_params P, DevGlobals* g) {
-  int a = xcdThread();
-  double newDt = __longlong_as_double(0x7ff0000000000000ll);
-  if (a < ns)
-    while (walkForce<VARH, VISC, ARTIF, LIQDEM, OMG, NEAR>(S, a, ns, nbl, nbcnt, hinv, P, newDt))
-      a = anew(a);
+  static_assert(VARH || !OMG, "omega is only fused under VAR_H");
+  const int a = xcdThread();
+  const double inf = __longlong_as_double(0x7ff0000000000000ll);
+  double newDt = inf;
+  if (a < ns) {
+    const bool fluid = S.iam[a] == T_SPH;  // viscosity only acts on sph (sphIncompress.h:927)
+    const double4 pa = S.posh[a];
+    const double4 va = S.vhm[a];
+    const double4 da = S.dpo[a];
+    const double ha = pa.w;
+    const double rha = 1.0 / ha;
+    const double rom = (VARH && !OMG) ? 1.0 / da.z : 1.0;
+    const double i3 = OMG ? 1.0 / cube(ha) : 0.0, c3 = OMG ? 3.0 / pow4(ha) : 0.0;
+    double om = OMG ? va.w * wendPdWhi(P.wcon, 0, ha, rha, i3, c3) : 0.0;
+    // gradW = dr * F(q, h) (/ omega_a under VAR_H), F = WCON poly(q) / (q h^5)
+    // = dr * poly(q) * K(h) / r with K(h) = WCON h^-4 (/ omega_a)
+    const double Ka = P.wcon * (rha * rha) * (rha * rha) * rom;
+    const double wrom = P.wcon * rom;
+    const double viscLiq = 2.0 * P.viscosity * P.dens;  // numerator under LIQ_DEM
+    const double vsigC = (VISC == VISC_MOR || VISC == VISC_CLE) ? 2.0 * P.spsound : 0.0;
+    const double cdiff = VISC == VISC_MON ? 0.06 : 0.125;  // viscDiffusionCondition
+    const double alphaM = monaghanAlpha(P);
+    double minA = inf, minB = inf;  // min over pairs of 0.6 hav and cdiff hav^2
+    // both numerators and their rounded values increase with h_b: a near list's
+    // pairs keep their smallest h_b, which saves two FP64 operations an entry
+    double minHb = inf;
+    const double4 zero4 = make_double4(0.0, 0.0, 0.0, 0.0);
+    double4 f = OMG ? zero4 : S.frc[a], fpa = OMG ? zero4 : S.fp[a], fva = OMG ? zero4 : S.fv[a];
+    const int n = walkLength<NEAR>(flags, S.posh, a, ns, nbl, nbcnt);
+    constexpr int U = 4;
+    for (int k0 = 0; k0 < n; k0 += U) {
+      SPHDEM_FETCH_ENTRIES(U)
+      double4 p[U], v[U];
+      double2 d[U], hi[U];
+#pragma unroll
+      for (int u = 0; u < U; u++) {
+        const int j = e[u];
+        p[u] = S.posh[j];
+        v[u] = S.vhm[j];
+        d[u] = *reinterpret_cast<const double2*>(&S.dpo[j]);  // dens, pdr2
+        hi[u] = hinv[j];
+      }
+#pragma unroll
+      for (int u = 0; u < U; u++) {
+        if (k0 + u >= n) break;
+        const double hb = p[u].w, mb = v[u].w, rhob = d[u].x, pdr2b = d[u].y;
+        const double dx = pa.x - p[u].x, dy = pa.y - p[u].y, dz = pa.z - p[u].z;
+        const double l2 = dot3(dx, dy, dz, dx, dy, dz);
+        const double r = sqrt(l2);
+        const double rinv = r > 0.0 ? 1.0 / r : 0.0;  // r = 0: dr = 0, gradW = 0
+        const double qa = divr(r, ha, rha), qb = divr(r, hb, hi[u].x);
+        if (OMG) om += mb * wendPdWhi(P.wcon, qa, ha, rha, i3, c3);
+        const double Kb = wrom * (hi[u].y * hb);  // WCON hb^-4 (/ omega_a)
+        double Ga = qa <= 2.0 ? wendPoly(qa) * Ka * rinv : 0.0;
+        double Gb = qb <= 2.0 ? wendPoly(qb) * Kb * rinv : 0.0;
+        if (!VARH) Ga = Gb = 0.5 * (Ga + Gb);  // the average gradient
+        if (fluid) {
+          const double dv0 = va.x - v[u].x, dv1 = va.y - v[u].y, dv2 = va.z - v[u].z;
+          const double Gbar = 0.5 * (Ga + Gb);  // gradW-bar = dr * Gbar
+          const double hav = 0.5 * (ha + hb);
+          // is_neighbr (particle.h:236-238)
+          const double lim = 2.0 * dmax2(fabs(ha), fabs(hb));
+          const bool isPair = !NEAR || l2 <= lim * lim;
+          double fvs = 0.0;  // fv = dv * fvs (Morris)
+          double fvr = 0.0;  // fv = dr * fvr (Cleary, Monaghan: m_b visc gradW-bar)
+          double vsig = vsigC;
+          const double vdr = (ARTIF || VISC == VISC_CLE || VISC == VISC_MON)
+                                 ? dot3(dx, dy, dz, dv0, dv1, dv2)
+                                 : 0.0;
+          if (VISC == VISC_MOR) {
+            const double rab = 1.0 / (da.x * rhob);
+            const double visc = LIQDEM ? viscLiq * rab : P.viscosity * (da.x + rhob) * rab;
+            const double den = l2 + 0.01 * (hav * hav);
+            fvs = mb * visc * (Gbar * l2) / den;  // dr . gradW-bar = Gbar |dr|^2
+          }
+          if (VISC == VISC_CLE) {  // sph.h:598-604
+            const double den = l2 + 0.01 * (hav * hav);
+            const double visc = 19.8 * P.viscosity * vdr / ((da.x + rhob) * den);
+            fvr = mb * visc * Gbar;
+          }
+          if (VISC == VISC_MON) {  // sph.h:606-630, no SLK
+            const double viss = vdr * rinv;
+            if (!LIQDEM) vsig = 2.0 * P.spsound + 2.0 * fabs(viss);
+            const double visc = viss * vsig * alphaM / (da.x + rhob);
+            fvr = mb * visc * Gbar;
+          }
+          if (ARTIF) {
+            double avsig = 0, avisc = 0.0;
+            if (vdr < 0) {
+              const double viss = vdr * rinv;
+              avsig = 2.0 * P.spsound - 4.0 * viss;
+              avisc = viss * avsig * P.alpha_artificial / (da.x + rhob);
+            }
+            const double sg = mb * avisc * Gbar;
+            f.x += sg * dx;
+            f.y += sg * dy;
+            f.z += sg * dz;
+            vsig = dmax2(vsig, avsig);
+          }
+          if (ARTIF || VISC == VISC_MON)
+            newDt = dmin2(newDt, isPair ? 0.6 * hav / vsig : inf);
+          else if (!NEAR)
+            minA = dmin2(minA, 0.6 * hav);
+          if (NEAR)
+            minHb = dmin2(minHb, isPair ? hb : inf);
+          else
+            minB = dmin2(minB, cdiff * (hav * hav));
+          constexpr bool alongDr = VISC == VISC_CLE || VISC == VISC_MON;
+          const double fv0 = alongDr ? dx * fvr : dv0 * fvs;
+          const double fv1 = alongDr ? dy * fvr : dv1 * fvs;
+          const double fv2 = alongDr ? dz * fvr : dv2 * fvs;
+          fva.x += fv0;
+          fva.y += fv1;
+          fva.z += fv2;
+          f.x += fv0;
+          f.y += fv1;
+          f.z += fv2;
+        }
+        // calcPressForce (sph.h:698-710), antic = 0 under NO_ANTICLUMPING:
+        // -mb (pdr2a gradWa + pdr2b gradWb) = dr * pp
+        const double pp = -mb * (da.y * Ga + pdr2b * Gb);
+        const double p0 = pp * dx, p1 = pp * dy, p2 = pp * dz;
+        fpa.x += p0;
+        fpa.y += p1;
+        fpa.z += p2;
+        f.x += p0;
+        f.y += p1;
+        f.z += p2;
+      }
+    }
+    if (NEAR && minHb != inf) {
+      const double hav = 0.5 * (ha + minHb);
+      minA = 0.6 * hav;
+      minB = cdiff * (hav * hav);
+    }
+    if (!ARTIF && VISC != VISC_MON && minA != inf) newDt = dmin2(newDt, minA / vsigC);
+    if (minB != inf) newDt = dmin2(newDt, minB / P.viscosity);
+    if (OMG) {
+      const double omega = 1 + ha * om / (da.x * 3);
+      S.dpo[a].z = omega;
+      const double rw = 1.0 / omega;
+      const double4 f0 = S.frc[a], fp0 = S.fp[a], fv0 = S.fv[a];
+      f = make_double4(f0.x + rw * f.x, f0.y + rw * f.y, f0.z + rw * f.z, f0.w);
+      fpa = make_double4(fp0.x + rw * fpa.x, fp0.y + rw * fpa.y, fp0.z + rw * fpa.z, fp0.w);
+      fva = make_double4(fv0.x + rw * fva.x, fv0.y + rw * fva.y, fv0.z + rw * fva.z, fv0.w);
+    }
+    S.frc[a] = f;
+    S.fp[a] = fpa;
+    S.fv[a] = fva;
+  }
   atomicMinPos(&g->newDt_bits, newDt);
 }
 
