@@ -516,11 +516,12 @@ int launchLists(sphdem_ctx* ctx, const double4* pos) {
 // Up to this many targets (two tiles a CU) a tile's columns are searched by nine
 // wavefronts side by side instead of three after one another: a build is then a
 // chain of latencies, that of the tile with the most groups.  Sedimentation
-// boxes, one build, nine against three (and the most groups of a tile): 12^3 28 /
-// 42 us (2), 16^3 48 / 73 (4), 20^3 31 / 47 (2), 24^3 39 / 42 (2), 28^3 57 / 68
-// (3); past it the wavefronts queue: 32^3 68 / 55 (2), 64^3 321 / 166.  (Where a
-// box is a third of a cell longer than whole cells, as 16^3 and 28^3 are, its
-// last columns hold a third of the others' particles and a tile spans several.)
+// boxes, one build by events around it, nine against three (and the most groups
+// of a tile): 12^3 28 / 42 us (2), 16^3 48 / 73 (4), 20^3 31 / 47 (2), 24^3 39 / 42
+// (2), 28^3 57 / 68 (3); past it the wavefronts queue: 32^3 68 / 55 (2), 64^3 321 /
+// 166.  (Where a box is a third of a cell longer than whole cells, as 16^3 and 28^3
+// are, its last columns hold a third of the others' particles and a tile spans
+// several.)
 constexpr int kNearSmall = 64 * 512;
 // Whether a step's walks take near lists: not with a segmented tile shape, and
 // not where a cell holds over kNearOccupancy particles at
