@@ -1073,8 +1073,35 @@ SumPool g_sumPool[kScratchDevices];
 class LaunchSums {
  public:
   LaunchSums(hipStream_t stream, unsigned blocks) : stream_(stream) {
-    int dev = -1;
-    if (blocks < 2 || hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kScratchDevices) return;
+    // the stream's device, where the launch runs, need not be the current one
+    int cur = -1, dev = -1;
+    if (blocks < 2 || hipGetDevice(&cur) != hipSuccess) return;
+    dev = cur;
+    if (stream && stream != hipStreamPerThread && hipStreamGetDevice(stream, &dev) != hipSuccess) {
+      (void)hipGetLastError();
+      return;
+    }
+    if (dev < 0 || dev >= kScratchDevices) return;
+    if (dev != cur && hipSetDevice(dev) != hipSuccess) {
+      (void)hipGetLastError();
+      return;
+    }
+    find(dev, stream);
+    if (dev != cur) (void)hipSetDevice(cur);
+  }
+  ~LaunchSums() {
+    if (!pool_) return;
+    const bool ok = hipEventRecord(pool_->ended[k_], stream_) == hipSuccess;
+    if (!ok) (void)hipGetLastError();  // these cells are not used again
+    std::lock_guard<std::mutex> lock(g_sumMu);
+    pool_->taken[k_] = !ok;
+  }
+  LaunchSums(const LaunchSums&) = delete;
+  LaunchSums& operator=(const LaunchSums&) = delete;
+  sphdem_adj::SumCells* cells() const { return cells_; }
+
+ private:
+  void find(int dev, hipStream_t stream) {
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(stream, &cap) != hipSuccess) {
       (void)hipGetLastError();
@@ -1101,10 +1128,12 @@ class LaunchSums {
       const int k = (p.next + i) % kSumLaunches;
       if (p.taken[k]) continue;
       if (i >= kSumLaunches) {  // all in use
-        if (p.stream[k] != stream || hipStreamWaitEvent(stream, p.ended[k], 0) != hipSuccess)
-          continue;
-        take(p, k, stream);
-        break;
+        if (p.stream[k] != stream || !p.ended[k]) continue;
+        if (hipStreamWaitEvent(stream, p.ended[k], 0) == hipSuccess)
+          take(p, k, stream);
+        else
+          (void)hipGetLastError();
+        continue;
       }
       if (!p.ended[k] &&
           hipEventCreateWithFlags(&p.ended[k], hipEventDisableTiming) != hipSuccess) {
@@ -1120,18 +1149,6 @@ class LaunchSums {
     }
     (void)hipThreadExchangeStreamCaptureMode(&mode);
   }
-  ~LaunchSums() {
-    if (!pool_) return;
-    const bool ok = hipEventRecord(pool_->ended[k_], stream_) == hipSuccess;
-    if (!ok) (void)hipGetLastError();  // these cells are not used again
-    std::lock_guard<std::mutex> lock(g_sumMu);
-    pool_->taken[k_] = !ok;
-  }
-  LaunchSums(const LaunchSums&) = delete;
-  LaunchSums& operator=(const LaunchSums&) = delete;
-  sphdem_adj::SumCells* cells() const { return cells_; }
-
- private:
   void take(SumPool& p, int k, hipStream_t stream) {
     p.taken[k] = p.used[k] = true;
     p.stream[k] = stream;
