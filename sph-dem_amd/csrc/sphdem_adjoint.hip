@@ -22,6 +22,7 @@
 #include <hip/hip_runtime.h>
 #include <math.h>
 #include <stdint.h>
+#include <string.h>
 
 #include <mutex>
 
@@ -153,11 +154,20 @@ struct SumCells {
   double part[3][kSumCells];
   unsigned done;  // blocks that have added; zero between launches, as the cells
 };
+// The cells of a launch (or null), and the host's word that receives `turn` when
+// they are zero again (or null).
+struct LaunchCells {
+  SumCells* cells;
+  unsigned* ended;
+  unsigned turn;
+};
 
 // Sums NV per-thread values over the block and adds each total to dst[k], by way
 // of the launch's cells if it has any.  Every thread of the block must call it.
 template <int NV>
-__device__ void blockAdd(double (&v)[NV], double* dst, SumCells* cells = nullptr) {
+__device__ void blockAdd(double (&v)[NV], double* dst,
+                         const LaunchCells& launch = LaunchCells{}) {
+  SumCells* const cells = launch.cells;
   static_assert(NV <= 3, "SumCells holds three sums");
   __shared__ double part[NV][kTPB / 64];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
@@ -192,6 +202,10 @@ __device__ void blockAdd(double (&v)[NV], double* dst, SumCells* cells = nullptr
   }
   if (lane == 0)
     __hip_atomic_store(&cells->done, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (!launch.ended) return;
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  if (lane == 0)
+    __hip_atomic_store(launch.ended, launch.turn, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // ---------------------------------------------------------------- SPH force
@@ -261,7 +275,7 @@ __global__ void __launch_bounds__(kTPB) k_force_bwd(int32_t nq, const int32_t* _
                             const int32_t* __restrict__ pimg, sphdem_adj_fields in,
                             sphdem_adj_consts C, const double* __restrict__ gfv,
                             const double* __restrict__ gfp, sphdem_adj_grads g,
-                            SumCells* cells) {
+                            LaunchCells cells) {
   const int i = queryIndex<kSphLanes>(), gl = queryLane<kSphLanes>();
   double gnu[1] = {0.0};
   if (i < nq) {
@@ -821,7 +835,7 @@ __global__ void __launch_bounds__(kTPB) k_fpi_bwd(int32_t nq, const int32_t* __r
                           const int64_t* __restrict__ off, const int32_t* __restrict__ pb,
                           const int32_t* __restrict__ pimg, sphdem_adj_fields in,
                           sphdem_adj_consts C, const double* __restrict__ gfd,
-                          sphdem_adj_grads g, SumCells* cells) {
+                          sphdem_adj_grads g, LaunchCells cells) {
   const int i = queryIndex<kFpiLanes>(), gl = queryLane<kFpiLanes>();
   __shared__ Add3Stage stage[kTPB / 64];
   double gpar[3] = {0.0, 0.0, 0.0};  // nu, drag_a, drag_b
@@ -1048,121 +1062,94 @@ int scratchOfCurrentDevice(double** out) {
 }
 
 // ---- the launches' partial sums
-// A launch has its SumCells to itself until it has ended (an event after it
-// says so), whatever streams and threads launch beside it; where all are in use
-// it takes those of an earlier launch on its own stream, behind which it runs.
-// A captured launch keeps its cells: it may be replayed at any time (two replays
-// of one captured launch at once would race on its outputs as well).  With none
-// left, or on a device past the kept ones, the blocks add to the result directly.
-constexpr int kSumLaunches = 32, kSumCaptured = 64;
+// A launch has its SumCells to itself until its last block has cleared them and
+// said so in a word of the host's memory, whatever streams and threads launch
+// beside it.  (An event after each launch says the same for 15 us of the host's.)
+// A captured launch keeps its cells: it may be replayed at any time (two replays of
+// one captured launch at once would race on its outputs as well).  With none free,
+// or on a device past the kept ones, the blocks add to the result directly.
+constexpr int kSumLaunches = 256, kSumCaptured = 64;
 __device__ sphdem_adj::SumCells sumCells[kSumLaunches + kSumCaptured];
 
 struct SumPool {
   sphdem_adj::SumCells* base = nullptr;
-  hipEvent_t ended[kSumLaunches] = {};
-  hipStream_t stream[kSumLaunches] = {};  // of its last launch
-  bool taken[kSumLaunches] = {};  // until its event is recorded
-  bool used[kSumLaunches] = {};
+  unsigned* ended = nullptr;  // pinned: the last turn of each that has ended
+  unsigned* endedDev = nullptr;
+  unsigned turn[kSumLaunches] = {};
   int next = 0, captured = 0;
+  bool failed = false;
 };
 std::mutex g_sumMu;
 SumPool g_sumPool[kScratchDevices];
 
-// The cells of one launch on `stream`: taken here, given back when destroyed,
-// right after the launch.
-class LaunchSums {
- public:
-  LaunchSums(hipStream_t stream, unsigned blocks) : stream_(stream) {
-    // the stream's device, where the launch runs, need not be the current one
-    int cur = -1, dev = -1;
-    if (blocks < 2 || hipGetDevice(&cur) != hipSuccess) return;
-    dev = cur;
-    if (stream && stream != hipStreamPerThread && hipStreamGetDevice(stream, &dev) != hipSuccess) {
-      (void)hipGetLastError();
-      return;
-    }
-    if (dev < 0 || dev >= kScratchDevices) return;
-    if (dev != cur && hipSetDevice(dev) != hipSuccess) {
-      (void)hipGetLastError();
-      return;
-    }
-    find(dev, stream);
-    if (dev != cur) (void)hipSetDevice(cur);
+// Looks up (and at first makes) what a device keeps; that device is current.
+bool sumPoolReady(SumPool& p) {
+  if (p.endedDev) return true;
+  if (p.failed) return false;
+  void *q = nullptr, *e = nullptr, *d = nullptr;
+  p.failed = hipGetSymbolAddress(&q, HIP_SYMBOL(sumCells)) != hipSuccess ||
+             hipHostMalloc(&e, sizeof(unsigned) * kSumLaunches, hipHostMallocCoherent) !=
+                 hipSuccess ||
+             hipHostGetDevicePointer(&d, e, 0) != hipSuccess;
+  if (p.failed) {
+    (void)hipGetLastError();
+    return false;
   }
-  ~LaunchSums() {
-    if (!pool_) return;
-    const bool ok = hipEventRecord(pool_->ended[k_], stream_) == hipSuccess;
-    if (!ok) (void)hipGetLastError();  // these cells are not used again
-    std::lock_guard<std::mutex> lock(g_sumMu);
-    pool_->taken[k_] = !ok;
+  memset(e, 0, sizeof(unsigned) * kSumLaunches);
+  p.base = (sphdem_adj::SumCells*)q;
+  p.ended = (unsigned*)e;
+  p.endedDev = (unsigned*)d;
+  return true;
+}
+// The cells for one launch of that many blocks on `stream`, which follows.
+sphdem_adj::LaunchCells launchCells(hipStream_t stream, unsigned blocks) {
+  sphdem_adj::LaunchCells out{};
+  // the stream's device, where the launch runs, need not be the current one
+  int cur = -1, dev = -1;
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  if (blocks < 2 || hipGetDevice(&cur) != hipSuccess) return out;
+  dev = cur;
+  if ((stream && stream != hipStreamPerThread && hipStreamGetDevice(stream, &dev) != hipSuccess) ||
+      hipStreamIsCapturing(stream, &cap) != hipSuccess) {
+    (void)hipGetLastError();
+    return out;
   }
-  LaunchSums(const LaunchSums&) = delete;
-  LaunchSums& operator=(const LaunchSums&) = delete;
-  sphdem_adj::SumCells* cells() const { return cells_; }
-
- private:
-  void find(int dev, hipStream_t stream) {
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(stream, &cap) != hipSuccess) {
-      (void)hipGetLastError();
-      return;
-    }
-    std::lock_guard<std::mutex> lock(g_sumMu);
-    SumPool& p = g_sumPool[dev];
-    if (!p.base) {
-      void* q = nullptr;
-      if (hipGetSymbolAddress(&q, HIP_SYMBOL(sumCells)) != hipSuccess) {
-        (void)hipGetLastError();
-        return;
-      }
-      p.base = (sphdem_adj::SumCells*)q;
-    }
-    if (cap != hipStreamCaptureStatusNone) {
-      if (p.captured < kSumCaptured) cells_ = p.base + kSumLaunches + p.captured++;
-      return;
-    }
-    // another thread's capture is none of these calls' concern
+  if (dev < 0 || dev >= kScratchDevices) return out;
+  std::lock_guard<std::mutex> lock(g_sumMu);
+  SumPool& p = g_sumPool[dev];
+  if (!p.endedDev) {
+    // not under a capture's rules for allocations, this thread's or another's
     hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
     (void)hipThreadExchangeStreamCaptureMode(&mode);
-    for (int i = 0; i < 2 * kSumLaunches && !pool_; i++) {
-      const int k = (p.next + i) % kSumLaunches;
-      if (p.taken[k]) continue;
-      if (i >= kSumLaunches) {  // all in use
-        if (p.stream[k] != stream || !p.ended[k]) continue;
-        if (hipStreamWaitEvent(stream, p.ended[k], 0) == hipSuccess)
-          take(p, k, stream);
-        else
-          (void)hipGetLastError();
-        continue;
-      }
-      if (!p.ended[k] &&
-          hipEventCreateWithFlags(&p.ended[k], hipEventDisableTiming) != hipSuccess) {
-        p.ended[k] = nullptr;
-        (void)hipGetLastError();
-        break;
-      }
-      if (p.used[k] && hipEventQuery(p.ended[k]) != hipSuccess) {
-        (void)hipGetLastError();
-        continue;
-      }
-      take(p, k, stream);
-    }
+    const bool ready = (dev == cur || hipSetDevice(dev) == hipSuccess) && sumPoolReady(p);
+    if (dev != cur) (void)hipSetDevice(cur);
     (void)hipThreadExchangeStreamCaptureMode(&mode);
+    if (!ready) return out;
   }
-  void take(SumPool& p, int k, hipStream_t stream) {
-    p.taken[k] = p.used[k] = true;
-    p.stream[k] = stream;
+  if (cap != hipStreamCaptureStatusNone) {
+    if (p.captured < kSumCaptured) out.cells = p.base + kSumLaunches + p.captured++;
+    return out;
+  }
+  for (int i = 0; i < kSumLaunches; i++) {
+    const int k = (p.next + i) % kSumLaunches;
+    if (__atomic_load_n(&p.ended[k], __ATOMIC_ACQUIRE) != p.turn[k]) continue;
     p.next = k + 1;
-    pool_ = &p;
-    k_ = k;
-    cells_ = p.base + k;
+    out = sphdem_adj::LaunchCells{p.base + k, p.endedDev + k, ++p.turn[k]};
+    break;
   }
-
-  hipStream_t stream_;
-  SumPool* pool_ = nullptr;
-  int k_ = 0;
-  sphdem_adj::SumCells* cells_ = nullptr;
-};
+  return out;
+}
+// After a launch: its error, and its cells given back where it did not run.
+int adjLaunched(const sphdem_adj::LaunchCells& c) {
+  const int rc = adjLaunched();
+  if (rc && c.ended) {
+    std::lock_guard<std::mutex> lock(g_sumMu);
+    for (SumPool& p : g_sumPool)
+      if (p.endedDev && c.ended >= p.endedDev && c.ended < p.endedDev + kSumLaunches)
+        p.turn[c.ended - p.endedDev]--;
+  }
+  return rc;
+}
 
 // zero fill (a kernel, not a memset: the call stays a plain kernel sequence)
 __global__ void __launch_bounds__(sphdem_adj::kTPB) k_zero_doubles(double* __restrict__ p, int64_t n) {
@@ -1200,11 +1187,11 @@ int sphdem_adj_force_bwd(int32_t nquery, const int32_t* query, const int64_t* of
       !in->iam || !g->r || !g->vhat || !g->h || !g->dens || !g->omega || !g->pdr2 || !g->params)
     return SPHDEM_E_ARG;
   const unsigned grid = sphdem_adj::gridFor(nquery, sphdem_adj::kSphLanes);
-  const LaunchSums sums((hipStream_t)stream, grid);
+  const sphdem_adj::LaunchCells cells = launchCells((hipStream_t)stream, grid);
   hipLaunchKernelGGL(sphdem_adj::k_force_bwd, dim3(grid), dim3(sphdem_adj::kTPB), 0,
                      (hipStream_t)stream, nquery, query, off, b, img, *in, *c, gfv, gfp, *g,
-                     sums.cells());
-  return adjLaunched();
+                     cells);
+  return adjLaunched(cells);
 }
 
 int sphdem_adj_omega(int32_t nquery, const int32_t* query, const int64_t* off, const int32_t* b,
@@ -1353,11 +1340,10 @@ int sphdem_adj_fpi_bwd(int32_t nquery, const int32_t* query, const int64_t* off,
       !g->dens || !g->fpfb || !g->fv || !g->por || !g->params)
     return SPHDEM_E_ARG;
   const unsigned grid = sphdem_adj::gridFor(nquery, sphdem_adj::kFpiLanes);
-  const LaunchSums sums((hipStream_t)stream, grid);
+  const sphdem_adj::LaunchCells cells = launchCells((hipStream_t)stream, grid);
   hipLaunchKernelGGL(sphdem_adj::k_fpi_bwd, dim3(grid), dim3(sphdem_adj::kTPB), 0,
-                     (hipStream_t)stream, nquery, query, off, b, img, *in, *c, gfdrag, *g,
-                     sums.cells());
-  return adjLaunched();
+                     (hipStream_t)stream, nquery, query, off, b, img, *in, *c, gfdrag, *g, cells);
+  return adjLaunched(cells);
 }
 
 int sphdem_adj_contacts(int64_t npairs, const int32_t* a, const int32_t* b, const int32_t* img,

@@ -160,7 +160,7 @@ def test_launches_beside_and_behind_one_another():
         launch(cnt, want[k])
         torch.cuda.synchronize()
     streams = [torch.cuda.Stream() for _ in range(3)]
-    got = torch.zeros((240, 5), dtype=torch.float64, device="cuda")
+    got = torch.zeros((600, 5), dtype=torch.float64, device="cuda")
     torch.cuda.synchronize()
     for i in range(len(got)):
         with torch.cuda.stream(streams[i % 3]):
